@@ -139,6 +139,26 @@ int ttsp_nf4_gemm_swiglu(const void* X, int x_dtype, const uint8_t* W1, const ui
  * double-quant scales), else 0. Host-only. Replaces: nothing separate. */
 int ttsp_nf4_gemm_swiglu_fits(int M, int K, int N, int blocksize, int blocksize2, int nested);
 
+/* Long prompts: the product in two launches, the weight dequantised once into
+ * the caller's workspace, then a dense matrix kernel on it.
+ * ttsp_nf4_gemm_dense_splits: the K splits it runs in, 0 where it does not
+ * serve the shape (N below 513, small weights, byte offsets of 2^31 or more).
+ * work: 16-byte aligned, 2 * M * K bytes of dense weights, then (splits > 1)
+ * splits * N * M fp32 partial sums. Other arguments as ttsp_nf4_gemm's. */
+int ttsp_nf4_gemm_dense_splits(int M, int K, int N);
+int ttsp_nf4_gemm_dense(const void* X, int x_dtype, const uint8_t* W, const uint8_t* A8, const float* AMAX,
+                        const float* CODE2, float offset, const float* LUT, void* Y, const void* R, int epi, int M,
+                        int K, int N, int blocksize, int blocksize2, void* work, hipStream_t stream);
+/* The SwiGLU pair likewise (arguments as ttsp_nf4_gemm_swiglu's), with the
+ * bits of two ttsp_nf4_gemm_dense launches; served where each runs unsplit.
+ * work: 4 * M * K bytes. */
+int ttsp_nf4_gemm_dense_swiglu_fits(int M, int K, int N);
+int ttsp_nf4_gemm_dense_swiglu(const void* X, int x_dtype, const uint8_t* W1, const uint8_t* A8_1,
+                               const float* AMAX_1, const float* CODE2_1, float offset_1, const uint8_t* W3,
+                               const uint8_t* A8_3, const float* AMAX_3, const float* CODE2_3, float offset_3,
+                               const float* LUT, void* Y, int M, int K, int N, int blocksize, int blocksize2,
+                               void* work, hipStream_t stream);
+
 /* The batch-1 matmuls of a decode block in one launch each (K <= 32768,
  * K <= 4096 with NORM_W; ttsp_gemv_shape says whether a shape fits):
  *   W3 == NULL: Y = epi(n(X) . dequant(W1)^T), epi as ttsp_nf4_gemm;

@@ -527,6 +527,19 @@ static GemmPlan gemm_plan(int M, int K, int N) {
   return splits > 1 ? GemmPlan{2, splits} : GemmPlan{unsplit_shape(M, N), 1};
 }
 
+// Y = epilogue(round(sum of the splits' partials)) (epi bit 2: vectorised)
+int gemm_reduce(int dt, const float* YP, int splits, void* Y, const void* R, int epi, int M, int N, hipStream_t st) {
+  const long long chunks = (long long)((M + 7) / 8) * N;
+  const dim3 rg((unsigned)((chunks + 255) / 256));
+  if (dt == DT_BF16)
+    hipLaunchKernelGGL(nf4_gemm_reduce_kernel<DT_BF16>, rg, dim3(256), 0, st, YP, splits, (uint16_t*)Y,
+                       (const uint16_t*)R, epi, M, N);
+  else
+    hipLaunchKernelGGL(nf4_gemm_reduce_kernel<DT_F16>, rg, dim3(256), 0, st, YP, splits, (uint16_t*)Y,
+                       (const uint16_t*)R, epi, M, N);
+  TTSP_RETURN_LAUNCH();
+}
+
 int gemm_mfma(const void* X, int dt, const uint8_t* W, const uint8_t* A8, const float* AMAX,
               const float* CODE2, float offset, const float* LUT, void* Y, const void* R, int epi,
               int M, int K, int N, int bs_shift, int bs2_shift, const GemmPlan& plan, float* YP,
@@ -563,16 +576,7 @@ int gemm_mfma(const void* X, int dt, const uint8_t* W, const uint8_t* A8, const 
     return (int)hipErrorInvalidValue;
   }
 #undef TTSP_G
-  if (splits > 1 && reduce) {
-    const long long chunks = (long long)((M + 7) / 8) * N;
-    const dim3 rg((unsigned)((chunks + 255) / 256));
-    if (dt == DT_BF16)
-      hipLaunchKernelGGL(nf4_gemm_reduce_kernel<DT_BF16>, rg, dim3(256), 0, st, YP, splits, (uint16_t*)Y,
-                         (const uint16_t*)R, epi, M, N);
-    else
-      hipLaunchKernelGGL(nf4_gemm_reduce_kernel<DT_F16>, rg, dim3(256), 0, st, YP, splits, (uint16_t*)Y,
-                         (const uint16_t*)R, epi, M, N);
-  }
+  if (splits > 1 && reduce) return gemm_reduce(dt, YP, splits, Y, R, epi, M, N, st);
   TTSP_RETURN_LAUNCH();
 }
 

@@ -202,8 +202,16 @@ def matmul(module, x, *, epi: int = EPI_NONE, operand=None, out=None):
     elif out.dtype != x.dtype or out.numel() != rows * M or not out.is_contiguous():
         return None
     lib = _lib.lib()
-    splits = lib.ttsp_nf4_gemm_splits(M, K, rows) if rows > 1 else 1
-    if splits > 1:
+    dense = lib.ttsp_nf4_gemm_dense_splits(M, K, rows) if rows >= DENSE_MIN_ROWS else 0
+    splits = lib.ttsp_nf4_gemm_splits(M, K, rows) if rows > 1 and not dense else 1
+    if dense:
+        # the dequantised weight, then (K split) the partial sums
+        work = torch.empty(2 * M * K + (4 * dense * rows * M if dense > 1 else 0), dtype=torch.uint8, device=x.device)
+        rc = lib.ttsp_nf4_gemm_dense(
+            flat.data_ptr(), dt, fast["w"], fast["a8"], fast["amax"], fast["code2"], fast["offset"],
+            fast["lut"].data_ptr(), out.data_ptr(), _lib.ptr(operand) if epi else 0, epi, M, K, rows,
+            fast["bs"], fast["bs2"], work.data_ptr(), _lib.stream())
+    elif splits > 1:
         # K split over workgroups (too few output tiles to fill the GPU): fp32
         # partials in a workspace, summed in split order by a second kernel
         work = torch.empty(splits * rows * M, dtype=torch.float32, device=x.device)
@@ -220,6 +228,15 @@ def matmul(module, x, *, epi: int = EPI_NONE, operand=None, out=None):
         raise RuntimeError(f"ttsp_nf4_gemm failed: hipError_t {rc}")
     _stats["fast"] += 1
     return out.view(*x.shape[:-1], M)
+
+
+#: From this many rows `matmul` and `matmul_swiglu` ask for the dense form (the weight dequantised once a call into a
+#: workspace): below it the kernels that read the codes in place are as fast.
+DENSE_MIN_ROWS = 513
+
+
+def _dense(M: int, K: int, rows: int) -> bool:
+    return rows >= DENSE_MIN_ROWS and _lib.lib().ttsp_nf4_gemm_dense_splits(M, K, rows) > 0
 
 
 #: Widest output row whose RMSNorm the split-K reduce folds in (eight 8-value
@@ -244,7 +261,7 @@ def matmul_partials(module, x):
     if x.shape[-1] != K or not x.is_contiguous() or x.data_ptr() % 16:
         return None
     rows = x.numel() // K
-    if rows < 2:
+    if rows < 2 or _dense(M, K, rows):
         return None
     lib = _lib.lib()
     splits = lib.ttsp_nf4_gemm_splits(M, K, rows)
@@ -278,7 +295,7 @@ def matmul_norm(module, x, norm_weight, eps: float, *, epi: int = EPI_NONE, oper
     if x.shape[-1] != K or not x.is_contiguous() or x.data_ptr() % 16 or M % 8 or M > NORM_MAX_M:
         return None
     rows = x.numel() // K
-    if rows < 2:
+    if rows < 2 or _dense(M, K, rows):
         return None
     if (norm_weight.dtype != x.dtype or norm_weight.numel() != M or not norm_weight.is_contiguous()
             or norm_weight.data_ptr() % 16 or norm_weight.device != x.device):
@@ -417,16 +434,21 @@ def matmul_swiglu(module1, module3, x, *, out=None):
         return None
     rows = x.numel() // K
     lib = _lib.lib()
-    if not lib.ttsp_nf4_gemm_swiglu_fits(M, K, rows, f1["bs"], f1["bs2"], int(f1["nested"])):
+    dense = rows >= DENSE_MIN_ROWS and lib.ttsp_nf4_gemm_dense_swiglu_fits(M, K, rows)
+    if not dense and not lib.ttsp_nf4_gemm_swiglu_fits(M, K, rows, f1["bs"], f1["bs2"], int(f1["nested"])):
         return None
     if out is None:
         out = torch.empty((rows, M), dtype=x.dtype, device=x.device)
     elif out.dtype != x.dtype or out.numel() != rows * M or not out.is_contiguous():
         return None
-    rc = lib.ttsp_nf4_gemm_swiglu(
-        x.data_ptr(), dt, f1["w"], f1["a8"], f1["amax"], f1["code2"], f1["offset"],
-        f3["w"], f3["a8"], f3["amax"], f3["code2"], f3["offset"], f1["lut"].data_ptr(), out.data_ptr(),
-        M, K, rows, f1["bs"], f1["bs2"], _lib.stream())
+    args = (x.data_ptr(), dt, f1["w"], f1["a8"], f1["amax"], f1["code2"], f1["offset"],
+            f3["w"], f3["a8"], f3["amax"], f3["code2"], f3["offset"], f1["lut"].data_ptr(), out.data_ptr(),
+            M, K, rows, f1["bs"], f1["bs2"])
+    if dense:
+        work = torch.empty(4 * M * K, dtype=torch.uint8, device=x.device)  # both dequantised weights
+        rc = lib.ttsp_nf4_gemm_dense_swiglu(*args, work.data_ptr(), _lib.stream())
+    else:
+        rc = lib.ttsp_nf4_gemm_swiglu(*args, _lib.stream())
     if rc:
         raise RuntimeError(f"ttsp_nf4_gemm_swiglu failed: hipError_t {rc}")
     _stats["fast"] += 2
