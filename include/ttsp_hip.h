@@ -148,7 +148,7 @@ int ttsp_nf4_gemm_swiglu_fits(int M, int K, int N, int blocksize, int blocksize2
 int ttsp_nf4_gemm_dense_splits(int M, int K, int N);
 int ttsp_nf4_gemm_dense(const void* X, int x_dtype, const uint8_t* W, const uint8_t* A8, const float* AMAX,
                         const float* CODE2, float offset, const float* LUT, void* Y, const void* R, int epi, int M,
-                        int K, int N, int blocksize, int blocksize2, void* work, hipStream_t stream);
+                        int K, int N, int blocksize, int blocksize2, void* work, void* stream);
 /* The SwiGLU pair likewise (arguments as ttsp_nf4_gemm_swiglu's), with the
  * bits of two ttsp_nf4_gemm_dense launches; served where each runs unsplit.
  * work: 4 * M * K bytes. */
@@ -157,7 +157,7 @@ int ttsp_nf4_gemm_dense_swiglu(const void* X, int x_dtype, const uint8_t* W1, co
                                const float* AMAX_1, const float* CODE2_1, float offset_1, const uint8_t* W3,
                                const uint8_t* A8_3, const float* AMAX_3, const float* CODE2_3, float offset_3,
                                const float* LUT, void* Y, int M, int K, int N, int blocksize, int blocksize2,
-                               void* work, hipStream_t stream);
+                               void* work, void* stream);
 
 /* The batch-1 matmuls of a decode block in one launch each (K <= 32768,
  * K <= 4096 with NORM_W; ttsp_gemv_shape says whether a shape fits):
