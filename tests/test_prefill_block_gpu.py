@@ -721,3 +721,49 @@ def test_first_span_window_matches_the_whole_cache_window(roomy):
             a, b = a.float(), b.float()
             assert float((a - b).norm() / b.norm()) < 2e-2
     _set_kv(m, initial)
+
+
+def test_wide_spans_merge_runs_of_the_largest_bucket():
+    from ttspipe_amd.dualar import PREFILL_BUCKETS, WIDE_SPANS, _wide_spans, prefill_spans
+
+    top = PREFILL_BUCKETS[-1]
+    assert _wide_spans([]) == [] and _wide_spans(prefill_spans(40)) == [(0, 40, 64)]
+    assert _wide_spans(prefill_spans(top + 100)) == [(0, top, top), (top, 100, 128)]
+    assert _wide_spans(prefill_spans(2 * top)) == [(0, 2 * top, 2 * top)]
+    assert _wide_spans(prefill_spans(3 * top + 300)) == [(0, 3 * top + 300, 4 * top)]
+    assert _wide_spans(prefill_spans(9 * top + 5)) == [(0, 4 * top, 4 * top), (4 * top, 4 * top, 4 * top),
+                                                     (8 * top, top, top), (9 * top, 5, 8)]
+    for n in range(1, 6000, 101):
+        narrow, wide = prefill_spans(n), _wide_spans(prefill_spans(n))
+        assert sum(s for _, s, _ in wide) == n and sum(b for _, _, b in wide) == sum(b for _, _, b in narrow)
+        assert all(o == sum(b for _, _, b in wide[:i]) for i, (o, _, _) in enumerate(wide))
+        assert all(b <= WIDE_SPANS * top for _, _, b in wide)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("start,n", [(0, 1024), (0, 900), (200, 1000)])
+def test_wide_span_prefill_matches_its_narrow_spans(roomy, monkeypatch, start, n):
+    """A prompt of two largest-bucket spans as one span: graphed equals eager
+    bit for bit (twice, with other work between), and the spans run one by one
+    agree within the 2e-2 block bar (other GEMM tiles and attention splits
+    round differently); layer 0's K/V rows, which see no attention, closely."""
+    from ttspipe_amd import dualar
+
+    m = roomy
+    toks = _tokens(m, n, 11 + n)
+    initial = _kv_state(m, m.cfg.max_seq_len)
+    got = {}
+    for name, wide, graphed in (("eager", 4, False), ("graph", 4, True), ("again", 4, True), ("narrow", 1, False)):
+        monkeypatch.setattr(dualar, "WIDE_SPANS", wide)
+        _set_kv(m, initial)
+        assert m.prefill(toks, start, graphed=graphed)
+        torch.cuda.synchronize()
+        got[name] = {"kv": _kv_state(m, start + n), "logits": m.logits.clone(), "token": int(m.prefill_token.item())}
+    for name in ("graph", "again"):
+        assert torch.equal(got[name]["logits"], got["eager"]["logits"]) and got[name]["token"] == got["eager"]["token"]
+        for (k0, v0), (k1, v1) in zip(got["eager"]["kv"], got[name]["kv"]):
+            assert torch.equal(k0, k1) and torch.equal(v0, v1)
+    assert _rel(got["eager"]["logits"], got["narrow"]["logits"]) < 2e-2
+    for i, ((k0, v0), (k1, v1)) in enumerate(zip(got["eager"]["kv"], got["narrow"]["kv"])):
+        bar = 2e-3 if i == 0 else 2e-2
+        assert _rel(k0, k1) < bar and _rel(v0, v1) < bar

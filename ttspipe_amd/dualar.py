@@ -91,6 +91,26 @@ def prefill_spans(n: int):
     return out
 
 
+#: Spans of the largest bucket run together, up to this many of them a launch
+#: (2048 rows): the linears take a long span's rows in one product, which
+#: dequantises each weight once (1900 tokens after none, 12 layers: 11.7 ms in
+#: four spans of 512, 7.6 ms in one of 2048). More would only grow the
+#: activations: past 2048 rows the products gain nothing.
+WIDE_SPANS = 4
+
+
+def _wide_spans(spans):
+    """`prefill_spans`' list with each run of largest-bucket spans merged, up to
+    `WIDE_SPANS` to one: the same padded positions in fewer spans."""
+    top, out = PREFILL_BUCKETS[-1], []
+    for off, size, b in spans:
+        if out and b == top and out[-1][2] % top == 0 and out[-1][2] < WIDE_SPANS * top:
+            out[-1] = (out[-1][0], out[-1][1] + size, out[-1][2] + b)
+        else:
+            out.append((off, size, b))
+    return out
+
+
 SMALL = DualARConfig(dim=512, n_layer=3, n_head=4, n_local_heads=2, intermediate_size=1024,
                      vocab_size=512, fast_dim=256, fast_n_layer=2, fast_n_head=2, fast_n_local_heads=1,
                      fast_intermediate_size=512, num_codebooks=4, codebook_size=512, max_seq_len=320,
@@ -602,8 +622,8 @@ class SyntheticDualAR:
 
     def prefill(self, tokens, start: int, graphed: bool = True) -> bool:
         """KV entries for `tokens` (n_tokens, n) int32 at [start, start + n),
-        in spans of the largest bucket and a last span padded to a bucket (the
-        padding repeats the last real token; its KV entries land past the
+        in spans of the largest bucket (up to `WIDE_SPANS` of them run as one)
+        and a last span padded to a bucket (the padding repeats the last real token; its KV entries land past the
         prompt, where decoding overwrites them before reading them); the last
         real position's token in `prefill_token`. False (nothing done) when
         the padded span runs past the cache (reference: graphs.py:304-335).
@@ -615,7 +635,7 @@ class SyntheticDualAR:
         spans = prefill_spans(n)
         if not spans or start + spans[-1][0] + spans[-1][2] > self.cfg.max_seq_len:
             return False
-        for off, size, b in spans:
+        for off, size, b in _wide_spans(spans):
             first = start + off == 0
             if graphed:
                 graphs = self.prefill_first_graphs if first else self.prefill_graphs
@@ -741,8 +761,7 @@ def prefill_benchmark(n_tokens: int = 512, reps: int = 20, cfg: DualARConfig = D
     g = torch.Generator(device=model.device).manual_seed(cfg.seed)
     toks = torch.randint(0, cfg.codebook_size, (cfg.n_tokens, n_tokens), generator=g, device=model.device,
                          dtype=torch.int32)
-    model.capture_prefill(sorted({b for _, _, b in prefill_spans(n_tokens)}))
-    assert model.prefill(toks, 0)
+    assert model.prefill(toks, 0)  # captures the graphs it replays
     torch.cuda.synchronize()
     stream = torch.cuda.current_stream()
     start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
