@@ -200,6 +200,16 @@ int ttsp_nf4_dequant(const uint8_t* W, const uint8_t* A8, const float* AMAX, con
                      float offset, const float* LUT, void* out, int out_dtype, long long n,
                      int blocksize, int blocksize2, void* stream);
 
+/* The NF4 format of a dense weight: n (even) elements A of x_dtype (fp16, bf16
+ * or fp32, 16-byte aligned) to n / 2 bytes W (4-byte aligned, the even element
+ * in the high nibble) and fp32 AMAX per block of blocksize (64 to 512).
+ * ttsp_quantize_scales: the second level, X - *OFFSET in blocks of 256 to
+ * indices Q into the 256 ascending points CODE, fp32 AMAX per block. */
+int ttsp_nf4_quantize(const void* A, int dtype, long long n, int blocksize, const float* LUT, uint8_t* W,
+                      float* AMAX, void* stream);
+int ttsp_quantize_scales(const float* X, long long n, const float* OFFSET, const float* CODE, uint8_t* Q,
+                         float* AMAX, void* stream);
+
 /* Launch shape the N == 1 GEMV uses for [M, K]: J 64-dword chunks per lane,
  * K split over KS waves, RPW rows per wave. The arithmetic order depends on KS
  * only. Returns nonzero (and zeros) when the GEMV cannot hold the rows

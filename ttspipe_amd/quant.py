@@ -20,8 +20,9 @@ provides the same objects and the same byte layout:
   is the dequantise-then-matmul path bitsandbytes' forward takes (HIP
   dequantisation kernel + torch matmul). `nf4gemv.install()` patches it.
 
-Quantisation is a load-time data-format step (torch ops on whatever device
-the weight lives on); every operation on the decode path is a HIP kernel.
+Quantisation is a load-time data-format step: a HIP kernel for weights on a
+GPU, torch ops (the same bytes) elsewhere and for the forms the kernel does
+not take; every operation on the decode path is a HIP kernel.
 """
 
 from __future__ import annotations
@@ -135,16 +136,75 @@ def dequantize_blockwise_scales(qabsmax, state2, offset):
     return state2.code[qabsmax.long()] * state2.absmax[blocks // state2.blocksize] + offset
 
 
+_constants: dict = {}
+
+
+def _constant(name: str, device):
+    """A fresh copy of the NF4 code points ("nf4") or the dynamic map
+    ("dynamic") on a GPU, from one kept per device: building the map takes the
+    host 0.4 ms, and a copy from the host waits for the stream."""
+    key = (name, device)
+    t = _constants.get(key)
+    if t is None:
+        t = torch.tensor(NF4_CODE, dtype=torch.float32) if name == "nf4" else create_dynamic_map()
+        t = _constants[key] = t.to(device)
+    return t.clone()
+
+
+def _kernel_serves(A, flat, blocksize: int) -> bool:
+    """Whether the quantisation kernel takes this weight: plain fp16 / bf16 /
+    fp32 values on the current GPU, blocks of 64 to 512 (8 to 64 lanes of a
+    wave), nothing that follows the operations (gradients, wrapped tensors)."""
+    return (A.device.type == "cuda" and type(A) in (torch.Tensor, torch.nn.Parameter) and 64 <= blocksize <= 512
+            and A.dtype in (torch.float16, torch.bfloat16, torch.float32) and flat.numel() > 0
+            and not (A.requires_grad and torch.is_grad_enabled())
+            and not torch._C._functorch.is_functorch_wrapped_tensor(A)
+            and A.device.index == torch.cuda.current_device() and flat.data_ptr() % 16 == 0)
+
+
+def _quantize_4bit_kernel(A, flat, blocksize: int, compress_statistics: bool):
+    """`quantize_4bit` in one pass over the weight, the same bytes and scales
+    (`csrc/nf4_quantize.hip`); the mean of the scales stays torch's, whose sum
+    order the second-level indices depend on."""
+    from ttspipe_amd import _lib
+
+    lib, st, dev = _lib.lib(), _lib.stream(), flat.device
+    n = flat.numel()
+    nb = -(-n // blocksize)
+    code = _constant("nf4", dev)
+    packed = torch.empty((n // 2, 1), dtype=torch.uint8, device=dev)
+    absmax = torch.empty(nb, dtype=torch.float32, device=dev)
+    _lib.check(lib.ttsp_nf4_quantize(flat.data_ptr(), _lib.dtype_code(flat.dtype), n, blocksize, code.data_ptr(),
+                                     packed.data_ptr(), absmax.data_ptr(), st), "ttsp_nf4_quantize")
+    offset = state2 = None
+    if compress_statistics:
+        offset = absmax.mean()
+        code2 = _constant("dynamic", dev)
+        a8 = torch.empty(nb, dtype=torch.uint8, device=dev)
+        absmax2 = torch.empty(-(-nb // 256), dtype=torch.float32, device=dev)
+        _lib.check(lib.ttsp_quantize_scales(absmax.data_ptr(), nb, offset.data_ptr(), code2.data_ptr(), a8.data_ptr(),
+                                            absmax2.data_ptr(), st), "ttsp_quantize_scales")
+        state2 = QuantState(absmax=absmax2, shape=(nb,), code=code2, blocksize=256, quant_type="dynamic",
+                            dtype=torch.float32)
+        absmax = a8
+    state = QuantState(absmax=absmax, shape=A.shape, code=code, blocksize=blocksize, quant_type="nf4", dtype=A.dtype,
+                       offset=offset, state2=state2)
+    return packed, state
+
+
 def quantize_4bit(A, blocksize: int = 64, compress_statistics: bool = False, quant_type: str = "nf4"):
     """(packed uint8 [n/2, 1], QuantState) in bitsandbytes' NF4 layout."""
     if quant_type != "nf4":
         raise ValueError("only nf4 is supported")
     if blocksize < 64 or blocksize & (blocksize - 1):
         raise ValueError("blocksize must be a power of two >= 64")
-    flat = A.reshape(-1).float()
+    flat = A.reshape(-1)
     n = flat.numel()
     if n % 2:
         raise ValueError("NF4 packs two codes per byte: the element count must be even")
+    if _kernel_serves(A, flat, blocksize):
+        return _quantize_4bit_kernel(A, flat, blocksize, compress_statistics)
+    flat = flat.float()
     nb = -(-n // blocksize)
     pad = nb * blocksize - n
     blocks = torch.nn.functional.pad(flat, (0, pad)).view(nb, blocksize)
