@@ -139,6 +139,19 @@ int ttsp_nf4_gemm_swiglu(const void* X, int x_dtype, const uint8_t* W1, const ui
  * double-quant scales), else 0. Host-only. Replaces: nothing separate. */
 int ttsp_nf4_gemm_swiglu_fits(int M, int K, int N, int blocksize, int blocksize2, int nested);
 
+/* 9 to 64 rows, the K-steps split over workgroups where that fills the GPU.
+ * ttsp_nf4_gemm_few_splits: the splits, 0 where the kernel does not take the
+ * shape. work (16-byte aligned): splits * N * M fp32 sums (splits > 1). Y NULL
+ * leaves the sums in work (splits > 1); with G, the RMSNorm weight of the
+ * output rows, YN = rms_norm(Y, G, eps) in the reduce's launch (splits > 1,
+ * M % 8 == 0, M <= 4096, 16-byte aligned Y, YN, G and R). Other arguments as
+ * ttsp_nf4_gemm's. */
+int ttsp_nf4_gemm_few_splits(int M, int K, int N);
+int ttsp_nf4_gemm_few(const void* X, int x_dtype, const uint8_t* W, const uint8_t* A8, const float* AMAX,
+                      const float* CODE2, float offset, const float* LUT, void* Y, const void* R, int epi, int M,
+                      int K, int N, int blocksize, int blocksize2, float* work, const void* G, float eps, void* YN,
+                      void* stream);
+
 /* Long prompts: the product in two launches, the weight dequantised once into
  * the caller's workspace, then a dense matrix kernel on it.
  * ttsp_nf4_gemm_dense_splits: the K splits it runs in, 0 where it does not

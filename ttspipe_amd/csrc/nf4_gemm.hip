@@ -445,8 +445,9 @@ static void launch_gemm(const void* X, const uint8_t* W, const uint8_t* A8, cons
 // split keeps a long K run. Between 128 and 256 tiles no split fits one pass,
 // and 4 splits pay only past 16 K-steps each. Unsplit launches take 64 x 128
 // tiles down to 128 of them, 64 x 64 below. 33 to 64 rows take 64 x 64 tiles
-// with a K split (below); up to SKINNY_MAX_N rows otherwise the skinny kernel
-// (nf4_skinny.hip), shape 0, never split. Measured on the five
+// with a K split (below; callers with a choice take the few-row kernel, which
+// is faster: ttsp_nf4_gemm_few); up to 64 rows otherwise the few-row kernel or
+// the skinny kernel (nf4_gemm_few.hip, nf4_skinny.hip), shape 0, never split. Measured on the five
 // projections of a 2560-wide layer (wqkv 6144 x 2560, wo 2560 x 4096, w1 and
 // w3 9728 x 2560, w2 2560 x 9728): 187 -> 125 us at 128 rows against a rule
 // that sought two workgroups a CU, 200 -> 184 us at 256 rows, equal at 512
@@ -455,9 +456,13 @@ static void launch_gemm(const void* X, const uint8_t* W, const uint8_t* A8, cons
 struct GemmPlan {
   int shape, splits;
 };
-constexpr int SKINNY_MAX_N = 64;
-int skinny_max_k(int N);
-static bool skinny(int K, int N) { return N <= SKINNY_MAX_N && K <= skinny_max_k(N); }
+constexpr int SKINNY_MAX_N = 16;
+int skinny_max_k();
+bool few_unsplit(int M, int K, int N);
+int few_splits(int M, int K, int N);
+bool few_pair(int M, int K, int N);
+// Up to 64 rows, unsplit: the few-row kernel, or up to 16 the skinny one.
+static bool skinny(int K, int N) { return N <= SKINNY_MAX_N && K <= skinny_max_k(); }
 
 static long long gemm_tiles(int M, int N, int bm, int bn) {
   return (long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
@@ -465,16 +470,8 @@ static long long gemm_tiles(int M, int N, int bm, int bn) {
 
 static int unsplit_shape(int M, int N) { return gemm_tiles(M, N, 64, 128) >= 128 ? 2 : 3; }
 
-// From 33 rows (where the skinny kernel's tiles double) a K split of 64 x 64
-// tiles - one row tile covers every input row - beats the skinny kernel:
-// 4 ways where each split keeps 8 or more K-steps, else 2. Measured at 33-64
-// rows: 20-45 % faster on the five layer shapes (9728 x 2560 at 33 rows
-// 20.4 against 26.0 us, 2560 x 9728 at 64 rows 25.9 against 45.6) and on
-// the 1024-wide fast-transformer shapes (1024 x 3072 at 64 rows 13.1 against
-// 25.2); at 28-32 rows the two tie over a layer, below that the skinny kernel
-// wins (8 rows: 12.1 against 17.4 at 9728 x 2560). The unsplit entry has no
-// workspace, and unsplit tiles lose to the skinny kernel there, so it keeps
-// the skinny kernel up to SKINNY_MAX_N rows.
+// 33 to 64 rows through the split entry: 64 x 64 tiles, 4 ways where each split
+// keeps 8 or more K-steps, else 2.
 constexpr int SPLIT_SMALL_N = 32;
 
 bool gemm_dl_fits(int M, int K, int N, int splits);
@@ -510,7 +507,7 @@ static GemmPlan gemm_plan(int M, int K, int N) {
   if (N > SPLIT_SMALL_N && N <= 64)
     for (int sp = 4; sp >= 2; sp /= 2)
       if (steps % (2 * sp) == 0 && steps / sp >= 8) return {3, sp};
-  if (skinny(K, N)) return {0, 1};
+  if (skinny(K, N) || few_unsplit(M, K, N)) return {0, 1};
   GemmPlan dl;
   if (dl_plan(M, K, N, &dl)) return dl;
   const long long t = gemm_tiles(M, N, 64, 128);
@@ -537,6 +534,28 @@ int gemm_reduce(int dt, const float* YP, int splits, void* Y, const void* R, int
   else
     hipLaunchKernelGGL(nf4_gemm_reduce_kernel<DT_F16>, rg, dim3(256), 0, st, YP, splits, (uint16_t*)Y,
                        (const uint16_t*)R, epi, M, N);
+  TTSP_RETURN_LAUNCH();
+}
+
+// gemm_reduce with the fork's RMSNorm of each row to YN (2, 4 or 8 splits; M
+// and the pointers as nf4_gemm_reduce_norm_kernel takes them, checked by the caller)
+static int gemm_reduce_norm(int x_dtype, const float* work, int splits, void* Y, const void* R, int epi, int M, int N,
+                            const void* G, float eps, void* YN, hipStream_t stream) {
+  const dim3 grid((unsigned)N), block((unsigned)(64 * ((M / 8 + 63) / 64)));
+#define TTSP_RN(DTV, SV)                                                                                      \
+  hipLaunchKernelGGL((nf4_gemm_reduce_norm_kernel<DTV, SV>), grid, block, 0, stream, work, (uint16_t*)Y, \
+                     (const uint16_t*)R, epi, M, N, (const uint16_t*)G, eps, (uint16_t*)YN)
+#define TTSP_RS(DTV)                  \
+  if (splits == 2) TTSP_RN(DTV, 2);   \
+  else if (splits == 4) TTSP_RN(DTV, 4); \
+  else TTSP_RN(DTV, 8);
+  if (x_dtype == DT_BF16) {
+    TTSP_RS(DT_BF16)
+  } else {
+    TTSP_RS(DT_F16)
+  }
+#undef TTSP_RS
+#undef TTSP_RN
   TTSP_RETURN_LAUNCH();
 }
 
@@ -600,21 +619,27 @@ int gemm_skinny_pair(const void* X, int dt, const uint8_t* W1, const uint8_t* A8
                      const float* CODE2_3, float offset_3, const float* LUT, void* Y, int M, int K, int N, int bs_shift,
                      int bs2_shift, hipStream_t st);
 bool skinny_pair_fits(int K, int N);
+int gemm_few(const void* X, int dt, const uint8_t* W, const uint8_t* A8, const float* AMAX, const float* CODE2,
+             float offset, const float* LUT, void* Y, const void* R, int epi, int M, int K, int N, int bs_shift,
+             int bs2_shift, int splits, float* YP, hipStream_t st);
+int gemm_few_pair(const void* X, int dt, const uint8_t* W1, const uint8_t* A8_1, const float* AMAX_1,
+                  const float* CODE2_1, float offset_1, const uint8_t* W3, const uint8_t* A8_3, const float* AMAX_3,
+                  const float* CODE2_3, float offset_3, const float* LUT, void* Y, int M, int K, int N, int bs_shift,
+                  int bs2_shift, hipStream_t st);
 
-// Whether the SwiGLU pair takes the skinny kernel's pair form: where each of
-// its two GEMMs would run the skinny kernel (3 to 32 rows, unsplit; two rows
-// take the GEMV, whose one-launch pair is ttsp_nf4_gemv_fused_rows).
+// Whether the SwiGLU pair takes the few-row or the skinny kernel's pair form:
+// where each of its two GEMMs would run that kernel (3 to 32 rows, unsplit;
+// two rows take the GEMV, whose one-launch pair is ttsp_nf4_gemv_fused_rows).
 static bool swiglu_skinny(int M, int K, int N) {
-  if (M <= 0 || K <= 0 || K % 128 || N <= GEMV_ROWS_N || !skinny_pair_fits(K, N)) return false;
-  const GemmPlan p = gemm_plan(M, K, N);
-  return p.shape == 0 && p.splits == 1;
+  if (M <= 0 || K <= 0 || K % 128 || N <= GEMV_ROWS_N) return false;
+  return few_unsplit(M, K, N) ? few_pair(M, K, N) : skinny_pair_fits(K, N);
 }
 
 // Whether the SwiGLU pair fits one launch of the direct-to-LDS kernel: where
 // each of its two GEMMs would run that kernel unsplit (so the one launch
 // gives their bits).
 static bool swiglu_fits(int M, int K, int N, int bs_shift, int bs2_shift, bool nested) {
-  if (M <= 0 || K <= 0 || K % 128 || N <= SKINNY_MAX_N) return false;
+  if (M <= 0 || K <= 0 || K % 128 || N <= 64) return false;
   GemmPlan dl;
   if (!dl_plan(M, K, N, &dl) || dl.splits != 1 || dl.shape != 4) return false;
   // the plan's fallback to 64 x 128 tiles for small second-level groups
@@ -643,8 +668,8 @@ static int gemm_args(const void* X, const uint8_t* W, const uint8_t* A8, const f
 
 // One entry for every row count: up to GEMV_ROWS_N rows take the
 // bandwidth-bound GEMV (or, past the rows it holds, the kernels below), up
-// to 64 rows the skinny MFMA kernel (weights streamed once), more rows the
-// tiled MFMA kernel (weights read once per BN rows), unsplit.
+// to 64 rows the skinny or the few-row MFMA kernel (weights streamed once),
+// more rows the tiled MFMA kernel (weights read once per BN rows), unsplit.
 extern "C" int ttsp_nf4_gemm(const void* X, int x_dtype, const uint8_t* W, const uint8_t* A8,
                              const float* AMAX, const float* CODE2, float offset, const float* LUT,
                              void* Y, const void* R, int epi, int M, int K, int N, int blocksize,
@@ -658,6 +683,9 @@ extern "C" int ttsp_nf4_gemm(const void* X, int x_dtype, const uint8_t* W, const
                          &bs2_shift))
     return rc;
   // (one row whose K the GEMV cannot hold, K > 32768, takes the tiled kernel below)
+  if (few_unsplit(M, K, N) && (uintptr_t)X % 16 == 0 && (uintptr_t)W % 16 == 0)
+    return gemm_few(X, x_dtype, W, A8, AMAX, CODE2, offset, LUT, Y, R, epi, M, K, N, bs_shift, bs2_shift, 1, nullptr,
+                    stream);
   if (N >= 2 && skinny(K, N))
     return gemm_skinny(X, x_dtype, W, A8, AMAX, CODE2, offset, LUT, Y, R, epi, M, K, N, bs_shift, bs2_shift, stream);
   // vectorised output rows: 8 elements per 16-byte store
@@ -718,6 +746,9 @@ extern "C" int ttsp_nf4_gemm_swiglu(const void* X, int x_dtype, const uint8_t* W
   if (!W3 || !AMAX_3 || (A8_3 != nullptr) != (A8_1 != nullptr) || (A8_3 && !CODE2_3))
     return (int)hipErrorInvalidValue;
   if ((uintptr_t)X % 16 || (uintptr_t)W1 % 16 || (uintptr_t)W3 % 16) return (int)hipErrorInvalidValue;
+  if (few_pair(M, K, N))
+    return gemm_few_pair(X, x_dtype, W1, A8_1, AMAX_1, CODE2_1, offset_1, W3, A8_3, AMAX_3, CODE2_3, offset_3, LUT, Y,
+                         M, K, N, bs_shift, bs2_shift, stream);
   if (swiglu_skinny(M, K, N))
     return gemm_skinny_pair(X, x_dtype, W1, A8_1, AMAX_1, CODE2_1, offset_1, W3, A8_3, AMAX_3, CODE2_3, offset_3, LUT,
                             Y, M, K, N, bs_shift, bs2_shift, stream);
@@ -760,20 +791,35 @@ extern "C" int ttsp_nf4_gemm_split_norm(const void* X, int x_dtype, const uint8_
   if (int rc = gemm_mfma(X, x_dtype, W, A8, AMAX, CODE2, offset, LUT, Y, R, epi, M, K, N, bs_shift, bs2_shift,
                          gemm_plan(M, K, N), work, stream, false))
     return rc;
-  const dim3 grid((unsigned)N), block((unsigned)(64 * ((M / 8 + 63) / 64)));
-#define TTSP_RN(DTV, SV)                                                                                      \
-  hipLaunchKernelGGL((nf4_gemm_reduce_norm_kernel<DTV, SV>), grid, block, 0, stream, work, (uint16_t*)Y, \
-                     (const uint16_t*)R, epi, M, N, (const uint16_t*)G, eps, (uint16_t*)YN)
-#define TTSP_RS(DTV)                  \
-  if (splits == 2) TTSP_RN(DTV, 2);   \
-  else if (splits == 4) TTSP_RN(DTV, 4); \
-  else TTSP_RN(DTV, 8);
-  if (x_dtype == DT_BF16) {
-    TTSP_RS(DT_BF16)
-  } else {
-    TTSP_RS(DT_F16)
+  return gemm_reduce_norm(x_dtype, work, splits, Y, R, epi, M, N, G, eps, YN, stream);
+}
+
+// ---- 9 to 64 rows with the sums of K splits in a caller's workspace
+
+extern "C" int ttsp_nf4_gemm_few_splits(int M, int K, int N) { return few_splits(M, K, N); }
+
+extern "C" int ttsp_nf4_gemm_few(const void* X, int x_dtype, const uint8_t* W, const uint8_t* A8, const float* AMAX,
+                                 const float* CODE2, float offset, const float* LUT, void* Y, const void* R, int epi,
+                                 int M, int K, int N, int blocksize, int blocksize2, float* work, const void* G,
+                                 float eps, void* YN, hipStream_t stream) {
+  const int splits = few_splits(M, K, N);
+  if (splits < 1 || (splits > 1 && (!work || (uintptr_t)work % 16)) || (!Y && (splits == 1 || G)))
+    return (int)hipErrorInvalidValue;
+  int bs_shift, bs2_shift;
+  if (int rc = gemm_args(X, W, A8, AMAX, CODE2, LUT, Y ? Y : work, R, epi, M, K, N, blocksize, blocksize2, &bs_shift,
+                         &bs2_shift))
+    return rc;
+  if (G) {
+    if (splits == 1 || M % 8 || M > 64 * 8 * NRM_CH || !YN) return (int)hipErrorInvalidValue;
+    if ((uintptr_t)Y % 16 || (uintptr_t)YN % 16 || (uintptr_t)G % 16 || (epi && (uintptr_t)R % 16))
+      return (int)hipErrorInvalidValue;
   }
-#undef TTSP_RS
-#undef TTSP_RN
-  TTSP_RETURN_LAUNCH();
+  if (x_dtype != DT_BF16 && x_dtype != DT_F16) return (int)hipErrorInvalidValue;
+  if (int rc = gemm_few(X, x_dtype, W, A8, AMAX, CODE2, offset, LUT, Y, R, epi, M, K, N, bs_shift, bs2_shift, splits,
+                        work, stream))
+    return rc;
+  if (splits == 1 || !Y) return 0;
+  if (G) return gemm_reduce_norm(x_dtype, work, splits, Y, R, epi, M, N, G, eps, YN, stream);
+  const bool vec = M % 8 == 0 && (uintptr_t)Y % 16 == 0 && (!epi || (uintptr_t)R % 16 == 0);
+  return gemm_reduce(x_dtype, work, splits, Y, R, epi | (vec ? 4 : 0), M, N, stream);
 }

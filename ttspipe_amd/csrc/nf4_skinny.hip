@@ -1,9 +1,9 @@
-// NF4 matmul for a few activation rows (2 <= N <= 64; the split plan takes
-// 64 x 64 GEMM tiles from 33 rows, see nf4_gemm.hip): Y[N][M] = X[N][K] . W^T,
-// W in the bitsandbytes layout (nf4_gemv.hip describes it).
+// NF4 matmul for a few activation rows (2 <= N <= 16; from 9 rows larger
+// matrices take nf4_gemm_few.hip): Y[N][M] = X[N][K] . W^T, W in the
+// bitsandbytes layout (nf4_gemv.hip describes it).
 //
 // With few rows the weights are still the traffic - every weight byte is used
-// by at most 64 rows - so the kernel is shaped like the GEMV: the weight is
+// by at most 16 rows - so the kernel is shaped like the GEMV: the weight is
 // streamed once across the whole chip and the row dimension rides along on
 // the matrix cores.
 //
@@ -95,7 +95,9 @@ struct SkinnyW3 {
   float offset;
 };
 
-template <int DT, int R, int NT, int NW, int MS, bool NESTED, int TG = 1, bool PAIR = false>
+constexpr int NT = 1;  // 16-row tiles of X
+
+template <int DT, int R, int NW, int MS, bool NESTED, int TG = 1, bool PAIR = false>
 __global__ __launch_bounds__(64 * NW * TG) void nf4_skinny_kernel(
     const uint16_t* __restrict__ X, const uint8_t* __restrict__ W, const uint8_t* __restrict__ A8,
     const float* __restrict__ AMAX, const float* __restrict__ CODE2, float offset, const float* __restrict__ LUT,
@@ -298,29 +300,27 @@ __global__ __launch_bounds__(64 * NW * TG) void nf4_skinny_kernel(
   }
 }
 
-int skinny_max_k(int N);
+int skinny_max_k();
 
 bool skinny_pair_fits(int K, int N);
 
 // PAIR: the SwiGLU pair (w3 set), with half the row tiles a workgroup of the
-// single form where that has several, and one with two X tiles (each tile
-// slot is a tile of one matrix; a pair tile is two slots, which keeps the
-// loads in flight and the registers near the single form's; two X tiles and
-// four slots held one wave a SIMD: 9728 x 2560 at 32 rows 32.3 against
-// 24.7 us with one tile, at 17 rows 28.1 against 20.5).
-template <int DT, int RV, int NT, int NW, int MS, int TG = 1, bool PAIR = false>
+// single form where that has several (each tile slot is a tile of one matrix;
+// a pair tile is two slots, which keeps the loads in flight and the registers
+// near the single form's).
+template <int DT, int RV, int NW, int MS, int TG = 1, bool PAIR = false>
 static void launch_skinny(const void* X, const uint8_t* W, const uint8_t* A8, const float* AMAX, const float* CODE2,
                           float offset, const float* LUT, void* Y, const void* RES, int epi, int M, int K, int N,
                           int bs_shift, int bs2_shift, hipStream_t st, const SkinnyW3& w3) {
-  constexpr int R = PAIR && RV > 1 ? (NT >= 2 ? 1 : RV / 2) : RV;
+  constexpr int R = PAIR && RV > 1 ? RV / 2 : RV;
   const int tiles = (M + 16 * R - 1) / (16 * R);
   const dim3 grid((tiles + TG - 1) / TG);  // TG tiles a workgroup (the last may hold fewer)
   if (A8)
-    hipLaunchKernelGGL((nf4_skinny_kernel<DT, R, NT, NW, MS, true, TG, PAIR>), grid, dim3(64 * NW * TG), 0, st,
+    hipLaunchKernelGGL((nf4_skinny_kernel<DT, R, NW, MS, true, TG, PAIR>), grid, dim3(64 * NW * TG), 0, st,
                        (const uint16_t*)X, W, A8, AMAX, CODE2, offset, LUT, (uint16_t*)Y, (const uint16_t*)RES, epi,
                        M, K, N, bs_shift, bs2_shift, w3);
   else
-    hipLaunchKernelGGL((nf4_skinny_kernel<DT, R, NT, NW, MS, false, TG, PAIR>), grid, dim3(64 * NW * TG), 0, st,
+    hipLaunchKernelGGL((nf4_skinny_kernel<DT, R, NW, MS, false, TG, PAIR>), grid, dim3(64 * NW * TG), 0, st,
                        (const uint16_t*)X, W, A8, AMAX, CODE2, offset, LUT, (uint16_t*)Y, (const uint16_t*)RES, epi,
                        M, K, N, bs_shift, bs2_shift, w3);
 }
@@ -331,17 +331,13 @@ static void launch_skinny(const void* X, const uint8_t* W, const uint8_t* A8, co
 // tile a workgroup takes the smallest of 2, 3, 4, 5, 6, 8, 10 that holds the
 // run (every step past the run repeats a load: 2560 x 4096, runs of 4, 6.1
 // against 7.0 us with MS = 5 at 4 rows, 7.7 against 9.1 at 16), the other
-// forms 5 when the runs fit it, else SK_MAXS. R: with 512 or more
-// row tiles, several tiles a workgroup (each X fragment then serves R of them:
-// the activation traffic, which binds from 16 rows up, drops by R) - 4 for
-// 17-32 rows and 2 otherwise with 4 waves, 2 from 9 rows with 8 - else 1.
-// (Measured: at 9728 x 2560 two tiles cost 0.4-0.9 us more than one up to 8
-// rows and save 0.7 at 16; 32 rows 16.8 us with R = 4 against 18.3 with 2,
-// 64 rows 32.7 with R = 2 against 38.7 with 1; at 1024 x 2560 four waves take
-// 5.7 / 6.4 / 9.3 us for 4 / 16 / 32 rows against 6.9 / 9.1 / 14.2 with
-// eight, at 2560 x 4096 and 1024 x 3072 eight are faster.) Returns false when
-// no shape fits (see skinny_max_k).
-template <int DT, int NT, bool PAIR = false>
+// forms 5 when the runs fit it, else SK_MAXS. R: with 512 or more row tiles
+// two tiles a workgroup from 9 rows (each X fragment then serves both), else
+// one. (Measured: at 9728 x 2560 two tiles cost 0.4-0.9 us more than one up to
+// 8 rows and save 0.7 at 16; at 1024 x 2560 four waves take 5.7 / 6.4 us for 4
+// / 16 rows against 6.9 / 9.1 with eight, at 2560 x 4096 and 1024 x 3072 eight
+// are faster.) Returns false when no shape fits (see skinny_max_k).
+template <int DT, bool PAIR = false>
 static bool skinny_shape(const void* X, const uint8_t* W, const uint8_t* A8, const float* AMAX, const float* CODE2,
                          float offset, const float* LUT, void* Y, const void* RES, int epi, int M, int K, int N,
                          int bs_shift, int bs2_shift, hipStream_t st, const SkinnyW3& w3 = SkinnyW3{}) {
@@ -352,9 +348,9 @@ static bool skinny_shape(const void* X, const uint8_t* W, const uint8_t* A8, con
   if (tiles < 256 && nw < 8 && steps > 4 * 5) nw = 8;
   const int run = (steps + nw - 1) / nw;
   const bool ms5 = run <= 5;
-  const bool r2 = NT <= 2 && nw <= 8 && tiles >= 2 * 256 && N > 8;
+  const bool r2 = nw <= 8 && tiles >= 2 * 256 && N > 8;
 #define TTSP_L(RV, NWV, MSV)                                                                                 \
-  launch_skinny<DT, RV, NT, NWV, MSV, 1, PAIR>(X, W, A8, AMAX, CODE2, offset, LUT, Y, RES, epi, M, K, N, bs_shift, \
+  launch_skinny<DT, RV, NWV, MSV, 1, PAIR>(X, W, A8, AMAX, CODE2, offset, LUT, Y, RES, epi, M, K, N, bs_shift, \
                                                bs2_shift, st, w3)
 #define TTSP_MS(RV, NWV) \
   do {                   \
@@ -375,26 +371,16 @@ static bool skinny_shape(const void* X, const uint8_t* W, const uint8_t* A8, con
   // 2-3 row tiles a CU, up to 8 rows: three tiles a workgroup (12 waves, one
   // table) run in one round instead of two and a tail (9728 x 2560: 9.4
   // against 10.4 us at 4 rows, 10.5 against 10.7 at 8; 16 rows tie)
-  if constexpr (NT == 1) {
-    if (many && tiles < 3 * 256 && N <= 8 && nw == 4 && ms5) {
-      launch_skinny<DT, 1, 1, 4, 5, 3, PAIR>(X, W, A8, AMAX, CODE2, offset, LUT, Y, RES, epi, M, K, N, bs_shift,
-                                              bs2_shift, st, w3);
-      return true;
-    }
+  if (many && tiles < 3 * 256 && N <= 8 && nw == 4 && ms5) {
+    launch_skinny<DT, 1, 4, 5, 3, PAIR>(X, W, A8, AMAX, CODE2, offset, LUT, Y, RES, epi, M, K, N, bs_shift, bs2_shift,
+                                         st, w3);
+    return true;
   }
-  if constexpr (NT == 2) {
-    if (many && nw == 4 && ms5) { TTSP_L(4, 4, 5); return true; }
-  }
-  if constexpr (NT == 4 && !PAIR) {
-    if (many && nw == 4 && ms5) { TTSP_L(2, 4, 5); return true; }
-  }
-  if constexpr (NT <= 2) {
-    if (r2 && nw == 4) { TTSP_MS(2, 4); return true; }
-    if (r2) { TTSP_MS(2, 8); return true; }
-  }
+  if (r2 && nw == 4) { TTSP_MS(2, 4); return true; }
+  if (r2) { TTSP_MS(2, 8); return true; }
   if (nw == 4) TTSP_MS1(4);
   else if (nw == 8) TTSP_MS1(8);
-  else if constexpr (NT == 1 && !PAIR) TTSP_MS1(16);  // 1024 threads: 128 registers a lane, enough for one X tile only
+  else if constexpr (!PAIR) TTSP_MS1(16);
   else return false;
 #undef TTSP_MS1
 #undef TTSP_MS
@@ -405,30 +391,22 @@ static bool skinny_shape(const void* X, const uint8_t* W, const uint8_t* A8, con
 int gemm_skinny(const void* X, int dt, const uint8_t* W, const uint8_t* A8, const float* AMAX, const float* CODE2,
                 float offset, const float* LUT, void* Y, const void* RES, int epi, int M, int K, int N, int bs_shift,
                 int bs2_shift, hipStream_t st) {
-  if (N < 2 || N > 64 || K % 128 || K > skinny_max_k(N) || bs_shift < 6 || (uintptr_t)X % 16 || (uintptr_t)W % 16)
+  if (N < 2 || N > 16 || K % 128 || K > skinny_max_k() || bs_shift < 6 || (uintptr_t)X % 16 || (uintptr_t)W % 16)
     return (int)hipErrorInvalidValue;
-  const int NT = (N + 15) / 16;
   bool ok;
-#define TTSP_SK(DTV)                                                                                               \
-  do {                                                                                                             \
-    if (NT == 1) ok = skinny_shape<DTV, 1>(X, W, A8, AMAX, CODE2, offset, LUT, Y, RES, epi, M, K, N, bs_shift,      \
-                                           bs2_shift, st);                                                         \
-    else if (NT == 2) ok = skinny_shape<DTV, 2>(X, W, A8, AMAX, CODE2, offset, LUT, Y, RES, epi, M, K, N,          \
-                                                bs_shift, bs2_shift, st);                                          \
-    else ok = skinny_shape<DTV, 4>(X, W, A8, AMAX, CODE2, offset, LUT, Y, RES, epi, M, K, N, bs_shift, bs2_shift,   \
-                                   st);                                                                            \
-  } while (0)
-  if (dt == DT_BF16) TTSP_SK(DT_BF16);
-  else if (dt == DT_F16) TTSP_SK(DT_F16);
-  else return (int)hipErrorInvalidValue;
-#undef TTSP_SK
+  if (dt == DT_BF16)
+    ok = skinny_shape<DT_BF16>(X, W, A8, AMAX, CODE2, offset, LUT, Y, RES, epi, M, K, N, bs_shift, bs2_shift, st);
+  else if (dt == DT_F16)
+    ok = skinny_shape<DT_F16>(X, W, A8, AMAX, CODE2, offset, LUT, Y, RES, epi, M, K, N, bs_shift, bs2_shift, st);
+  else
+    return (int)hipErrorInvalidValue;
   if (!ok) return (int)hipErrorInvalidValue;
   TTSP_RETURN_LAUNCH();
 }
 
 // The SwiGLU pair in one launch: Y = silu(X W1^T) * (X W3^T), rounded and
 // with the bits of gemm_skinny(W1) then gemm_skinny(W3, epi 2) on its output.
-// Up to 32 rows (one or two X tiles) and K runs of at most 8 waves.
+// Up to 16 rows and K runs of at most 8 waves.
 int gemm_skinny_pair(const void* X, int dt, const uint8_t* W1, const uint8_t* A8_1, const float* AMAX_1,
                      const float* CODE2_1, float offset_1, const uint8_t* W3, const uint8_t* A8_3, const float* AMAX_3,
                      const float* CODE2_3, float offset_3, const float* LUT, void* Y, int M, int K, int N, int bs_shift,
@@ -437,25 +415,21 @@ int gemm_skinny_pair(const void* X, int dt, const uint8_t* W1, const uint8_t* A8
     return (int)hipErrorInvalidValue;
   const SkinnyW3 w3{W3, A8_3, AMAX_3, CODE2_3, offset_3};
   bool ok;
-#define TTSP_SK(DTV)                                                                                                \
-  do {                                                                                                              \
-    if (N <= 16) ok = skinny_shape<DTV, 1, true>(X, W1, A8_1, AMAX_1, CODE2_1, offset_1, LUT, Y, nullptr, 0, M, K, N, \
-                                                 bs_shift, bs2_shift, st, w3);                                      \
-    else ok = skinny_shape<DTV, 2, true>(X, W1, A8_1, AMAX_1, CODE2_1, offset_1, LUT, Y, nullptr, 0, M, K, N,        \
-                                         bs_shift, bs2_shift, st, w3);                                              \
-  } while (0)
-  if (dt == DT_BF16) TTSP_SK(DT_BF16);
-  else if (dt == DT_F16) TTSP_SK(DT_F16);
-  else return (int)hipErrorInvalidValue;
-#undef TTSP_SK
+  if (dt == DT_BF16)
+    ok = skinny_shape<DT_BF16, true>(X, W1, A8_1, AMAX_1, CODE2_1, offset_1, LUT, Y, nullptr, 0, M, K, N, bs_shift,
+                                     bs2_shift, st, w3);
+  else if (dt == DT_F16)
+    ok = skinny_shape<DT_F16, true>(X, W1, A8_1, AMAX_1, CODE2_1, offset_1, LUT, Y, nullptr, 0, M, K, N, bs_shift,
+                                    bs2_shift, st, w3);
+  else
+    return (int)hipErrorInvalidValue;
   if (!ok) return (int)hipErrorInvalidValue;
   TTSP_RETURN_LAUNCH();
 }
 
-bool skinny_pair_fits(int K, int N) { return N >= 2 && N <= 32 && K % 128 == 0 && K <= 8 * SK_MAXS * 128; }
+bool skinny_pair_fits(int K, int N) { return N >= 2 && N <= 16 && K % 128 == 0 && K <= 8 * SK_MAXS * 128; }
 
-// The longest row the skinny kernel takes for N activation rows: 16 waves of
-// SK_MAXS steps for one X tile (N <= 16), 8 waves otherwise.
-int skinny_max_k(int N) { return (N <= 16 ? 16 : 8) * SK_MAXS * 128; }
+// The longest row the skinny kernel takes: 16 waves of SK_MAXS steps.
+int skinny_max_k() { return 16 * SK_MAXS * 128; }
 
 }  // namespace ttsp

@@ -302,7 +302,7 @@ def prefill_block_chain(block, x, freqs_cis, mask, input_pos, *, xn=None, next_n
     # rotary / KV kernel, which adds them as the split's own reduce would
     part = None
     if qkv is None and rows_ok and a.wqkv._nf4_fast["M"] == (nh + 2 * nkv) * hd:
-        part = nf4gemv.matmul_partials(a.wqkv, xn)
+        part = nf4gemv.matmul_partials(a.wqkv, xn, few_rows=True)
     if part is None and qkv is None:
         qkv = nf4gemv.matmul(a.wqkv, xn)
         if qkv is None:
@@ -360,7 +360,7 @@ def prefill_block_chain(block, x, freqs_cis, mask, input_pos, *, xn=None, next_n
         if y is None:
             y = fastpath.decode_attention(q, k, v, mask, nh, nkv, hd)
         y = y.transpose(1, 2).contiguous().view(bsz, n, nh * hd)
-    hh = nf4gemv.matmul_norm(a.wo, y, fn.weight, fn.eps, epi=nf4gemv.EPI_RESIDUAL, operand=x)
+    hh = nf4gemv.matmul_norm(a.wo, y, fn.weight, fn.eps, epi=nf4gemv.EPI_RESIDUAL, operand=x, few_rows=True)
     if hh is not None:
         h, hn = hh
     else:
@@ -384,7 +384,8 @@ def prefill_block_chain(block, x, freqs_cis, mask, input_pos, *, xn=None, next_n
         u = None if g is None else nf4gemv.matmul(ff.w3, hn, epi=nf4gemv.EPI_SILU_GATE, operand=g)
     oo = None
     if u is not None and next_norm is not None:
-        oo = nf4gemv.matmul_norm(ff.w2, u, next_norm.weight, next_norm.eps, epi=nf4gemv.EPI_RESIDUAL, operand=h)
+        oo = nf4gemv.matmul_norm(ff.w2, u, next_norm.weight, next_norm.eps, epi=nf4gemv.EPI_RESIDUAL, operand=h,
+                                 few_rows=True)
     if oo is not None:
         out, out_n = oo
     else:

@@ -10,9 +10,11 @@ bitsandbytes put them; `libttsp_hip.so` reads them directly:
   stream of the packed weight: 256-byte wave loads, both codes of a byte
   looked up at once in an LDS table, fp32 fma chains and DPP lane sums in a
   fixed order (so results are reproducible bit for bit);
-* two or more rows go to the GEMM (`csrc/nf4_gemm.hip`), where each K-step's
-  weight tile is dequantised into LDS and multiplied by
-  `v_mfma_f32_32x32x16`: one dequantisation serves a whole tile of rows.
+* two or more rows go to the matrix cores, one dequantisation serving a tile
+  of rows: the few-row kernels up to 64 (`csrc/nf4_skinny.hip`,
+  `csrc/nf4_gemm_few.hip`), the tiled ones above (`csrc/nf4_gemm.hip`,
+  `csrc/nf4_gemm_dl.hip`), and past 512 rows one dequantisation a call
+  (`csrc/nf4_gemm_dense.hip`).
 
 Unlike the reference (fp16 only, nf4gemv.py:439) both fp16 and bf16
 activations are served; anything else is declined (`None`), exactly where the
@@ -203,8 +205,12 @@ def matmul(module, x, *, epi: int = EPI_NONE, operand=None, out=None):
         return None
     lib = _lib.lib()
     dense = lib.ttsp_nf4_gemm_dense_splits(M, K, rows) if rows >= DENSE_MIN_ROWS else 0
-    splits = lib.ttsp_nf4_gemm_splits(M, K, rows) if rows > 1 and not dense else 1
-    if dense:
+    few = lib.ttsp_nf4_gemm_few_splits(M, K, rows) if FEW_SPLIT_ROWS <= rows <= FEW_MAX_ROWS else 0
+    splits = lib.ttsp_nf4_gemm_splits(M, K, rows) if rows > 1 and not dense and not few else 1
+    if few:
+        work = torch.empty(few * rows * M, dtype=torch.float32, device=x.device) if few > 1 else None
+        rc = _few(lib, fast, flat, dt, rows, out, operand, epi, work)
+    elif dense:
         # the dequantised weight, then (K split) the partial sums
         work = torch.empty(2 * M * K + (4 * dense * rows * M if dense > 1 else 0), dtype=torch.uint8, device=x.device)
         rc = lib.ttsp_nf4_gemm_dense(
@@ -230,6 +236,18 @@ def matmul(module, x, *, epi: int = EPI_NONE, operand=None, out=None):
     return out.view(*x.shape[:-1], M)
 
 
+#: Rows the few-row kernel takes (`ttsp_nf4_gemm_few`), and from how many `matmul` lets it split K: at fewer the
+#: reduce launch costs what the split saves, unless the reduce runs anyway (`matmul_norm(few_rows=True)`).
+FEW_MIN_ROWS, FEW_SPLIT_ROWS, FEW_MAX_ROWS = 9, 33, 64
+
+
+def _few(lib, fast, x, dt, rows, out, operand, epi, work, norm_weight=None, eps=0.0, out_n=None):
+    return lib.ttsp_nf4_gemm_few(
+        x.data_ptr(), dt, fast["w"], fast["a8"], fast["amax"], fast["code2"], fast["offset"], fast["lut"].data_ptr(),
+        _lib.ptr(out), _lib.ptr(operand) if epi else 0, epi, fast["M"], fast["K"], rows, fast["bs"], fast["bs2"],
+        _lib.ptr(work), _lib.ptr(norm_weight), float(eps), _lib.ptr(out_n), _lib.stream())
+
+
 #: From this many rows `matmul` and `matmul_swiglu` ask for the dense form (the weight dequantised once a call into a
 #: workspace): below it the kernels that read the codes in place are as fast.
 DENSE_MIN_ROWS = 513
@@ -244,11 +262,12 @@ def _dense(M: int, K: int, rows: int) -> bool:
 NORM_MAX_M = 4096
 
 
-def matmul_partials(module, x):
+def matmul_partials(module, x, *, few_rows: bool = False):
     """`(work, splits)`: the K-split launch of `matmul(module, x)` without its
     reduce, work the fp32 partial sums [splits, rows, M] for a consumer that
     adds them in split order; None where the shape runs unsplit (or the
-    kernels do not take the call)."""
+    kernels do not take the call). `few_rows`: split 9 to 32 rows too, whose
+    `matmul` runs unsplit (it would pay a reduce launch; the consumer does not)."""
     import torch
 
     fast = getattr(module, "_nf4_fast", None)
@@ -264,25 +283,31 @@ def matmul_partials(module, x):
     if rows < 2 or _dense(M, K, rows):
         return None
     lib = _lib.lib()
-    splits = lib.ttsp_nf4_gemm_splits(M, K, rows)
+    few = lib.ttsp_nf4_gemm_few_splits(M, K, rows) if few_rows or FEW_SPLIT_ROWS <= rows <= FEW_MAX_ROWS else 0
+    splits = few or lib.ttsp_nf4_gemm_splits(M, K, rows)
     if splits < 2:
         return None
     work = torch.empty(splits, rows, M, dtype=torch.float32, device=x.device)
-    rc = lib.ttsp_nf4_gemm_partials(
-        x.data_ptr(), dt, fast["w"], fast["a8"], fast["amax"], fast["code2"], fast["offset"],
-        fast["lut"].data_ptr(), M, K, rows, fast["bs"], fast["bs2"], work.data_ptr(), splits, _lib.stream())
+    if few:
+        rc = _few(lib, fast, x, dt, rows, None, None, EPI_NONE, work)
+    else:
+        rc = lib.ttsp_nf4_gemm_partials(
+            x.data_ptr(), dt, fast["w"], fast["a8"], fast["amax"], fast["code2"], fast["offset"],
+            fast["lut"].data_ptr(), M, K, rows, fast["bs"], fast["bs2"], work.data_ptr(), splits, _lib.stream())
     if rc:
         raise RuntimeError(f"ttsp_nf4_gemm_partials failed: hipError_t {rc}")
     _stats["fast"] += 1
     return work, splits
 
 
-def matmul_norm(module, x, norm_weight, eps: float, *, epi: int = EPI_NONE, operand=None):
+def matmul_norm(module, x, norm_weight, eps: float, *, epi: int = EPI_NONE, operand=None, few_rows: bool = False):
     """`(y, rms_norm(y))` for several rows with the norm folded into the
     split-K reduce, or None where that form does not serve the call (one row,
     an unsplit shape, M over NORM_MAX_M); y is `matmul(module, x, epi=epi,
     operand=operand)` and the second output is `fusedops.rms_norm(y,
-    norm_weight, eps)`, both bit for bit."""
+    norm_weight, eps)`, both bit for bit. `few_rows` serves 9 to 32 rows too,
+    whose `matmul` runs unsplit: y is then the sum of K splits (the norm's
+    launch adds them), rounded as a split's reduce rounds."""
     import torch
 
     fast = getattr(module, "_nf4_fast", None)
@@ -306,17 +331,21 @@ def matmul_norm(module, x, norm_weight, eps: float, *, epi: int = EPI_NONE, oper
         if operand.device != x.device or not operand.is_contiguous() or operand.data_ptr() % 16:
             return None
     lib = _lib.lib()
-    splits = lib.ttsp_nf4_gemm_splits(M, K, rows)
+    few = lib.ttsp_nf4_gemm_few_splits(M, K, rows) if few_rows or FEW_SPLIT_ROWS <= rows <= FEW_MAX_ROWS else 0
+    splits = few or lib.ttsp_nf4_gemm_splits(M, K, rows)
     if splits not in (2, 4, 8):
         return None
     out = torch.empty((rows, M), dtype=x.dtype, device=x.device)
     out_n = torch.empty((rows, M), dtype=x.dtype, device=x.device)
     work = torch.empty(splits * rows * M, dtype=torch.float32, device=x.device)
-    rc = lib.ttsp_nf4_gemm_split_norm(
-        x.data_ptr(), dt, fast["w"], fast["a8"], fast["amax"], fast["code2"], fast["offset"],
-        fast["lut"].data_ptr(), out.data_ptr(), _lib.ptr(operand) if epi else 0, epi, M, K, rows,
-        fast["bs"], fast["bs2"], work.data_ptr(), splits, norm_weight.data_ptr(), float(eps), out_n.data_ptr(),
-        _lib.stream())
+    if few:
+        rc = _few(lib, fast, x, dt, rows, out, operand, epi, work, norm_weight, eps, out_n)
+    else:
+        rc = lib.ttsp_nf4_gemm_split_norm(
+            x.data_ptr(), dt, fast["w"], fast["a8"], fast["amax"], fast["code2"], fast["offset"],
+            fast["lut"].data_ptr(), out.data_ptr(), _lib.ptr(operand) if epi else 0, epi, M, K, rows,
+            fast["bs"], fast["bs2"], work.data_ptr(), splits, norm_weight.data_ptr(), float(eps), out_n.data_ptr(),
+            _lib.stream())
     if rc:
         raise RuntimeError(f"ttsp_nf4_gemm_split_norm failed: hipError_t {rc}")
     _stats["fast"] += 1
