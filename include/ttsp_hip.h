@@ -64,8 +64,7 @@ enum { TTSP_FAST_SYNC_WORDS = 192, TTSP_FAST_SYNC_FAILED = 128 };
 
 /* Y[N][M] = epi(X[N][K] . dequant(W)^T). N == 1 runs the HBM-bound GEMV (rows
  * of up to 32768 codes; a longer row takes the tiled kernel), N > 1 the MFMA
- * GEMM (LDS-staged dequantisation; from 256 to 512 rows on large shapes,
- * direct-to-LDS operand streams). epi 1: Y = round(R + round(XW)); epi 2:
+ * kernels (few rows, tiles). epi 1: Y = round(R + round(XW)); epi 2:
  * Y = round(round(silu(R)) * round(XW)); R has Y's shape. Requires K % 128 == 0,
  * K % blocksize == 0, blocksize a power of two >= 64, blocksize2 a power of two
  * (nested only), 16-byte aligned X and W. A8 == NULL selects plain scales.
@@ -79,11 +78,13 @@ int ttsp_nf4_gemm(const void* X, int x_dtype, const uint8_t* W, const uint8_t* A
 /* How many K splits ttsp_nf4_gemm_split uses for this shape (1: none, then no
  * workspace is needed). The split is chosen so the output tiles times the
  * splits give every CU a workgroup; from 256 to 512 rows on large or long-K
- * shapes it is the direct-to-LDS kernel's (1, 2 or 4, at most 64 K-steps of
- * 64 codes per split). Host-only. Replaces: the reference's
+ * shapes it is 1, 2 or 4 with at most 64 K-steps of 64 codes per split. Host-only. Replaces: the reference's
  * slicing of the rows into MAX_N = 32 launches (app/engine/nf4gemv.py:460-477),
  * which it does instead of splitting K. */
 int ttsp_nf4_gemm_splits(int M, int K, int N);
+/* The splits that are fastest where the caller may choose: either
+ * ttsp_nf4_gemm_splits' or 1 (then ttsp_nf4_gemm). */
+int ttsp_nf4_gemm_tile_splits(int M, int K, int N);
 
 /* ttsp_nf4_gemm with the K loop split `splits` ways (exactly
  * ttsp_nf4_gemm_splits(M, K, N), N > 1): each split writes fp32 partial sums
@@ -122,9 +123,9 @@ int ttsp_nf4_gemm_split_norm(const void* X, int x_dtype, const uint8_t* W, const
  * Y[N][M] = round(round(silu(round(X . W1^T))) * round(X . W3^T)), W1 and W3
  * of one shape [M, K] with the same blocksize and nesting, every value the
  * bits of ttsp_nf4_gemm(W1) then ttsp_nf4_gemm(W3, epi 2, R = the first's
- * output). Served where both of those would run the direct-to-LDS kernel
+ * output). Served where both of those would run the tile kernel
  * unsplit (ttsp_nf4_gemm_swiglu_fits; e.g. 385-512 rows of 9728 x 2560) or
- * the few-row kernel unsplit (3-32 rows, K up to 10240); other shapes return
+ * the skinny or few-row kernel unsplit (3-32 rows; up to 16, K up to 10240); other shapes return
  * hipErrorInvalidValue and the caller runs the two launches.
  * 16-byte aligned X, W1, W3. Replaces: w1 then w3 with the SwiGLU gate in
  * the fork's FeedForward for S > 1 (the unfused block the reference runs

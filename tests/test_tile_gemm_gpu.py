@@ -1,0 +1,81 @@
+"""The tiled NF4 product (csrc/nf4_gemm_tile.hip) in each of its forms: 64, 128
+and 256 weight rows a workgroup, one or both K halves, unsplit and split."""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as o
+from tests.conftest import beyond_rounding_error
+from tests.gpuutil import bits, dt_code, from_bits, randn_bits
+from tests.nf4data import oracle_args, random_layer, to_linear
+
+
+@pytest.fixture(scope="module")
+def nf4():
+    from ttspipe_amd import nf4gemv
+
+    assert nf4gemv.install()
+    return nf4gemv
+
+
+def test_tile_splits_follow_the_split_plan():
+    """The split plan's, or 1 in place of 2 at 256 rows and more where the row
+    is too wide for the norm's reduce."""
+    from ttspipe_amd import _lib
+
+    lib = _lib.load()
+    for M, K in ((9728, 2560), (6144, 2560), (2560, 9728), (2560, 4096), (4096, 2560), (1536, 1024), (1540, 2560)):
+        for N in (65, 100, 128, 200, 256, 257, 384, 400, 512):
+            plan, tile = lib.ttsp_nf4_gemm_splits(M, K, N), lib.ttsp_nf4_gemm_tile_splits(M, K, N)
+            assert tile == plan or (tile == 1 and plan == 2 and N >= 256 and M > 4096)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,rows,nested,bs,bs2,dtype,epi", [
+    ((64, 128), 65, True, 64, 256, torch.bfloat16, 0),       # KG 2: one K-step a half
+    ((70, 384), 129, False, 128, 0, torch.float16, 1),       # three steps a half, one activation row in the last tile
+    ((1542, 2688), 200, True, 64, 16, torch.bfloat16, 2),    # 21 steps a half: scales resolved twice; M % 4 == 2
+    ((9728, 2560), 256, True, 64, 256, torch.float16, 0),    # 128 rows a workgroup
+    ((9000, 2560), 250, False, 256, 0, torch.bfloat16, 1),   # the same, ragged both ways
+    ((9730, 2560), 500, True, 64, 32, torch.bfloat16, 0),    # 256 rows a workgroup, M % 4 == 2
+    ((9728, 2176), 512, True, 128, 256, torch.float16, 2),   # 34 steps: a ring remainder of one past two chunks
+    ((9728, 2048), 400, False, 64, 0, torch.bfloat16, 0),    # 32 steps: a remainder of two
+    ((2560, 9728), 512, True, 64, 256, torch.bfloat16, 1),   # four K splits
+])
+def test_tile_gemm_against_fp64(nf4, orc, shape, rows, nested, bs, bs2, dtype, epi):
+    """Within the 2e-3 bar beyond the output's own rounding, nothing stored
+    past N, every epilogue."""
+    (M, K), dt = shape, dt_code(dtype)
+    layer = random_layer(M, K, nested, seed=M + rows, bs=bs, bs2=bs2 or 256)
+    lin = to_linear(layer, dtype)
+    assert nf4.prepare(lin)
+    xb = randn_bits(rows * K, dtype, seed=rows, scale=0.5)
+    x = from_bits(xb, dtype).view(rows, K)
+    rb = randn_bits(rows * M, dtype, seed=5)
+    guard = torch.full((rows + 1, M), 7.0, dtype=dtype, device="cuda")
+    y = nf4.matmul(lin, x, epi=epi, operand=from_bits(rb, dtype).view(rows, M) if epi else None, out=guard[:rows])
+    assert bool((guard[rows] == 7.0).all())
+    sample = np.unique(np.r_[0:rows:17, rows - 1])
+    ref = orc.nf4_gemm_ref(xb.reshape(rows, K)[sample], dt, **oracle_args(layer), M=M, K=K, N=sample.size, bs=bs,
+                           bs2=bs2 or 256).astype(np.float64).reshape(sample.size, M)
+    if epi:
+        ref = o.to_f32(o.from_f32(ref.astype(np.float32), dt), dt).astype(np.float64)
+        r = o.to_f32(rb, dt).astype(np.float64).reshape(rows, M)[sample]
+        silu = o.to_f32(o.from_f32((r / (1 + np.exp(-r))).astype(np.float32), dt), dt).astype(np.float64)
+        ref = r + ref if epi == 1 else silu * ref
+    got = o.to_f32(bits(y), dt).reshape(rows, M)[sample]
+    assert beyond_rounding_error(got, ref, dt) < 2e-3
+
+
+@pytest.mark.gpu
+def test_tile_gemm_is_reproducible(nf4):
+    """Twenty runs of each form give the same bits (a stage refilled while
+    another wave still reads it would not)."""
+    for (M, K), rows in (((1542, 2688), 200), ((9728, 2560), 256), ((9728, 2560), 512)):
+        lin = to_linear(random_layer(M, K, True, seed=3), torch.bfloat16)
+        assert nf4.prepare(lin)
+        x = from_bits(randn_bits(rows * K, torch.bfloat16, seed=4), torch.bfloat16).view(rows, K)
+        first = nf4.matmul(lin, x).clone()
+        for _ in range(20):
+            assert torch.equal(nf4.matmul(lin, x).view(torch.int16), first.view(torch.int16))

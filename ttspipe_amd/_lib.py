@@ -52,6 +52,7 @@ FAST_SYNC_WORDS, FAST_SYNC_FAILED = 192, 128
 SIGNATURES: dict[str, list] = {
     "ttsp_nf4_gemm": [_vp, _i, _vp, _vp, _vp, _vp, _f, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp],
     "ttsp_nf4_gemm_splits": [_i, _i, _i],
+    "ttsp_nf4_gemm_tile_splits": [_i, _i, _i],
     "ttsp_nf4_gemm_split": [_vp, _i, _vp, _vp, _vp, _vp, _f, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp, _i, _vp],
     "ttsp_nf4_gemm_partials": [_vp, _i, _vp, _vp, _vp, _vp, _f, _vp, _i, _i, _i, _i, _i, _vp, _i, _vp],
     "ttsp_nf4_gemm_split_norm": [_vp, _i, _vp, _vp, _vp, _vp, _f, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp, _i,

@@ -1,302 +1,12 @@
-// NF4 GEMM for several activation rows (prompt prefill): Y[N][M] = X[N][K] . W^T
-// with W the bitsandbytes NF4 weight (nf4_gemv.hip gives the layout).
-//
-// Each workgroup owns a BM x BN tile of the output (BM weight rows, BN input
-// rows), WM x WN waves of 32x32 MFMA blocks. Per K-step of 64 codes, the
-// workgroup's threads
-//   * dequantise BM x 64 weights, 8 packed bytes (16 codes) each, as
-//     round(code * scale) in the activation type - the exact value
-//     bitsandbytes' dequantize_4bit produces, so the product is the dense
-//     fork's matmul on identical weights - straight into an LDS A tile (the
-//     16 code points in LDS: 64 lanes hit at most 16 banks, no conflicts; one
-//     hardware pack-convert rounds two products);
-//   * copy BN x 64 activations into an LDS B tile;
-// and the waves run v_mfma_f32_32x32x16 over their sub-tiles, fp32
-// accumulate. The packed weights, scales and activations of the next PF
-// steps are in flight in registers while a step multiplies (the K loop is
-// latency-bound otherwise: a lone workgroup waits a memory round trip per
-// step), and LDS is double-buffered. Rows are padded to 72 elements (144 B) so
-// the 16-byte operand reads of 16 consecutive rows hit disjoint banks. The
-// output tile is rounded, staged in LDS and written (with the epilogue) as
-// 16-byte row pieces.
-//
-// MFMA 32x32x16 operand layout: lane l supplies row (l % 32) of A and column
-// (l % 32) of B, each as 8 consecutive k at 8 * (l / 32); accumulator r of
-// lane l is D[8*(r/4) + 4*(l/32) + r%4][l % 32]. A and B only need to agree on
-// which k a lane carries, so any k permutation inside a step is harmless.
+// The launch plans of the NF4 matrix products, the reduce kernels of their K
+// splits and the C entry points. The products themselves: nf4_gemv.hip (one
+// and two rows), nf4_skinny.hip (to 16), nf4_gemm_few.hip (9 to 64),
+// nf4_gemm_tile.hip (65 to 512) and nf4_gemm_dense.hip (more).
 #include "gemv_common.h"
 
 namespace ttsp {
 
-typedef __bf16 bf16x8_v __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8_v __attribute__((ext_vector_type(8)));
-typedef float f32x16_v __attribute__((ext_vector_type(16)));
-typedef __bf16 bf16x2_v __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x2_v __attribute__((ext_vector_type(2)));
-typedef float f32x2_v __attribute__((ext_vector_type(2)));
-
-constexpr int KT = 64;        // codes per K-step (one bs=64 scale block)
-constexpr int LROW = KT + 8;  // LDS row stride in elements
-
-template <int DT>
-__device__ __forceinline__ f32x16_v mfma32(uint4 a, uint4 b, f32x16_v c) {
-  if constexpr (DT == DT_BF16)
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_v, a),
-                                                   __builtin_bit_cast(bf16x8_v, b), c, 0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_v, a),
-                                                  __builtin_bit_cast(f16x8_v, b), c, 0, 0, 0);
-}
-
-// Two fp32 values, each already rounded to fp32, to the activation type
-// (round to nearest even, one hardware pack-convert); lo in the low half.
-template <int DT>
-__device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-  const f32x2_v v = {opaque(lo), opaque(hi)};
-  if constexpr (DT == DT_BF16)
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_v));
-  else
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2_v));
-}
-
-// WM x WN waves; each wave covers (BM/WM) x (BN/WN) with 32x32 MFMA blocks;
-// PF K-steps of operands in flight (nsteps a multiple of PF).
-template <int DT, int BM, int BN, int WM, int WN, bool NESTED, int PF>
-__global__ __launch_bounds__(64 * WM * WN) void nf4_gemm_kernel(
-    const uint16_t* __restrict__ X, const uint8_t* __restrict__ W, const uint8_t* __restrict__ A8,
-    const float* __restrict__ AMAX, const float* __restrict__ CODE2, float offset,
-    const float* __restrict__ LUT, uint16_t* __restrict__ Y, const uint16_t* __restrict__ R,
-    int epi, int M, int K, int N, int bs_shift, int bs2_shift, float* __restrict__ YP) {
-  constexpr int GEMM_THREADS = 64 * WM * WN;
-  constexpr int TM = BM / WM / 32, TN = BN / WN / 32;  // MFMA blocks per wave
-  constexpr int A_CH = BM * (KT / 16);                                  // 8-byte packed chunks (16 codes) per step
-  constexpr int A_PER_T = (A_CH + GEMM_THREADS - 1) / GEMM_THREADS;     // per thread (the last partly idle)
-  constexpr int B_PER_T = BN * (KT / 8) / GEMM_THREADS;                 // 16-byte activation chunks per thread
-  static_assert(B_PER_T >= 1 && BN * (KT / 8) % GEMM_THREADS == 0, "tile too small for the workgroup");
-  static_assert(GEMM_THREADS >= 256, "the code tables are filled one entry per thread");
-
-  // the operand tiles (two buffers each); after the K loop the same memory
-  // holds the output tile, BN rows of BM + 8 elements
-  constexpr int YROW = BM + 8;
-  constexpr int OPS = 2 * (BM + BN) * LROW, YS = BN * YROW;
-  __shared__ __align__(16) uint16_t smem[OPS > YS ? OPS : YS];
-  uint16_t (*As)[BM * LROW] = reinterpret_cast<uint16_t (*)[BM * LROW]>(smem);
-  uint16_t (*Bs)[BN * LROW] = reinterpret_cast<uint16_t (*)[BN * LROW]>(smem + 2 * BM * LROW);
-  __shared__ float2 lut2_s[256];  // byte -> (code of its high nibble, code of its low nibble)
-  __shared__ float code2_s[NESTED ? 256 : 1];
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave / WN, wn = wave % WN;
-  const int m0 = blockIdx.x * BM, n0 = blockIdx.y * BN;
-  // split-K (gridDim.z > 1): workgroup z takes K-steps [z S, z S + S) and
-  // writes its fp32 partial sums to YP[z][n][m]; a second kernel adds them
-  const int nsteps = K / KT / gridDim.z, kbase = blockIdx.z * nsteps * KT;
-  const size_t rowbytes = (size_t)K / 2;
-
-  if (tid < 256) lut2_s[tid] = make_float2(LUT[tid >> 4], LUT[tid & 15]);
-  if constexpr (NESTED)
-    if (tid < 256) code2_s[tid] = CODE2[tid];
-
-  struct Stage {
-    uint2 w[A_PER_T];
-    float s[A_PER_T];
-    uint32_t a8[NESTED ? A_PER_T : 1];
-    uint4 x[B_PER_T];
-  };
-  Stage stg[PF];
-
-  // step clamped into range: the loads past the last step repeat it and go unused
-  auto load_step = [&](Stage& sg, int step) {
-    const int k0 = kbase + min(step, nsteps - 1) * KT;
-#pragma unroll
-    for (int i = 0; i < A_PER_T; ++i) {
-      const int c = min(tid + i * GEMM_THREADS, A_CH - 1);  // chunk: row c / 4, codes 16 (c % 4) ..
-      const int row = min(m0 + c / (KT / 16), M - 1);
-      const int kc = k0 + (c % (KT / 16)) * 16;
-      typedef uint32_t u32x2_v __attribute__((ext_vector_type(2)));
-      const u32x2_v v = __builtin_nontemporal_load(
-          reinterpret_cast<const u32x2_v*>(W + (size_t)row * rowbytes + kc / 2));
-      sg.w[i] = make_uint2(v.x, v.y);
-      const long long b = ((long long)row * K + kc) >> bs_shift;
-      if constexpr (NESTED) {
-        sg.a8[i] = A8[b];
-        sg.s[i] = AMAX[b >> bs2_shift];
-      } else {
-        sg.s[i] = AMAX[b];
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < B_PER_T; ++i) {
-      const int c = tid + i * GEMM_THREADS;  // chunk: row c/8, 8 elements at (c%8)*8
-      const int n = min(n0 + c / (KT / 8), N - 1);
-      sg.x[i] = *reinterpret_cast<const uint4*>(X + (size_t)n * K + k0 + (c % (KT / 8)) * 8);
-    }
-  };
-  auto store_step = [&](const Stage& sg, int buf) {
-#pragma unroll
-    for (int i = 0; i < A_PER_T; ++i) {
-      const int c = tid + i * GEMM_THREADS;
-      if (A_CH % GEMM_THREADS && c >= A_CH) break;
-      float s = sg.s[i];
-      if constexpr (NESTED) s = __fadd_rn(__fmul_rn(code2_s[sg.a8[i]], s), offset);
-      const uint32_t wv[2] = {sg.w[i].x, sg.w[i].y};
-      // one lookup per byte (both codes), all 8 in flight before the first
-      // is used (one LDS round trip per step instead of one per byte)
-      float cv[16];
-#pragma unroll
-      for (int q = 0; q < 2; ++q)
-#pragma unroll
-        for (int bb = 0; bb < 4; ++bb) {
-          const float2 pc = lut2_s[(wv[q] >> (8 * bb)) & 0xffu];
-          cv[2 * (q * 4 + bb)] = pc.x;
-          cv[2 * (q * 4 + bb) + 1] = pc.y;
-        }
-      uint32_t o[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) o[e] = pack2<DT>(__fmul_rn(cv[2 * e], s), __fmul_rn(cv[2 * e + 1], s));
-      uint4* dst = reinterpret_cast<uint4*>(&As[buf][(c / (KT / 16)) * LROW + (c % (KT / 16)) * 16]);
-#pragma unroll
-      for (int q = 0; q < 2; ++q) dst[q] = make_uint4(o[4 * q], o[4 * q + 1], o[4 * q + 2], o[4 * q + 3]);
-    }
-#pragma unroll
-    for (int i = 0; i < B_PER_T; ++i) {
-      const int c = tid + i * GEMM_THREADS;
-      const int n = n0 + c / (KT / 8);
-      *reinterpret_cast<uint4*>(&Bs[buf][(c / (KT / 8)) * LROW + (c % (KT / 8)) * 8]) =
-          n < N ? sg.x[i] : make_uint4(0, 0, 0, 0);
-    }
-  };
-
-  f32x16_v acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-
-#pragma unroll
-  for (int i = 0; i < PF; ++i) load_step(stg[i], i);
-  __syncthreads();  // lut2_s / code2_s
-  store_step(stg[0], 0);
-  __syncthreads();
-  load_step(stg[0], PF);
-  // Step s multiplies buffer s & 1 while the same waves dequantise step s + 1
-  // into the other buffer (read by nobody since the previous barrier); one
-  // barrier per step. The last step stages a repeat of itself, unread.
-  for (int s0 = 0; s0 < nsteps; s0 += PF) {
-#pragma unroll
-    for (int i = 0; i < PF; ++i) {
-      const int step = s0 + i;
-      const int buf = step & 1;
-      const uint16_t* as = As[buf];
-      const uint16_t* bs = Bs[buf];
-#pragma unroll
-      for (int kk = 0; kk < KT / 16; ++kk) {
-        const int ko = kk * 16 + (lane >> 5) * 8;
-        uint4 af[TM], bf[TN];
-#pragma unroll
-        for (int a = 0; a < TM; ++a)
-          af[a] = *reinterpret_cast<const uint4*>(as + (wm * (BM / WM) + a * 32 + (lane & 31)) * LROW + ko);
-#pragma unroll
-        for (int b = 0; b < TN; ++b)
-          bf[b] = *reinterpret_cast<const uint4*>(bs + (wn * (BN / WN) + b * 32 + (lane & 31)) * LROW + ko);
-#pragma unroll
-        for (int a = 0; a < TM; ++a)
-#pragma unroll
-          for (int b = 0; b < TN; ++b) acc[a][b] = mfma32<DT>(af[a], bf[b], acc[a][b]);
-      }
-      store_step(stg[(i + 1) % PF], buf ^ 1);
-      __syncthreads();
-      load_step(stg[(i + 1) % PF], step + 1 + PF);
-    }
-  }
-
-  if (YP) {  // split-K partials: 4 consecutive rows m per 16-byte store
-    // (n * M + m is a multiple of 4 only when M is: m always is)
-    float* yp = YP + (size_t)blockIdx.z * N * M;
-    const bool v4 = (M & 3) == 0;
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int n = n0 + wn * (BN / WN) + j * 32 + (lane & 31);
-        if (n >= N) continue;
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int m = m0 + wm * (BM / WM) + i * 32 + 8 * g + 4 * (lane >> 5);
-          if (v4 && m + 4 <= M) {
-            *reinterpret_cast<float4*>(yp + (size_t)n * M + m) =
-                make_float4(acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]);
-          } else {
-            for (int c = 0; c < 4 && m + c < M; ++c) yp[(size_t)n * M + m + c] = acc[i][j][4 * g + c];
-          }
-        }
-      }
-    return;
-  }
-  // epilogue: accumulator r of lane l is (row 8*(r/4) + 4*(l/32) + r%4, column
-  // l%32); each value is rounded to the activation type and the tile goes
-  // through LDS as Y rows (the operand buffers are free after the last
-  // barrier), so the stores and the operand reads are 16 bytes per lane
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int nl = wn * (BN / WN) + j * 32 + (lane & 31);
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int ml = wm * (BM / WM) + i * 32 + 8 * g + 4 * (lane >> 5);
-        const uint32_t lo = (uint32_t)Elem<DT>::store(acc[i][j][4 * g]) |
-                            ((uint32_t)Elem<DT>::store(acc[i][j][4 * g + 1]) << 16);
-        const uint32_t hi = (uint32_t)Elem<DT>::store(acc[i][j][4 * g + 2]) |
-                            ((uint32_t)Elem<DT>::store(acc[i][j][4 * g + 3]) << 16);
-        *reinterpret_cast<uint2*>(&smem[nl * YROW + ml]) = make_uint2(lo, hi);
-      }
-    }
-  __syncthreads();
-  const bool vec = (epi & 4) != 0;  // M % 8 == 0 and Y, R 16-byte aligned (host)
-  const int ep = epi & 3;
-  for (int cc = tid; cc < BN * (BM / 8); cc += GEMM_THREADS) {
-    const int nl = cc / (BM / 8), ml = (cc % (BM / 8)) * 8;
-    const int n = n0 + nl, m = m0 + ml;
-    if (n >= N || m >= M) continue;
-    const uint4 yv = *reinterpret_cast<const uint4*>(&smem[nl * YROW + ml]);
-    const uint32_t yw[4] = {yv.x, yv.y, yv.z, yv.w};
-    const size_t o = (size_t)n * M + m;
-    if (vec && m + 8 <= M) {
-      uint32_t rw[4] = {0u, 0u, 0u, 0u};
-      if (ep) {
-        const uint4 rv = *reinterpret_cast<const uint4*>(R + o);
-        rw[0] = rv.x, rw[1] = rv.y, rw[2] = rv.z, rw[3] = rv.w;
-      }
-      uint32_t ow[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        uint32_t h2[2];
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const float y = Elem<DT>::load(yw[q] >> (16 * u));
-          const float r = Elem<DT>::load(rw[q] >> (16 * u));
-          float v = y;
-          if (ep == 1) v = __fadd_rn(r, y);
-          else if (ep == 2) v = __fmul_rn(Elem<DT>::load(Elem<DT>::store(silu_rn(r))), y);
-          h2[u] = Elem<DT>::store(v);
-        }
-        ow[q] = h2[0] | (h2[1] << 16);
-      }
-      *reinterpret_cast<uint4*>(Y + o) = make_uint4(ow[0], ow[1], ow[2], ow[3]);
-    } else {
-      for (int u = 0; u < 8 && m + u < M; ++u) {
-        const float y = Elem<DT>::load(yw[u >> 1] >> (16 * (u & 1)));
-        float v = y;
-        if (ep == 1) v = __fadd_rn(Elem<DT>::load(R[o + u]), y);
-        else if (ep == 2) v = __fmul_rn(Elem<DT>::load(Elem<DT>::store(silu_rn(Elem<DT>::load(R[o + u])))), y);
-        Y[o + u] = Elem<DT>::store(v);
-      }
-    }
-  }
-}
+constexpr int KT = 64;  // codes per K-step
 
 // Y[n][m] = epilogue(round(sum over z of YP[z][n][m])), the sum in z order;
 // 8 consecutive m per thread (16-byte stores when vec).
@@ -421,41 +131,16 @@ __global__ __launch_bounds__(64 * NRM_CH) void nf4_gemm_reduce_norm_kernel(const
   if (own) *reinterpret_cast<uint4*>(YN + o) = norm8<DT>(h, gv, rr);
 }
 
-template <int DT, int BM, int BN, int WM, int WN, int PF>
-static void launch_gemm(const void* X, const uint8_t* W, const uint8_t* A8, const float* AMAX,
-                        const float* CODE2, float offset, const float* LUT, void* Y, const void* R,
-                        int epi, int M, int K, int N, int bs_shift, int bs2_shift, float* YP, int splits,
-                        hipStream_t st) {
-  const dim3 grid((M + BM - 1) / BM, (N + BN - 1) / BN, splits);
-  if (A8)
-    hipLaunchKernelGGL((nf4_gemm_kernel<DT, BM, BN, WM, WN, true, PF>), grid, dim3(64 * WM * WN), 0, st,
-                       (const uint16_t*)X, W, A8, AMAX, CODE2, offset, LUT, (uint16_t*)Y,
-                       (const uint16_t*)R, epi, M, K, N, bs_shift, bs2_shift, YP);
-  else
-    hipLaunchKernelGGL((nf4_gemm_kernel<DT, BM, BN, WM, WN, false, PF>), grid, dim3(64 * WM * WN), 0, st,
-                       (const uint16_t*)X, W, A8, AMAX, CODE2, offset, LUT, (uint16_t*)Y,
-                       (const uint16_t*)R, epi, M, K, N, bs_shift, bs2_shift, YP);
-}
-
-// Tile shape and K-split of a launch: 64 x 128 tiles (8 waves), unsplit when
-// they give every CU a workgroup. Up to 128 tiles, the largest split (2, 4,
-// 8; each split an even number of at least 8 K-steps) whose workgroups still
-// fit one to a CU: a split's fp32 partial sums cost a write and a read of
-// splits x N x M floats, so a second pass of workgroups only pays where each
-// split keeps a long K run. Between 128 and 256 tiles no split fits one pass,
-// and 4 splits pay only past 16 K-steps each. Unsplit launches take 64 x 128
-// tiles down to 128 of them, 64 x 64 below. 33 to 64 rows take 64 x 64 tiles
-// with a K split (below; callers with a choice take the few-row kernel, which
-// is faster: ttsp_nf4_gemm_few); up to 64 rows otherwise the few-row kernel or
-// the skinny kernel (nf4_gemm_few.hip, nf4_skinny.hip), shape 0, never split. Measured on the five
-// projections of a 2560-wide layer (wqkv 6144 x 2560, wo 2560 x 4096, w1 and
-// w3 9728 x 2560, w2 2560 x 9728): 187 -> 125 us at 128 rows against a rule
-// that sought two workgroups a CU, 200 -> 184 us at 256 rows, equal at 512
-// rows (where 64 x 128 beats 128 x 128 by 8-10 % at 9728 x 2560 and
-// 2560 x 9728; unsplit tile shapes give identical bits).
-struct GemmPlan {
-  int shape, splits;
-};
+// K splits of the split entry (ttsp_nf4_gemm_split and the forms that leave or
+// add its sums): none where 64 x 128 tiles give every CU a workgroup; up to
+// 128 tiles the largest split (2, 4, 8; each an even number of at least 8
+// K-steps) whose workgroups fit one to a CU: a split's fp32 partial sums cost
+// a write and a read of splits x N x M floats, so a second pass of workgroups
+// only pays where each split keeps a long K run. Between 128 and 256 tiles 4
+// splits pay only past 16 K-steps each. 256 to 512 rows: dl_plan below. 33 to
+// 64 rows: 4 ways where each split keeps 8 or more K-steps, else 2 (callers
+// with a choice take ttsp_nf4_gemm_few's plan, which is faster). Up to 64 rows
+// otherwise the few-row or the skinny kernel, never split.
 constexpr int SKINNY_MAX_N = 16;
 int skinny_max_k();
 bool few_unsplit(int M, int K, int N);
@@ -468,50 +153,34 @@ static long long gemm_tiles(int M, int N, int bm, int bn) {
   return (long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
 }
 
-static int unsplit_shape(int M, int N) { return gemm_tiles(M, N, 64, 128) >= 128 ? 2 : 3; }
-
-// 33 to 64 rows through the split entry: 64 x 64 tiles, 4 ways where each split
-// keeps 8 or more K-steps, else 2.
 constexpr int SPLIT_SMALL_N = 32;
 
-bool gemm_dl_fits(int M, int K, int N, int splits);
-int gemm_dl(const void* X, int dt, const uint8_t* W, const uint8_t* A8, const float* AMAX, const float* CODE2,
-            float offset, const float* LUT, void* Y, const void* R, int epi, int M, int K, int N, int bs_shift,
-            int bs2_shift, int waves, int splits, float* YP, hipStream_t st);
+int gemm_tile(const void* X, int dt, const uint8_t* W, const uint8_t* A8, const float* AMAX, const float* CODE2,
+              float offset, const float* LUT, void* Y, const void* R, int epi, int M, int K, int N, int bs_shift,
+              int bs2_shift, int splits, float* YP, hipStream_t st);
 
-// 256 to 512 rows: the direct-to-LDS kernel (nf4_gemm_dl.hip, shape 4, 64 x
-// 128 tiles of 2 waves) with 4 K-splits where K has 64 or more steps and
-// there are at least 75 tiles; with fewer steps unsplit from 512 tiles and
-// with 2 splits from 300. Measured against the 64 x 128 kernel at its best
-// split, 512 rows (bf16, nested scales): w1 / w3 9728 x 2560 71.5 -> 48.4 us,
-// w2 2560 x 9728 70.1 -> 48.5, wo 2560 x 4096 40.7 -> 30.1, wqkv 6144 x 2560
-// 46.6 -> 36.5; at 256 rows w1 45.8 -> 34.0, w2 48.0 -> 39.8. The 64 x 128
-// kernel stays ahead or ties at 128 rows, at 4096 x 2560 and on the
-// 1024-wide shapes.
+// 256 to 512 rows: 4 K-splits where K has 64 or more steps and there are at
+// least 75 64 x 128 tiles; with fewer steps none from 512 tiles and 2 from 300.
+// 0: no rule here.
 constexpr int DL_MIN_N = 256, DL_MAX_N = 512;
-static bool dl_plan(int M, int K, int N, GemmPlan* p) {
-  if (N < DL_MIN_N || N > DL_MAX_N) return false;
+static int dl_plan(int M, int K, int N) {
+  if (N < DL_MIN_N || N > DL_MAX_N) return 0;
   const int steps = K / KT;
   const long long t = gemm_tiles(M, N, 64, 128);
-  if (steps >= 64) {
-    if (t >= 75 && steps % 8 == 0 && gemm_dl_fits(M, K, N, 4)) return *p = GemmPlan{4, 4}, true;
-    return false;
-  }
-  if (t >= 512 && gemm_dl_fits(M, K, N, 1)) return *p = GemmPlan{4, 1}, true;
-  if (t >= 300 && steps % 4 == 0 && gemm_dl_fits(M, K, N, 2)) return *p = GemmPlan{4, 2}, true;
-  return false;
+  if (steps >= 64) return t >= 75 && steps % 8 == 0 && steps / 4 <= 64 ? 4 : 0;
+  if (t >= 512) return 1;
+  return t >= 300 && steps % 4 == 0 ? 2 : 0;
 }
 
-static GemmPlan gemm_plan(int M, int K, int N) {
+static int gemm_plan(int M, int K, int N) {
   const int steps = K / KT;
   if (N > SPLIT_SMALL_N && N <= 64)
     for (int sp = 4; sp >= 2; sp /= 2)
-      if (steps % (2 * sp) == 0 && steps / sp >= 8) return {3, sp};
-  if (skinny(K, N) || few_unsplit(M, K, N)) return {0, 1};
-  GemmPlan dl;
-  if (dl_plan(M, K, N, &dl)) return dl;
+      if (steps % (2 * sp) == 0 && steps / sp >= 8) return sp;
+  if (skinny(K, N) || few_unsplit(M, K, N)) return 1;
+  if (const int dl = dl_plan(M, K, N)) return dl;
   const long long t = gemm_tiles(M, N, 64, 128);
-  if (t >= 256) return {2, 1};
+  if (t >= 256) return 1;
   int splits = 1;
   if (t > 128) {
     if (steps % 8 == 0 && steps / 4 > 16) splits = 4;
@@ -521,8 +190,13 @@ static GemmPlan gemm_plan(int M, int K, int N) {
       splits = sp;
     }
   }
-  return splits > 1 ? GemmPlan{2, splits} : GemmPlan{unsplit_shape(M, N), 1};
+  return splits;
 }
+
+int gemm_few(const void* X, int dt, const uint8_t* W, const uint8_t* A8, const float* AMAX, const float* CODE2,
+             float offset, const float* LUT, void* Y, const void* R, int epi, int M, int K, int N, int bs_shift,
+             int bs2_shift, int splits, float* YP, hipStream_t st);
+bool few_takes(int M, int K, int N);
 
 // Y = epilogue(round(sum of the splits' partials)) (epi bit 2: vectorised)
 int gemm_reduce(int dt, const float* YP, int splits, void* Y, const void* R, int epi, int M, int N, hipStream_t st) {
@@ -559,44 +233,22 @@ static int gemm_reduce_norm(int x_dtype, const float* work, int splits, void* Y,
   TTSP_RETURN_LAUNCH();
 }
 
-int gemm_mfma(const void* X, int dt, const uint8_t* W, const uint8_t* A8, const float* AMAX,
-              const float* CODE2, float offset, const float* LUT, void* Y, const void* R, int epi,
-              int M, int K, int N, int bs_shift, int bs2_shift, const GemmPlan& plan, float* YP,
-              hipStream_t st, bool reduce = true) {
+// A product in `splits` K splits: the few-row kernel where it takes the rows,
+// else the tiles. splits > 1 leaves the sums in YP, and with reduce adds them
+// (epi bit 2: vectorised output).
+int gemm_mfma(const void* X, int dt, const uint8_t* W, const uint8_t* A8, const float* AMAX, const float* CODE2,
+              float offset, const float* LUT, void* Y, const void* R, int epi, int M, int K, int N, int bs_shift,
+              int bs2_shift, int splits, float* YP, hipStream_t st, bool reduce = true) {
   if (K % (2 * KT)) return (int)hipErrorInvalidValue;
-  const int splits = plan.splits;
   if (splits > 1 && (!YP || (K / KT) % (2 * splits))) return (int)hipErrorInvalidValue;
-  float* yp = splits > 1 ? YP : nullptr;
-  const bool pf4 = (K / KT / splits) % 4 == 0;
-#define TTSP_G(DTV, BMV, BNV, WMV, WNV)                                                                     \
-  (pf4 ? launch_gemm<DTV, BMV, BNV, WMV, WNV, 4>(X, W, A8, AMAX, CODE2, offset, LUT, Y, R, epi, M, K, N,    \
-                                                 bs_shift, bs2_shift, yp, splits, st)                       \
-       : launch_gemm<DTV, BMV, BNV, WMV, WNV, 2>(X, W, A8, AMAX, CODE2, offset, LUT, Y, R, epi, M, K, N,    \
-                                                 bs_shift, bs2_shift, yp, splits, st))
-  // 8 waves for the 64 x 128 tiles (two a SIMD: one wave's dequantisation
-  // runs while the other's matrix products do), 4 for 64 x 64
-  // The direct-to-LDS kernel resolves nested scales with at most one
-  // second-level group boundary inside a workgroup's K range (true for
-  // bitsandbytes' blocksize2 of 256); smaller groups take the 64 x 128
-  // kernel with the same split.
-  int shape = plan.shape;
-  if (shape == 4 && A8 && (long long)(K / splits) > (1LL << (bs_shift + bs2_shift))) shape = 2;
-  if (shape == 4) {
-    if (int rc = gemm_dl(X, dt, W, A8, AMAX, CODE2, offset, LUT, Y, R, epi, M, K, N, bs_shift, bs2_shift, 2,
-                         splits, yp, st))
-      return rc;
-  } else if (dt == DT_BF16) {
-    if (shape == 2) TTSP_G(DT_BF16, 64, 128, 2, 4);
-    else TTSP_G(DT_BF16, 64, 64, 2, 2);
-  } else if (dt == DT_F16) {
-    if (shape == 2) TTSP_G(DT_F16, 64, 128, 2, 4);
-    else TTSP_G(DT_F16, 64, 64, 2, 2);
-  } else {
-    return (int)hipErrorInvalidValue;
-  }
-#undef TTSP_G
+  const bool few = few_takes(M, K, N) && (uintptr_t)X % 16 == 0 && (uintptr_t)W % 16 == 0;
+  if (int rc = few ? gemm_few(X, dt, W, A8, AMAX, CODE2, offset, LUT, Y, R, epi, M, K, N, bs_shift, bs2_shift, splits,
+                              YP, st)
+                   : gemm_tile(X, dt, W, A8, AMAX, CODE2, offset, LUT, Y, R, epi, M, K, N, bs_shift, bs2_shift, splits,
+                               YP, st))
+    return rc;
   if (splits > 1 && reduce) return gemm_reduce(dt, YP, splits, Y, R, epi, M, N, st);
-  TTSP_RETURN_LAUNCH();
+  return 0;
 }
 
 bool gemv_fits(int M, int K, int blocksize, int N);
@@ -610,18 +262,15 @@ constexpr int GEMV_ROWS_N = 2;
 int gemm_skinny(const void* X, int dt, const uint8_t* W, const uint8_t* A8, const float* AMAX, const float* CODE2,
                 float offset, const float* LUT, void* Y, const void* RES, int epi, int M, int K, int N, int bs_shift,
                 int bs2_shift, hipStream_t st);
-int gemm_dl_swiglu(const void* X, int dt, const uint8_t* W1, const uint8_t* A8_1, const float* AMAX_1,
-                   const float* CODE2_1, float offset_1, const uint8_t* W3, const uint8_t* A8_3,
-                   const float* AMAX_3, const float* CODE2_3, float offset_3, const float* LUT, void* Y, int M, int K,
-                   int N, int bs_shift, int bs2_shift, hipStream_t st);
+int gemm_tile_swiglu(const void* X, int dt, const uint8_t* W1, const uint8_t* A8_1, const float* AMAX_1,
+                     const float* CODE2_1, float offset_1, const uint8_t* W3, const uint8_t* A8_3, const float* AMAX_3,
+                     const float* CODE2_3, float offset_3, const float* LUT, void* Y, int M, int K, int N, int bs_shift,
+                     int bs2_shift, hipStream_t st);
 int gemm_skinny_pair(const void* X, int dt, const uint8_t* W1, const uint8_t* A8_1, const float* AMAX_1,
                      const float* CODE2_1, float offset_1, const uint8_t* W3, const uint8_t* A8_3, const float* AMAX_3,
                      const float* CODE2_3, float offset_3, const float* LUT, void* Y, int M, int K, int N, int bs_shift,
                      int bs2_shift, hipStream_t st);
 bool skinny_pair_fits(int K, int N);
-int gemm_few(const void* X, int dt, const uint8_t* W, const uint8_t* A8, const float* AMAX, const float* CODE2,
-             float offset, const float* LUT, void* Y, const void* R, int epi, int M, int K, int N, int bs_shift,
-             int bs2_shift, int splits, float* YP, hipStream_t st);
 int gemm_few_pair(const void* X, int dt, const uint8_t* W1, const uint8_t* A8_1, const float* AMAX_1,
                   const float* CODE2_1, float offset_1, const uint8_t* W3, const uint8_t* A8_3, const float* AMAX_3,
                   const float* CODE2_3, float offset_3, const float* LUT, void* Y, int M, int K, int N, int bs_shift,
@@ -635,14 +284,12 @@ static bool swiglu_skinny(int M, int K, int N) {
   return few_unsplit(M, K, N) ? few_pair(M, K, N) : skinny_pair_fits(K, N);
 }
 
-// Whether the SwiGLU pair fits one launch of the direct-to-LDS kernel: where
-// each of its two GEMMs would run that kernel unsplit (so the one launch
-// gives their bits).
+// Whether the SwiGLU pair fits one launch of the tile kernel: where each of
+// its two GEMMs runs that kernel unsplit and over whole K (more than 256 64 x
+// 128 tiles), so that the one launch gives their bits. (Second-level groups
+// shorter than K keep two launches, as before the scales were resolved per step.)
 static bool swiglu_fits(int M, int K, int N, int bs_shift, int bs2_shift, bool nested) {
-  if (M <= 0 || K <= 0 || K % 128 || N <= 64) return false;
-  GemmPlan dl;
-  if (!dl_plan(M, K, N, &dl) || dl.splits != 1 || dl.shape != 4) return false;
-  // the plan's fallback to 64 x 128 tiles for small second-level groups
+  if (M <= 0 || K <= 0 || K % 128 || N <= 64 || dl_plan(M, K, N) != 1) return false;
   return !(nested && (long long)K > (1LL << (bs_shift + bs2_shift)));
 }
 
@@ -688,19 +335,23 @@ extern "C" int ttsp_nf4_gemm(const void* X, int x_dtype, const uint8_t* W, const
                     stream);
   if (N >= 2 && skinny(K, N))
     return gemm_skinny(X, x_dtype, W, A8, AMAX, CODE2, offset, LUT, Y, R, epi, M, K, N, bs_shift, bs2_shift, stream);
-  // vectorised output rows: 8 elements per 16-byte store
-  const bool vec = M % 8 == 0 && (uintptr_t)Y % 16 == 0 && (!epi || (uintptr_t)R % 16 == 0);
-  // unsplit: the direct-to-LDS kernel where the plan takes it unsplit, else
-  // 64 x 128 tiles, or 64 x 64 when fewer than 128 of those
-  GemmPlan plan{unsplit_shape(M, N), 1}, dl;
-  if (dl_plan(M, K, N, &dl) && dl.splits == 1) plan = dl;
-  return gemm_mfma(X, x_dtype, W, A8, AMAX, CODE2, offset, LUT, Y, R, epi | (vec ? 4 : 0), M, K, N, bs_shift,
-                   bs2_shift, plan, nullptr, stream);
+  return gemm_mfma(X, x_dtype, W, A8, AMAX, CODE2, offset, LUT, Y, R, epi, M, K, N, bs_shift, bs2_shift, 1, nullptr,
+                   stream);
 }
 
 extern "C" int ttsp_nf4_gemm_splits(int M, int K, int N) {
   if (M <= 0 || K <= 0 || N <= 1 || K % 128) return 1;
-  return gemm_plan(M, K, N).splits;
+  return gemm_plan(M, K, N);
+}
+
+// The splits a caller with a workspace should take at 65 to 512 rows:
+// ttsp_nf4_gemm_splits', but unsplit instead of 2 ways at 256 rows and more
+// where no norm follows in the reduce (M past its widest row): 9728 x 2560 at
+// 256 rows 28.0 us against 32 and a 10 us reduce, 6144 x 2560 at 512 28.7
+// against 30.3 and 7. (Sums that another kernel adds keep the two splits.)
+extern "C" int ttsp_nf4_gemm_tile_splits(int M, int K, int N) {
+  if (M <= 0 || K <= 0 || N <= 1 || K % 128) return 1;
+  return M > 64 * 8 * NRM_CH && dl_plan(M, K, N) == 2 ? 1 : gemm_plan(M, K, N);
 }
 
 extern "C" int ttsp_nf4_gemm_split(const void* X, int x_dtype, const uint8_t* W, const uint8_t* A8,
@@ -753,7 +404,7 @@ extern "C" int ttsp_nf4_gemm_swiglu(const void* X, int x_dtype, const uint8_t* W
     return gemm_skinny_pair(X, x_dtype, W1, A8_1, AMAX_1, CODE2_1, offset_1, W3, A8_3, AMAX_3, CODE2_3, offset_3, LUT,
                             Y, M, K, N, bs_shift, bs2_shift, stream);
   if (!swiglu_fits(M, K, N, bs_shift, bs2_shift, A8_1 != nullptr)) return (int)hipErrorInvalidValue;
-  return gemm_dl_swiglu(X, x_dtype, W1, A8_1, AMAX_1, CODE2_1, offset_1, W3, A8_3, AMAX_3, CODE2_3, offset_3, LUT, Y,
+  return gemm_tile_swiglu(X, x_dtype, W1, A8_1, AMAX_1, CODE2_1, offset_1, W3, A8_3, AMAX_3, CODE2_3, offset_3, LUT, Y,
                         M, K, N, bs_shift, bs2_shift, stream);
 }
 

@@ -28,43 +28,11 @@
 // within 5 % at 2048 rows and up to 20 % behind at 700; 256 x 256 leaves too
 // few tiles. Sums run along K in the same order in every tile shape, so the
 // shape does not change a bit of the result.
-#include "ttsp_common.h"
+#include "nf4_mfma.h"
 
 namespace ttsp {
 
 namespace {
-
-typedef __bf16 bf16x8_v __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8_v __attribute__((ext_vector_type(8)));
-typedef float f32x16_v __attribute__((ext_vector_type(16)));
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
-
-// s_waitcnt: vmcnt n, lgkmcnt 0 (gfx9 encoding; expcnt unbounded)
-#define TTSP_WAIT_VM_LGKM0(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | (7 << 4))
-
-template <int DT>
-__device__ __forceinline__ f32x16_v mfma32(u32x4 a, u32x4 b, f32x16_v c) {
-  if constexpr (DT == DT_BF16)
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_v, a), __builtin_bit_cast(bf16x8_v, b),
-                                                   c, 0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_v, a), __builtin_bit_cast(f16x8_v, b), c,
-                                                  0, 0, 0);
-}
-
-typedef __bf16 bf16x2_v __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x2_v __attribute__((ext_vector_type(2)));
-typedef float f32x2_v __attribute__((ext_vector_type(2)));
-
-// two fp32 values to the activation type (nearest even), one hardware pack-convert
-template <int DT>
-__device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-  const f32x2_v v = {opaque(lo), opaque(hi)};
-  if constexpr (DT == DT_BF16)
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_v));
-  else
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2_v));
-}
 
 // A workgroup's tile: BM weight rows x BN activation rows, WM x WN waves, a
 // ring of ST stages of KT elements of K.
@@ -148,14 +116,6 @@ __device__ __forceinline__ void step(const X& c, const uint8_t* __restrict__ rd,
     mul_slice<DT, C>(af[kk & 1], bf[kk & 1], acc);
     __builtin_amdgcn_sched_barrier(0);
   }
-}
-
-template <int DT>
-__device__ __forceinline__ uint16_t dense_epi(float y, uint16_t r, int ep) {
-  float v = y;
-  if (ep == 1) v = __fadd_rn(Elem<DT>::load(r), y);
-  else if (ep == 2) v = __fmul_rn(Elem<DT>::load(Elem<DT>::store(silu_rn(Elem<DT>::load(r)))), y);
-  return Elem<DT>::store(v);
 }
 
 template <int DT, typename C, bool SW>
@@ -302,45 +262,15 @@ __global__ __launch_bounds__(64 * C::NW) void nf4_gemm_dense_kernel(
       if (n >= N || m >= M) continue;
       const size_t o = (size_t)n * M + m;
       const bool full = vec && m + 8 <= M;
-      u32x4 yv, rv = {0, 0, 0, 0};
+      u32x4 y, r = {0, 0, 0, 0};
       if constexpr (SW) {
         const uint8_t* src = stg + nl * PITCH + (ch >> 2) * 128 + (ch & 3) * 16;
-        rv = *reinterpret_cast<const u32x4*>(src);
-        yv = *reinterpret_cast<const u32x4*>(src + 64);
+        r = *reinterpret_cast<const u32x4*>(src);
+        y = *reinterpret_cast<const u32x4*>(src + 64);
       } else {
-        yv = *reinterpret_cast<const u32x4*>(stg + nl * PITCH + ch * 16);
-        if (ep) {
-          if (full) {
-            rv = *reinterpret_cast<const u32x4*>(R + o);
-          } else {
-            for (int u = 0; u < 8; ++u)
-              if (m + u < M) {
-                const uint32_t h = (uint32_t)R[o + u] << (16 * (u & 1));
-                if (u < 2) rv.x |= h; else if (u < 4) rv.y |= h; else if (u < 6) rv.z |= h; else rv.w |= h;
-              }
-          }
-        }
+        y = *reinterpret_cast<const u32x4*>(stg + nl * PITCH + ch * 16);
       }
-      if (ep) {
-#pragma unroll 1
-        for (int q = 0; q < 4; ++q) {
-          // one dword of each a turn, the vectors rotated so that the loop indexes nothing at run time
-          const uint32_t y = yv.x, r = rv.x;
-          const uint32_t w = (uint32_t)dense_epi<DT>(Elem<DT>::load(y), (uint16_t)r, ep) |
-                             ((uint32_t)dense_epi<DT>(Elem<DT>::load(y >> 16), (uint16_t)(r >> 16), ep) << 16);
-          yv = u32x4{yv.y, yv.z, yv.w, w};
-          rv = u32x4{rv.y, rv.z, rv.w, r};
-        }
-      }
-      if (full) {
-        *reinterpret_cast<u32x4*>(Y + o) = yv;
-      } else {
-        for (int u = 0; u < 8; ++u)
-          if (m + u < M) {
-            const uint32_t w = u < 2 ? yv.x : u < 4 ? yv.y : u < 6 ? yv.z : yv.w;
-            Y[o + u] = (uint16_t)(w >> (16 * (u & 1)));
-          }
-      }
+      mm_store8<DT>(Y, R, o, m, M, full, ep, y, SW, r);
     }
   }
 #endif
@@ -482,7 +412,7 @@ static bool dense_fits(int M, int K, int N, int mats) {
 using namespace ttsp;
 
 // The K splits `ttsp_nf4_gemm_dense` takes a product in, 0 where it does not
-// serve it. Served from DENSE_MIN_N rows (one row more than the direct-to-LDS
+// serve it. Served from DENSE_MIN_N rows (one row more than the tile
 // kernel's plans; calls at 513 rows, fused kernels against this: 9728 x 2560
 // 69 -> 49 us, 2560 x 9728 90 -> 57, 2560 x 4096 43 -> 37, and 220 -> 119,
 // 225 -> 119, 101 -> 55 at 2048) for weights and products large enough to

@@ -31,42 +31,11 @@
 // 15.5 -> 8.7, 24.9 -> 9.9, 24.9 -> 13.0 and 2560 x 4096 7.7 -> 5.3, 12.2 ->
 // 5.9, 14.8 -> 7.8. Eight waves a workgroup instead of more workgroups were
 // slower (9728 x 2560 at 16 rows 12.9 us: one workgroup a CU, two rounds).
-#include "ttsp_common.h"
+#include "nf4_mfma.h"
 
 namespace ttsp {
 
 namespace {
-
-typedef __bf16 bf16x8_v __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8_v __attribute__((ext_vector_type(8)));
-typedef float f32x16_v __attribute__((ext_vector_type(16)));
-typedef __bf16 bf16x2_v __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x2_v __attribute__((ext_vector_type(2)));
-typedef float f32x2_v __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
-
-// s_waitcnt: vmcnt n, lgkmcnt 0 (gfx9 encoding; expcnt unbounded)
-#define TTSP_WAIT_VM_LGKM0(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | (7 << 4))
-#define TTSP_WAIT_LGKM0() __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4))
-
-template <int DT>
-__device__ __forceinline__ f32x16_v mfma32(u32x4 a, u32x4 b, f32x16_v c) {
-  if constexpr (DT == DT_BF16)
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_v, a), __builtin_bit_cast(bf16x8_v, b),
-                                                   c, 0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_v, a), __builtin_bit_cast(f16x8_v, b), c,
-                                                  0, 0, 0);
-}
-
-template <int DT>
-__device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-  const f32x2_v v = {opaque(lo), opaque(hi)};
-  if constexpr (DT == DT_BF16)
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_v));
-  else
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2_v));
-}
 
 constexpr int KT = 64;   // codes per K-step
 constexpr int CH = 1024; // bytes of one wave-wide load
@@ -153,14 +122,6 @@ __device__ __forceinline__ void few_step(const uint8_t* __restrict__ rd, uint8_t
     for (int b = 0; b < C::TN; ++b) acc[t][b] = mfma32<DT>(af, bf[kk][b], acc[t][b]);
     __builtin_amdgcn_sched_barrier(0);
   }
-}
-
-template <int DT>
-__device__ __forceinline__ uint16_t few_epi(float y, uint16_t r, int ep) {
-  float v = y;
-  if (ep == 1) v = __fadd_rn(Elem<DT>::load(r), y);
-  else if (ep == 2) v = __fmul_rn(Elem<DT>::load(Elem<DT>::store(silu_rn(Elem<DT>::load(r)))), y);
-  return Elem<DT>::store(v);
 }
 
 template <int DT, int XL, int MATS, bool NESTED>
@@ -339,9 +300,9 @@ __global__ __launch_bounds__(64 * KS, 2) void nf4_gemm_few_kernel(
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       if constexpr (MATS == 2)
-        ov[c] = few_epi<DT>(Elem<DT>::load(Elem<DT>::store(v[b][1][c])), Elem<DT>::store(v[b][0][c]), 2);
+        ov[c] = mm_epi<DT>(Elem<DT>::load(Elem<DT>::store(v[b][1][c])), Elem<DT>::store(v[b][0][c]), 2);
       else
-        ov[c] = few_epi<DT>(Elem<DT>::load(Elem<DT>::store(v[b][0][c])), ep && m + c < M ? R[o + c] : (uint16_t)0, ep);
+        ov[c] = mm_epi<DT>(Elem<DT>::load(Elem<DT>::store(v[b][0][c])), ep && m + c < M ? R[o + c] : (uint16_t)0, ep);
     }
     if (v4) {
       *reinterpret_cast<uint2*>(Y + o) =
@@ -388,7 +349,7 @@ constexpr int FEW_MIN_N = 9, FEW_MAX_N = 64, FEW_PAIR_MAX_N = 32;
 
 // Whether the kernel takes the shape: byte offsets of X and W and the scale
 // indices below 2^31.
-static bool few_takes(int M, int K, int N) {
+bool few_takes(int M, int K, int N) {
   if (M <= 0 || K <= 0 || K % 128 || N < FEW_MIN_N || N > FEW_MAX_N) return false;
   return (long long)N * K * 2 < (1ll << 31) && (long long)M * K / 2 < (1ll << 31);
 }

@@ -1,0 +1,105 @@
+// Device helpers shared by the NF4 matrix-core kernels (nf4_gemm_few.hip,
+// nf4_gemm_tile.hip, nf4_gemm_dense.hip): the 32x32x16 product, the 16-bit
+// roundings, the epilogue of one value, and the waits around LDS loads.
+#pragma once
+#include "ttsp_common.h"
+
+namespace ttsp {
+
+typedef __bf16 bf16x8_v __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8_v __attribute__((ext_vector_type(8)));
+typedef float f32x16_v __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x2_v __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x2_v __attribute__((ext_vector_type(2)));
+typedef float f32x2_v __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) void* lds_ptr_t;
+
+// s_waitcnt: vmcnt n, lgkmcnt 0 (gfx9 encoding; expcnt unbounded)
+#define TTSP_WAIT_VM_LGKM0(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | (7 << 4))
+// lgkmcnt 0 alone
+#define TTSP_WAIT_LGKM0() __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4))
+
+// Lane l supplies row l % 32 of A and column l % 32 of B, each as 8 consecutive
+// k at 8 (l / 32); accumulator r of lane l is D[8 (r / 4) + 4 (l / 32) + r % 4]
+// [l % 32]. A and B need only agree on which k a lane carries.
+template <int DT>
+__device__ __forceinline__ f32x16_v mfma32(u32x4 a, u32x4 b, f32x16_v c) {
+  if constexpr (DT == DT_BF16)
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_v, a), __builtin_bit_cast(bf16x8_v, b),
+                                                   c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_v, a), __builtin_bit_cast(f16x8_v, b), c,
+                                                  0, 0, 0);
+}
+
+// Two fp32 values, each already rounded to fp32, to the activation type
+// (nearest even), one hardware pack-convert; lo in the low half.
+template <int DT>
+__device__ __forceinline__ uint32_t pack2(float lo, float hi) {
+  const f32x2_v v = {opaque(lo), opaque(hi)};
+  if constexpr (DT == DT_BF16)
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_v));
+  else
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2_v));
+}
+
+// The epilogue of one value (y already rounded): ep 1 adds r, ep 2 multiplies
+// by round(silu(r)); the result rounded.
+template <int DT>
+__device__ __forceinline__ uint16_t mm_epi(float y, uint16_t r, int ep) {
+  float v = y;
+  if (ep == 1) v = __fadd_rn(Elem<DT>::load(r), y);
+  else if (ep == 2) v = __fmul_rn(Elem<DT>::load(Elem<DT>::store(silu_rn(Elem<DT>::load(r)))), y);
+  return Elem<DT>::store(v);
+}
+
+// Eight values of an output row (packed, rounded) through the epilogue with
+// their operands, a dword of each a turn: the vectors rotate, so a rolled loop
+// indexes nothing at run time and its code stays small.
+template <int DT>
+__device__ __forceinline__ u32x4 mm_epi8(u32x4 y, u32x4 r, int ep) {
+#pragma unroll 1
+  for (int q = 0; q < 4; ++q) {
+    const uint32_t a = y.x, b = r.x;
+    const uint32_t w = (uint32_t)mm_epi<DT>(Elem<DT>::load(a), (uint16_t)b, ep) |
+                       ((uint32_t)mm_epi<DT>(Elem<DT>::load(a >> 16), (uint16_t)(b >> 16), ep) << 16);
+    y = u32x4{y.y, y.z, y.w, w};
+    r = u32x4{r.y, r.z, r.w, b};
+  }
+  return y;
+}
+
+// Eight values at Y + o (m .. m + 7 of a row of M, full: aligned and all below
+// M) with the epilogue: the operand from R where ep needs one, or given (own).
+template <int DT>
+__device__ __forceinline__ void mm_store8(uint16_t* __restrict__ Y, const uint16_t* __restrict__ R, size_t o, int m,
+                                          int M, bool full, int ep, u32x4 y, bool own, u32x4 r) {
+  if (ep) {
+    if (!own) {
+      if (full) {
+        r = *reinterpret_cast<const u32x4*>(R + o);
+      } else {
+        for (int u = 0; u < 8; ++u)
+          if (m + u < M) {
+            const uint32_t h = (uint32_t)R[o + u] << (16 * (u & 1));
+            if (u < 2) r.x |= h;
+            else if (u < 4) r.y |= h;
+            else if (u < 6) r.z |= h;
+            else r.w |= h;
+          }
+      }
+    }
+    y = mm_epi8<DT>(y, r, ep);
+  }
+  if (full) {
+    *reinterpret_cast<u32x4*>(Y + o) = y;
+  } else {
+    for (int u = 0; u < 8; ++u)
+      if (m + u < M) {
+        const uint32_t w = u < 2 ? y.x : u < 4 ? y.y : u < 6 ? y.z : y.w;
+        Y[o + u] = (uint16_t)(w >> (16 * (u & 1)));
+      }
+  }
+}
+
+}  // namespace ttsp

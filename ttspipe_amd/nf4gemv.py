@@ -12,9 +12,8 @@ bitsandbytes put them; `libttsp_hip.so` reads them directly:
   fixed order (so results are reproducible bit for bit);
 * two or more rows go to the matrix cores, one dequantisation serving a tile
   of rows: the few-row kernels up to 64 (`csrc/nf4_skinny.hip`,
-  `csrc/nf4_gemm_few.hip`), the tiled ones above (`csrc/nf4_gemm.hip`,
-  `csrc/nf4_gemm_dl.hip`), and past 512 rows one dequantisation a call
-  (`csrc/nf4_gemm_dense.hip`).
+  `csrc/nf4_gemm_few.hip`), tiles above (`csrc/nf4_gemm_tile.hip`), and past
+  512 rows one dequantisation a call (`csrc/nf4_gemm_dense.hip`).
 
 Unlike the reference (fp16 only, nf4gemv.py:439) both fp16 and bf16
 activations are served; anything else is declined (`None`), exactly where the
@@ -206,7 +205,7 @@ def matmul(module, x, *, epi: int = EPI_NONE, operand=None, out=None):
     lib = _lib.lib()
     dense = lib.ttsp_nf4_gemm_dense_splits(M, K, rows) if rows >= DENSE_MIN_ROWS else 0
     few = lib.ttsp_nf4_gemm_few_splits(M, K, rows) if FEW_SPLIT_ROWS <= rows <= FEW_MAX_ROWS else 0
-    splits = lib.ttsp_nf4_gemm_splits(M, K, rows) if rows > 1 and not dense and not few else 1
+    splits = lib.ttsp_nf4_gemm_tile_splits(M, K, rows) if rows > 1 and not dense and not few else 1
     if few:
         work = torch.empty(few * rows * M, dtype=torch.float32, device=x.device) if few > 1 else None
         rc = _few(lib, fast, flat, dt, rows, out, operand, epi, work)
@@ -444,7 +443,7 @@ def matmul_swiglu(module1, module3, x, *, out=None):
     """silu(x W1^T) * (x W3^T) for several rows in one launch, rounded as the
     two-launch form `matmul(w3, x, epi=EPI_SILU_GATE, operand=matmul(w1, x))`
     and with its bits; None where one launch does not serve the shape (it
-    serves where both GEMMs would run the direct-to-LDS kernel unsplit, e.g.
+    serves where both GEMMs would run the tile kernel unsplit over whole K, e.g.
     385 to 512 rows of 9728 x 2560, and where both would run the few-row
     kernel, 3 to 32 rows, whose pair form reads each row tile of w1 and w3
     in one workgroup)."""
