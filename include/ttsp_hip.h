@@ -82,8 +82,9 @@ int ttsp_nf4_gemm(const void* X, int x_dtype, const uint8_t* W, const uint8_t* A
  * slicing of the rows into MAX_N = 32 launches (app/engine/nf4gemv.py:460-477),
  * which it does instead of splitting K. */
 int ttsp_nf4_gemm_splits(int M, int K, int N);
-/* The splits that are fastest where the caller may choose: either
- * ttsp_nf4_gemm_splits' or 1 (then ttsp_nf4_gemm). */
+/* The splits that are fastest where the caller may choose:
+ * ttsp_nf4_gemm_splits' or fewer. ttsp_nf4_gemm_split and
+ * ttsp_nf4_gemm_split_norm take either. */
 int ttsp_nf4_gemm_tile_splits(int M, int K, int N);
 
 /* ttsp_nf4_gemm with the K loop split `splits` ways (exactly

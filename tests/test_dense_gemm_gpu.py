@@ -28,29 +28,31 @@ def _plan(M, K, rows):
 
 def test_dense_plan_covers_long_prompts_only():
     """Not up to 512 rows, not small products, not byte offsets of 2^31; else
-    1, 2 or 4 splits of at least 8 whole K-steps."""
+    unsplit or the 512-row plan's splits."""
+    from ttspipe_amd import _lib
+
     assert _plan(9728, 2560, 512) == 0 and _plan(1024, 1024, 1024) == 0 and _plan(4096, 2560, 1 << 20) == 0
     assert _plan(1 << 17, 1 << 14, 1024) == 0
     for M, K in ((9728, 2560), (2560, 9728), (2560, 4096), (6144, 2560), (9730, 2560), (4096, 1024), (128, 32768)):
-        for rows in (513, 700, 1024, 1500, 2048, 5000):
+        for rows in (513, 700, 800, 1024, 1500, 2048, 5000):
             sp = _plan(M, K, rows)
-            assert sp in (0, 1, 2, 4)
-            if sp > 1:
-                assert K // 64 % sp == 0 and K // 64 // sp >= 8 and M % 4 == 0
+            assert sp in (0, 1, _lib.load().ttsp_nf4_gemm_splits(M, K, 512))
+            assert sp or rows < 1024 or M * K < 1 << 21 or M * K * rows < 2.5e9
+            assert sp < 2 or M % 4 == 0
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("shape,rows,splits,nested,dtype,epi", [
-    ((9728, 2560), 513, 1, True, torch.bfloat16, 0),     # one activation row in the last tile
-    ((9730, 2560), 640, 1, False, torch.float16, 0),     # M % 4 == 2: element-wise stores
-    ((9730, 2560), 640, 1, True, torch.bfloat16, 1),     # and element-wise residual reads
-    ((6144, 2560), 2048, 1, True, torch.bfloat16, 0),    # 192 x 256 tiles
+    ((9728, 2560), 1025, 1, True, torch.bfloat16, 0),    # one activation row in the last tile
+    ((9730, 2560), 900, 1, False, torch.float16, 0),     # M % 4 == 2: element-wise stores
+    ((9730, 2560), 900, 1, True, torch.bfloat16, 1),     # and element-wise residual reads
+    ((6144, 2560), 2048, 1, True, torch.bfloat16, 0),    # 192 x 256 tiles, two runs of K
     ((6150, 2560), 2047, 1, False, torch.float16, 2),    # the same, ragged both ways
-    ((2560, 9728), 700, 4, True, torch.bfloat16, 1),     # K splits, the reduce's epilogue
-    ((2564, 4096), 1030, 2, False, torch.float16, 2),    # M % 8 == 4 under a split
-    ((1540, 2688), 1300, 2, True, torch.float16, 0),     # 21 K-steps a split: a ring remainder
-    ((4096, 1024), 1500, 1, True, torch.bfloat16, 0),    # 16 K-steps
-    ((40, 65536), 1024, 4, True, torch.bfloat16, 0),     # fewer rows than a tile, a long K
+    ((2560, 9728), 1000, 4, True, torch.bfloat16, 1),    # K splits, the reduce's epilogue
+    ((2564, 8192), 1030, 4, False, torch.float16, 2),    # M % 8 == 4 under a split
+    ((2564, 8192), 1600, 1, True, torch.float16, 1),     # four runs of K in a workgroup
+    ((1540, 9600), 1300, 1, True, torch.float16, 0),     # 150 K-steps
+    ((4096, 1024), 4000, 1, True, torch.bfloat16, 0),    # 16 K-steps
 ])
 def test_dense_gemm_against_fp64(nf4, orc, shape, rows, splits, nested, dtype, epi):
     """Rows past N and weight rows past M repeat the last ones and must not be
@@ -80,9 +82,9 @@ def test_dense_gemm_against_fp64(nf4, orc, shape, rows, splits, nested, dtype, e
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,K,rows,nested,dtype", [(9728, 2560, 700, True, torch.bfloat16),
-                                                   (5000, 1024, 1100, False, torch.float16),
-                                                   (2562, 2688, 1300, True, torch.bfloat16)])
+@pytest.mark.parametrize("M,K,rows,nested,dtype", [(9728, 2560, 1300, True, torch.bfloat16),
+                                                   (4096, 1024, 4000, False, torch.float16),
+                                                   (2562, 2688, 2100, True, torch.bfloat16)])
 def test_dense_swiglu_pair_equals_its_two_launches(nf4, M, K, rows, nested, dtype):
     from ttspipe_amd import _lib
 
@@ -90,9 +92,7 @@ def test_dense_swiglu_pair_equals_its_two_launches(nf4, M, K, rows, nested, dtyp
     w3 = to_linear(random_layer(M, K, nested, seed=2), dtype)
     assert nf4.prepare(w1) and nf4.prepare(w3)
     x = from_bits(randn_bits(rows * K, dtype, seed=3), dtype).view(rows, K)
-    if _lib.load().ttsp_nf4_gemm_dense_swiglu_fits(M, K, rows) == 0:
-        assert _plan(M, K, rows) > 1 and nf4.matmul_swiglu(w1, w3, x) is None
-        return
+    assert _lib.load().ttsp_nf4_gemm_dense_swiglu_fits(M, K, rows) == 1
     two = nf4.matmul(w3, x, epi=nf4.EPI_SILU_GATE, operand=nf4.matmul(w1, x))
     one = nf4.matmul_swiglu(w1, w3, x)
     assert one is not None and torch.equal(one.view(torch.int16), two.view(torch.int16))

@@ -65,7 +65,7 @@ def test_few_rows_against_fp64(nf4, orc, shape, rows, nested, bs, bs2, dtype):
     nf4.matmul(lin, x, out=guard[:rows])
     assert bool((guard[rows] == 7.0).all())
     assert beyond_rounding_error(o.to_f32(bits(guard[:rows]), dt).reshape(rows, M), ref, dt) < 2e-3
-    part = nf4.matmul_partials(lin, x, few_rows=True)
+    part = nf4.matmul_partials(lin, x, span=True)
     assert (part is None) == (_splits(M, K, rows) == 1)
     if part is not None:
         work, sp = part
@@ -81,7 +81,7 @@ def test_few_rows_against_fp64(nf4, orc, shape, rows, nested, bs, bs2, dtype):
                                                          ((4088, 2048), 17, 2, True, torch.float16),
                                                          ((2560, 9728), 50, 1, True, torch.bfloat16)])
 def test_few_row_norm_equals_its_sums_reduced_then_normed(nf4, shape, rows, epi, nested, dtype):
-    """`matmul_norm(few_rows=True)`: its first output is the sums of
+    """`matmul_norm(span=True)`: its first output is the sums of
     `matmul_partials` added in split order with the epilogue's roundings, its
     second `fusedops.rms_norm` of it, bit for bit."""
     from ttspipe_amd import fusedops
@@ -92,8 +92,8 @@ def test_few_row_norm_equals_its_sums_reduced_then_normed(nf4, shape, rows, epi,
     x = from_bits(randn_bits(rows * K, dtype, seed=rows, scale=0.5), dtype).view(1, rows, K)
     r = from_bits(randn_bits(rows * M, dtype, seed=rows + 1), dtype).view(1, rows, M) if epi else None
     g = torch.rand(M, generator=torch.Generator().manual_seed(M)).add(0.5).to(dtype).cuda()
-    y, yn = nf4.matmul_norm(lin, x, g, 1e-5, epi=epi, operand=r, few_rows=True)
-    work, sp = nf4.matmul_partials(lin, x, few_rows=True)
+    y, yn = nf4.matmul_norm(lin, x, g, 1e-5, epi=epi, operand=r, span=True)
+    work, sp = nf4.matmul_partials(lin, x, span=True)
     acc = work[0].clone()
     for z in range(1, sp):
         acc += work[z]

@@ -767,3 +767,34 @@ def test_wide_span_prefill_matches_its_narrow_spans(roomy, monkeypatch, start, n
     for i, ((k0, v0), (k1, v1)) in enumerate(zip(got["eager"]["kv"], got["narrow"]["kv"])):
         bar = 2e-3 if i == 0 else 2e-2
         assert _rel(k0, k1) < bar and _rel(v0, v1) < bar
+
+
+@pytest.fixture(scope="module")
+def two_layers():
+    """Two layers of the benchmark model's widths."""
+    import dataclasses
+
+    from ttspipe_amd.dualar import DualARConfig, SyntheticDualAR
+
+    return SyntheticDualAR(dataclasses.replace(DualARConfig(), n_layer=2))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("start,n", [(0, 1900), (0, 1000), (0, 1500), (700, 1024)])
+def test_wide_spans_keep_the_bits_of_narrow_ones(two_layers, monkeypatch, start, n):
+    """At the model's widths a prompt's KV rows and logits are the same bits
+    whether its 512-row spans run one by one or 2, 3 or 4 together."""
+    from ttspipe_amd import dualar
+
+    m = two_layers
+    toks = _tokens(m, n, 3 + n)
+    got = []
+    for wide in (1, 4):
+        monkeypatch.setattr(dualar, "WIDE_SPANS", wide)
+        assert m.prefill(toks, start, graphed=False)
+        torch.cuda.synchronize()
+        got.append((_kv_state(m, start + n), m.logits.clone()))
+    (kva, la), (kvb, lb) = got
+    for i, ((ka, va), (kb, vb)) in enumerate(zip(kva, kvb)):
+        assert torch.equal(ka, kb) and torch.equal(va, vb), f"layer {i}"
+    assert torch.equal(la, lb)

@@ -20,15 +20,16 @@ def nf4():
 
 
 def test_tile_splits_follow_the_split_plan():
-    """The split plan's, or 1 in place of 2 at 256 rows and more where the row
-    is too wide for the norm's reduce."""
+    """The split plan's, or from 256 rows 1 in place of 2 where the row is too
+    wide for the norm's reduce and 2 in place of 4 at 64 to 127 K-steps."""
     from ttspipe_amd import _lib
 
     lib = _lib.load()
     for M, K in ((9728, 2560), (6144, 2560), (2560, 9728), (2560, 4096), (4096, 2560), (1536, 1024), (1540, 2560)):
         for N in (65, 100, 128, 200, 256, 257, 384, 400, 512):
             plan, tile = lib.ttsp_nf4_gemm_splits(M, K, N), lib.ttsp_nf4_gemm_tile_splits(M, K, N)
-            assert tile == plan or (tile == 1 and plan == 2 and N >= 256 and M > 4096)
+            assert tile == plan or (N >= 256 and ((tile == 1 and plan == 2 and M > 4096)
+                                                  or (tile == 2 and plan == 4 and 64 <= K // 64 < 128)))
 
 
 @pytest.mark.gpu

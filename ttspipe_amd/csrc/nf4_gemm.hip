@@ -344,21 +344,49 @@ extern "C" int ttsp_nf4_gemm_splits(int M, int K, int N) {
   return gemm_plan(M, K, N);
 }
 
-// The splits a caller with a workspace should take at 65 to 512 rows:
-// ttsp_nf4_gemm_splits', but unsplit instead of 2 ways at 256 rows and more
-// where no norm follows in the reduce (M past its widest row): 9728 x 2560 at
-// 256 rows 28.0 us against 32 and a 10 us reduce, 6144 x 2560 at 512 28.7
-// against 30.3 and 7. (Sums that another kernel adds keep the two splits.)
-extern "C" int ttsp_nf4_gemm_tile_splits(int M, int K, int N) {
+// The splits a caller with a workspace should take from 65 rows:
+// ttsp_nf4_gemm_splits', but from 256 rows unsplit instead of 2 ways where no
+// norm follows in the reduce (M past its widest row): 9728 x 2560 at 256 rows
+// 28.0 us against 32 and a 10 us reduce, 6144 x 2560 at 512 28.7 against 30.3
+// and 7 (sums that another kernel adds keep the two splits); and 2 instead of
+// 4 where a split still has 32 K-steps or more but fewer than 64 (2560 x 4096:
+// 18.1 against 18.1 us at 256 rows, 26.9 against 26.5 at 512, half the sums to
+// reduce).
+namespace ttsp {
+
+int tile_splits(int M, int K, int N) {
   if (M <= 0 || K <= 0 || N <= 1 || K % 128) return 1;
-  return M > 64 * 8 * NRM_CH && dl_plan(M, K, N) == 2 ? 1 : gemm_plan(M, K, N);
+  const int dl = dl_plan(M, K, N), plan = gemm_plan(M, K, N);
+  if (N <= 64 || !dl) return plan;
+  if (M > 64 * 8 * NRM_CH && dl == 2) return 1;
+  return dl == 4 && K / KT < 128 && K / KT % 4 == 0 ? 2 : plan;
 }
+
+// Estimated us of the tile kernel from 65 rows: rounds of 256 workgroups, each
+// its K-steps (measured a step: 0.75 us with both K halves in a workgroup,
+// 0.95 of 256 weight rows, 0.66 of 128) and ~5 us of first loads and epilogue;
+// a split's sums and reduce as the dense plan prices them. The forms follow
+// nf4_gemm_tile.hip's choice.
+double tile_estimate(int M, int K, int N) {
+  const int z = tile_splits(M, K, N), steps = K / KT / z;
+  const long long t64 = gemm_tiles(M, N, 64, 128) * z, t128 = gemm_tiles(M, N, 128, 128) * z,
+                  t256 = gemm_tiles(M, N, 256, 128) * z;
+  double us = t64 <= 256 ? steps / 2 * 0.75 + 5.0
+              : t256 >= 128 ? (double)((t256 + 255) / 256) * (steps * 0.95 + 5.0)
+                            : (double)((t128 + 255) / 256) * (steps * 0.66 + 5.0);
+  if (z > 1) us += 4.0 + (double)z * N * M * 8.0 / 4e6;
+  return us;
+}
+
+}  // namespace ttsp
+
+extern "C" int ttsp_nf4_gemm_tile_splits(int M, int K, int N) { return tile_splits(M, K, N); }
 
 extern "C" int ttsp_nf4_gemm_split(const void* X, int x_dtype, const uint8_t* W, const uint8_t* A8,
                                    const float* AMAX, const float* CODE2, float offset, const float* LUT,
                                    void* Y, const void* R, int epi, int M, int K, int N, int blocksize,
                                    int blocksize2, float* work, int splits, hipStream_t stream) {
-  if (N <= 1 || splits < 1 || splits != ttsp_nf4_gemm_splits(M, K, N))
+  if (N <= 1 || splits < 1 || (splits != ttsp_nf4_gemm_splits(M, K, N) && splits != tile_splits(M, K, N)))
     return (int)hipErrorInvalidValue;
   if (splits == 1)
     return ttsp_nf4_gemm(X, x_dtype, W, A8, AMAX, CODE2, offset, LUT, Y, R, epi, M, K, N, blocksize,
@@ -370,7 +398,7 @@ extern "C" int ttsp_nf4_gemm_split(const void* X, int x_dtype, const uint8_t* W,
   if (!work || (uintptr_t)work % 16) return (int)hipErrorInvalidValue;
   const bool vec = M % 8 == 0 && (uintptr_t)Y % 16 == 0 && (!epi || (uintptr_t)R % 16 == 0);
   return gemm_mfma(X, x_dtype, W, A8, AMAX, CODE2, offset, LUT, Y, R, epi | (vec ? 4 : 0), M, K, N, bs_shift,
-                   bs2_shift, gemm_plan(M, K, N), work, stream);
+                   bs2_shift, splits, work, stream);
 }
 
 static int log2_of(int v) {
@@ -428,7 +456,8 @@ extern "C" int ttsp_nf4_gemm_split_norm(const void* X, int x_dtype, const uint8_
                                         void* Y, const void* R, int epi, int M, int K, int N, int blocksize,
                                         int blocksize2, float* work, int splits, const void* G, float eps, void* YN,
                                         hipStream_t stream) {
-  if (N <= 1 || splits < 2 || splits != ttsp_nf4_gemm_splits(M, K, N) || (splits != 2 && splits != 4 && splits != 8))
+  if (N <= 1 || (splits != 2 && splits != 4 && splits != 8) ||
+      (splits != ttsp_nf4_gemm_splits(M, K, N) && splits != tile_splits(M, K, N)))
     return (int)hipErrorInvalidValue;
   if (M % 8 || M > 64 * 8 * NRM_CH || !G || !YN || !work) return (int)hipErrorInvalidValue;
   if ((uintptr_t)Y % 16 || (uintptr_t)YN % 16 || (uintptr_t)G % 16 || (uintptr_t)work % 16 ||
@@ -440,7 +469,7 @@ extern "C" int ttsp_nf4_gemm_split_norm(const void* X, int x_dtype, const uint8_
                          &bs2_shift))
     return rc;
   if (int rc = gemm_mfma(X, x_dtype, W, A8, AMAX, CODE2, offset, LUT, Y, R, epi, M, K, N, bs_shift, bs2_shift,
-                         gemm_plan(M, K, N), work, stream, false))
+                         splits, work, stream, false))
     return rc;
   return gemm_reduce_norm(x_dtype, work, splits, Y, R, epi, M, N, G, eps, YN, stream);
 }

@@ -27,7 +27,7 @@
 // 57 against 70 us). 128 x 128 and 160 x 128 with two workgroups a CU were
 // within 5 % at 2048 rows and up to 20 % behind at 700; 256 x 256 leaves too
 // few tiles. Sums run along K in the same order in every tile shape, so the
-// shape does not change a bit of the result.
+// shape does not change a bit of the result; see dense_plan for the order.
 #include "nf4_mfma.h"
 
 namespace ttsp {
@@ -96,18 +96,36 @@ __device__ __forceinline__ void mul_slice(const u32x4 (&af)[C::TM], const u32x4 
     for (int b = 0; b < C::TN; ++b) acc[a][b] = mfma32<DT>(af[a], bf[b], acc[a][b]);
 }
 
+// The end of a run of K-steps: its sums join those of the runs before (fold 1:
+// the first run), as a K split's reduce adds its splits.
+template <typename C>
+__device__ __forceinline__ void end_run(f32x16_v (&acc)[C::TM][C::TN], f32x16_v (&sum)[C::TM][C::TN], int fold) {
+#pragma unroll
+  for (int a = 0; a < C::TM; ++a)
+#pragma unroll
+    for (int b = 0; b < C::TN; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        sum[a][b][r] = fold == 1 ? acc[a][b][r] : __fadd_rn(sum[a][b][r], acc[a][b][r]);
+        acc[a][b][r] = 0.0f;
+      }
+}
+
 // One step: stage rd has landed for every wave; the stage dst, which every
 // wave has finished reading, takes the operands at K byte offset koff. The
 // last slice's fragments are read here and multiplied in the next call.
-template <int DT, typename C, bool FIRST, typename X>
+template <int DT, typename C, bool FIRST, bool RUNS, typename X>
 __device__ __forceinline__ void step(const X& c, const uint8_t* __restrict__ rd, uint8_t* __restrict__ dst, int koff,
-                                     u32x4 (&af)[2][C::TM], u32x4 (&bf)[2][C::TN], f32x16_v (&acc)[C::TM][C::TN]) {
+                                     u32x4 (&af)[2][C::TM], u32x4 (&bf)[2][C::TN], f32x16_v (&acc)[C::TM][C::TN],
+                                     f32x16_v (&sum)[RUNS ? C::TM : 1][RUNS ? C::TN : 1], int fold) {
   // (SL is even: slice kk's fragments are in set kk & 1, the pending ones in set 1)
   read_slice<C>(rd, c.afrag[0], c.bfrag[0], af[0], bf[0]);
   if constexpr (!FIRST) load_stage<C, C::LP>(c, dst, koff, 0);
   __builtin_amdgcn_sched_barrier(0);
   if constexpr (!FIRST) mul_slice<DT, C>(af[1], bf[1], acc);
   __builtin_amdgcn_sched_barrier(0);
+  if constexpr (RUNS && !FIRST)
+    if (fold) end_run<C>(acc, sum, fold);
 #pragma unroll
   for (int kk = 0; kk + 1 < C::SL; ++kk) {
     read_slice<C>(rd, c.afrag[kk + 1], c.bfrag[kk + 1], af[(kk + 1) & 1], bf[(kk + 1) & 1]);
@@ -118,10 +136,10 @@ __device__ __forceinline__ void step(const X& c, const uint8_t* __restrict__ rd,
   }
 }
 
-template <int DT, typename C, bool SW>
+template <int DT, typename C, bool SW, bool RUNS>
 __global__ __launch_bounds__(64 * C::NW) void nf4_gemm_dense_kernel(
     const uint16_t* __restrict__ X, const uint16_t* __restrict__ W, uint16_t* __restrict__ Y,
-    const uint16_t* __restrict__ R, int epi, int M, int K, int N, float* __restrict__ YP) {
+    const uint16_t* __restrict__ R, int epi, int M, int K, int N, int runs, float* __restrict__ YP) {
 #if defined(__HIP_DEVICE_COMPILE__)
   __shared__ __align__(16) uint8_t ring0[C::STAGE];
   __shared__ __align__(16) uint8_t ring1[C::STAGE];
@@ -162,7 +180,7 @@ __global__ __launch_bounds__(64 * C::NW) void nf4_gemm_dense_kernel(
     }
 #pragma unroll
     for (int kk = 0; kk < C::SL; ++kk) {
-      const int r = lane & 31, sg = 2 * kk + (lane >> 5);
+      const int r = lane & 31, sg = 4 * (lane >> 5) + kk;  // (the tile kernel's order of a step's products)
       const uint32_t o = r * C::ROWB + ((sg ^ C::swz(r)) << 4);
       c.afrag[kk] = o + wm * C::TM * 32 * C::ROWB;
       c.bfrag[kk] = o + wn * C::TN * 32 * C::ROWB + C::BM * C::ROWB;
@@ -175,6 +193,7 @@ __global__ __launch_bounds__(64 * C::NW) void nf4_gemm_dense_kernel(
     for (int b = 0; b < C::TN; ++b)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.0f;
+  f32x16_v sum[RUNS ? C::TM : 1][RUNS ? C::TN : 1];
   u32x4 af[2][C::TM], bf[2][C::TN];
   constexpr int L = C::LA + C::LB, SB = C::KT * 2;
   const int last = (nsteps - 1) * SB;
@@ -194,11 +213,16 @@ __global__ __launch_bounds__(64 * C::NW) void nf4_gemm_dense_kernel(
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
-  step<DT, C, true>(c, ring0, ring0, 0, af, bf, acc);
+  step<DT, C, true, RUNS>(c, ring0, ring0, 0, af, bf, acc, sum, 0);
+  // RUNS: the steps left of this run, and the fold its end takes
+  int left = RUNS ? nsteps / runs : 0, fold = 1;
   // step s reads stage s % ST and refills stage (s - 1) % ST with step s - 1 + ST
   auto one = [&](int s, const uint8_t* rd, uint8_t* dst) {
     meet();
-    step<DT, C, false>(c, rd, dst, min((s - 1 + C::ST) * SB, last), af, bf, acc);
+    int f = 0;
+    if constexpr (RUNS)
+      if (--left == 0) f = fold, fold = 2, left = nsteps / runs;
+    step<DT, C, false, RUNS>(c, rd, dst, min((s - 1 + C::ST) * SB, last), af, bf, acc, sum, f);
   };
   int s = 1;
   if constexpr (C::ST == 2) {
@@ -217,6 +241,14 @@ __global__ __launch_bounds__(64 * C::NW) void nf4_gemm_dense_kernel(
     if (s + 1 < nsteps) one(s + 1, ring2, ring1);
   }
   mul_slice<DT, C>(af[1], bf[1], acc);
+  if constexpr (RUNS) {
+#pragma unroll
+    for (int a = 0; a < C::TM; ++a)
+#pragma unroll
+      for (int b = 0; b < C::TN; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[a][b][r] = __fadd_rn(sum[a][b][r], acc[a][b][r]);
+  }
 
   // accumulator r of lane l is (weight row 8 (r / 4) + 4 (l / 32) + r % 4, activation row l % 32)
   if (YP) {  // (M % 4 == 0: the plan)
@@ -354,44 +386,68 @@ int launch_dequant16(const DqMat& a, const DqMat& b, int mats, const float* LUT,
 typedef Cfg<256, 128, 4, 2, 3> Tall;
 typedef Cfg<192, 256, 2, 4, 2> Wide;
 
-template <int DT, typename C, bool SW>
+template <int DT, typename C, bool SW, bool RUNS>
 int launch_dense(const void* X, const uint16_t* W, void* Y, const void* R, int epi, int M, int K, int N, int splits,
-                 float* YP, hipStream_t st) {
+                 int runs, float* YP, hipStream_t st) {
   constexpr int BMO = SW ? C::BM / 2 : C::BM;
   const dim3 grid(((M + BMO - 1) / BMO) * ((N + C::BN - 1) / C::BN), 1, splits);
-  hipLaunchKernelGGL((nf4_gemm_dense_kernel<DT, C, SW>), grid, dim3(64 * C::NW), 0, st, (const uint16_t*)X, W,
-                     (uint16_t*)Y, (const uint16_t*)R, epi, M, K, N, YP);
+  hipLaunchKernelGGL((nf4_gemm_dense_kernel<DT, C, SW, RUNS>), grid, dim3(64 * C::NW), 0, st, (const uint16_t*)X, W,
+                     (uint16_t*)Y, (const uint16_t*)R, epi, M, K, N, runs, YP);
   TTSP_RETURN_LAUNCH();
 }
+
+}  // namespace
+}  // namespace ttsp
+
+extern "C" int ttsp_nf4_gemm_splits(int M, int K, int N);
+
+namespace ttsp {
+namespace {
 
 struct DensePlan {
   bool wide;
   int splits;  // 0: not served
+  int runs;    // of each split's K-steps
 };
 
 long long tiles(int M, int N, int bm, int bn) { return (long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
 
-// Estimated us of one product: rounds of 256 workgroups, each its K-steps
-// (measured 0.72 us a 256 x 128 step, 1.05 a 192 x 256 step) and ~5 us of
-// first loads and epilogue; a K split adds the partial sums' traffic and a
-// launch. The split (each at least 8 steps) and the tile with the least win.
-DensePlan dense_plan(int M, int K, int N) {
-  const int steps = K / 64;
-  DensePlan best{false, 0};
+// The sums' order: the K splits the tile kernel takes at 512 rows, each summed
+// along K and then added in order, whether as splits here or as runs inside a
+// workgroup. A prompt's spans then give the same bits run together as one by
+// one. Estimated us: rounds of 256 workgroups, each its K-steps (measured 0.72
+// us a 256 x 128 step, 1.05 a 192 x 256 step) and ~5 us of first loads and
+// epilogue; splits add the partial sums' traffic and a launch. The least wins.
+DensePlan dense_plan(int M, int K, int N, double* us_out = nullptr) {
+  const int steps = K / 64, parts = ttsp_nf4_gemm_splits(M, K, 512);
+  DensePlan best{false, 0, 1};
   double least = 0.0;
   for (int wide = 0; wide < 2; ++wide)
-    for (int sp = 1; sp <= 4; sp *= 2) {
-      if (sp > 1 && (steps % sp || steps / sp < 8 || M % 4)) break;
+    for (int sp = 1; sp <= parts; sp += parts - 1) {
+      if (sp > 1 && M % 4) break;
       const long long t = (wide ? tiles(M, N, Wide::BM, Wide::BN) : tiles(M, N, Tall::BM, Tall::BN)) * sp;
       double us = (double)((t + 255) / 256) * (steps / sp * (wide ? 1.05 : 0.72) + 5.0);
       if (sp > 1) us += 4.0 + (double)sp * N * M * 8.0 / 4e6;
-      if (!best.splits || us < least) best = DensePlan{wide != 0, sp}, least = us;
+      if (!best.splits || us < least) best = DensePlan{wide != 0, sp, parts / sp}, least = us;
+      if (parts == 1) break;
     }
+  if (us_out) *us_out = least;
   return best;
+}
+
+template <int DT>
+int dense_form(const DensePlan& p, const void* X, const uint16_t* W, void* Y, const void* R, int epi, int M, int K,
+               int N, float* YP, hipStream_t st) {
+  if (p.runs > 1)
+    return p.wide ? launch_dense<DT, Wide, false, true>(X, W, Y, R, epi, M, K, N, p.splits, p.runs, YP, st)
+                  : launch_dense<DT, Tall, false, true>(X, W, Y, R, epi, M, K, N, p.splits, p.runs, YP, st);
+  return p.wide ? launch_dense<DT, Wide, false, false>(X, W, Y, R, epi, M, K, N, p.splits, 1, YP, st)
+                : launch_dense<DT, Tall, false, false>(X, W, Y, R, epi, M, K, N, p.splits, 1, YP, st);
 }
 
 }  // namespace
 
+double tile_estimate(int M, int K, int N);
 int gemm_reduce(int dt, const float* YP, int splits, void* Y, const void* R, int epi, int M, int N, hipStream_t st);
 
 constexpr int DENSE_MIN_N = 513;
@@ -412,15 +468,17 @@ static bool dense_fits(int M, int K, int N, int mats) {
 using namespace ttsp;
 
 // The K splits `ttsp_nf4_gemm_dense` takes a product in, 0 where it does not
-// serve it. Served from DENSE_MIN_N rows (one row more than the tile
-// kernel's plans; calls at 513 rows, fused kernels against this: 9728 x 2560
-// 69 -> 49 us, 2560 x 9728 90 -> 57, 2560 x 4096 43 -> 37, and 220 -> 119,
-// 225 -> 119, 101 -> 55 at 2048) for weights and products large enough to
-// pay for the second launch (4096 x 1024: 22 against 24 us at 513 rows, 42
-// against 26 at 2048).
+// serve it: small products, and below 1024 rows where the tile kernel's
+// estimate is lower, counting here the dequantisation's bytes at ~5.2 TB/s and
+// its launch (9728 x 2560 at 700 rows one round of tiles, 43 us against 50; at
+// 1024 two rounds, ~86 against 66; at 2048 114 against the 220 of the kernels
+// before both). From 1024 rows, a prompt's long spans, always: the order of
+// the sums is then the 512-row spans'.
 extern "C" int ttsp_nf4_gemm_dense_splits(int M, int K, int N) {
   if (!dense_fits(M, K, N, 1) || (long long)M * K < (1ll << 21) || (double)M * K * N < 2.5e9) return 0;
-  return dense_plan(M, K, N).splits;
+  double us = 0.0;
+  const DensePlan plan = dense_plan(M, K, N, &us);
+  return N >= 1024 || us + 3.0 + (double)M * K * 2.5 / 5.2e6 < tile_estimate(M, K, N) ? plan.splits : 0;
 }
 
 // Y = epilogue(X . W^T). `work` (16-byte aligned) holds M * K dense weights,
@@ -444,9 +502,7 @@ extern "C" int ttsp_nf4_gemm_dense(const void* X, int x_dtype, const uint8_t* W,
 #define TTSP_DENSE(DTV)                                                                                        \
   do {                                                                                                         \
     if (int rc = launch_dequant16<DTV>(m, m, 1, LUT, wd, nd, bs, bs2, stream)) return rc;                      \
-    if (int rc = plan.wide ? launch_dense<DTV, Wide, false>(X, wd, Y, R, e, M, K, N, splits, yp, stream)       \
-                           : launch_dense<DTV, Tall, false>(X, wd, Y, R, e, M, K, N, splits, yp, stream))      \
-      return rc;                                                                                               \
+    if (int rc = dense_form<DTV>(plan, X, wd, Y, R, e, M, K, N, yp, stream)) return rc;                        \
   } while (0)
   if (x_dtype == DT_BF16) TTSP_DENSE(DT_BF16);
   else TTSP_DENSE(DT_F16);
@@ -457,9 +513,10 @@ extern "C" int ttsp_nf4_gemm_dense(const void* X, int x_dtype, const uint8_t* W,
 }
 
 // Whether the SwiGLU pair is served as one matrix launch with the bits of two:
-// where each weight's own product is served unsplit.
+// where each weight's own product is served unsplit and in one run.
 extern "C" int ttsp_nf4_gemm_dense_swiglu_fits(int M, int K, int N) {
-  return dense_fits(M, K, N, 2) && ttsp_nf4_gemm_dense_splits(M, K, N) == 1 ? 1 : 0;
+  if (!dense_fits(M, K, N, 2) || ttsp_nf4_gemm_dense_splits(M, K, N) != 1) return 0;
+  return dense_plan(M, K, N).runs == 1 ? 1 : 0;
 }
 
 // Y = round(round(silu(X . W1^T)) * round(X . W3^T)); `work` holds 2 * M * K
@@ -484,8 +541,8 @@ extern "C" int ttsp_nf4_gemm_dense_swiglu(const void* X, int x_dtype, const uint
   const int e = (uintptr_t)Y % 16 == 0 ? 8 : 0;
   if (x_dtype == DT_BF16) {
     if (int rc = launch_dequant16<DT_BF16>(a, b, 2, LUT, wd, nd, bs, bs2, stream)) return rc;
-    return launch_dense<DT_BF16, Tall, true>(X, wd, Y, nullptr, e, M, K, N, 1, nullptr, stream);
+    return launch_dense<DT_BF16, Tall, true, false>(X, wd, Y, nullptr, e, M, K, N, 1, 1, nullptr, stream);
   }
   if (int rc = launch_dequant16<DT_F16>(a, b, 2, LUT, wd, nd, bs, bs2, stream)) return rc;
-  return launch_dense<DT_F16, Tall, true>(X, wd, Y, nullptr, e, M, K, N, 1, nullptr, stream);
+  return launch_dense<DT_F16, Tall, true, false>(X, wd, Y, nullptr, e, M, K, N, 1, 1, nullptr, stream);
 }

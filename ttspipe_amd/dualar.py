@@ -94,8 +94,11 @@ def prefill_spans(n: int):
 #: Spans of the largest bucket run together, up to this many of them a launch
 #: (2048 rows): the linears take a long span's rows in one product, which
 #: dequantises each weight once (1900 tokens after none, 12 layers: 11.7 ms in
-#: four spans of 512, 7.6 ms in one of 2048). More would only grow the
-#: activations: past 2048 rows the products gain nothing.
+#: four spans of 512, 7.7 ms in one of 2048). More would only grow the
+#: activations: past 2048 rows the products gain nothing. The products keep
+#: the order of the 512-row spans' sums and the attention runs per 512 rows,
+#: so a prompt's bits do not depend on how its spans are run together (a stack
+#: of layers can blow a difference in one rounding up to a different row).
 WIDE_SPANS = 4
 
 
@@ -568,6 +571,10 @@ class SyntheticDualAR:
                                            cfg.n_tokens, n, cfg.vocab_size, cfg.dim, x.data_ptr(),
                                            _lib.dtype_code(self.dtype), _lib.stream())
         self._check(rc, "ttsp_embed_sum_rows")
+        # a long span attends as the largest-bucket spans it is made of would
+        top, attend = PREFILL_BUCKETS[-1], None
+        if n > top and n % top == 0:
+            attend = [(r, r + top, top if r == 0 and width == n else cfg.max_seq_len) for r in range(0, n, top)]
         freqs = self.freqs.index_select(0, pos)
         mask = self.causal.index_select(0, pos)[None, None, :, :width]
         # each block hands the next its attention RMSNorm, written by w2's
@@ -575,7 +582,8 @@ class SyntheticDualAR:
         xn = None
         for i, blk in enumerate(self.layers):
             nxt = self.layers[i + 1].attention_norm if i + 1 < len(self.layers) else None
-            r = fusedlayer.prefill_block_chain(blk, x, freqs, mask, pos, xn=xn, next_norm=nxt, causal=True)
+            r = fusedlayer.prefill_block_chain(blk, x, freqs, mask, pos, xn=xn, next_norm=nxt, causal=True,
+                                               attend=attend)
             if r is None:
                 x, xn = blk(x, freqs, mask, pos), None
             else:

@@ -237,6 +237,23 @@ def _prefill_eligible(block, x, mask, input_pos) -> bool:
     return True
 
 
+def _attend_in_parts(q, kc, vc, input_pos, nh, nkv, parts):
+    """A long causal span's attention, `parts` of its rows a launch (each row
+    sees the cache up to its own position, so later parts' rows, which are in
+    the cache already, change nothing); (1, nh, S, 128), or None."""
+    import torch
+
+    from ttspipe_amd import fastpath
+
+    n = q.shape[2]
+    out = torch.empty(1, n, nh * HEAD_DIM, dtype=q.dtype, device=q.device)
+    for r0, r1, width in parts:
+        if fastpath.prefill_attention(q[:, :, r0:r1], kc[:, :, :width], vc[:, :, :width], None, nh, nkv, HEAD_DIM,
+                                      out=out[:, r0:r1], positions=input_pos[r0:r1]) is None:
+            return None
+    return out.view(1, n, nh, HEAD_DIM).transpose(1, 2)
+
+
 def prefill_block(block, x, freqs_cis, mask, input_pos):
     """`TransformerBlock.forward` for several positions (B = 1, S > 1), or None.
     The block of `prefill_block_chain` without a carried norm."""
@@ -244,7 +261,8 @@ def prefill_block(block, x, freqs_cis, mask, input_pos):
     return None if r is None else r[0]
 
 
-def prefill_block_chain(block, x, freqs_cis, mask, input_pos, *, xn=None, next_norm=None, causal=False):
+def prefill_block_chain(block, x, freqs_cis, mask, input_pos, *, xn=None, next_norm=None, causal=False,
+                        attend=None):
     """`(out, out_n)`: the block's output for several positions (B = 1, S > 1)
     and, with `next_norm` (an RMSNorm module), `next_norm(out)` for the next
     block (else None, and None for a span of up to `nf4gemv.FUSED_MAX_ROWS`
@@ -259,6 +277,9 @@ def prefill_block_chain(block, x, freqs_cis, mask, input_pos, *, xn=None, next_n
     `fastpath.CAUSAL_ROWS_MAX` rows then attends row by row as the decode
     step does (`fastpath.causal_rows_attention`), and a longer one computes
     the mask from `input_pos` in the attention kernel; neither reads it.
+    `attend` (with `causal`): `(first row, end row, window)` of each attention
+    launch, in order and covering the rows, each over the first `window` cache
+    positions; default one launch over the mask's width.
 
     The fork's block in its own order with the prefill kernels: RMSNorm,
     wqkv GEMM, q/k head norms + rotary + KV-cache write for every row in one
@@ -302,7 +323,7 @@ def prefill_block_chain(block, x, freqs_cis, mask, input_pos, *, xn=None, next_n
     # rotary / KV kernel, which adds them as the split's own reduce would
     part = None
     if qkv is None and rows_ok and a.wqkv._nf4_fast["M"] == (nh + 2 * nkv) * hd:
-        part = nf4gemv.matmul_partials(a.wqkv, xn, few_rows=True)
+        part = nf4gemv.matmul_partials(a.wqkv, xn, span=True)
     if part is None and qkv is None:
         qkv = nf4gemv.matmul(a.wqkv, xn)
         if qkv is None:
@@ -355,12 +376,15 @@ def prefill_block_chain(block, x, freqs_cis, mask, input_pos, *, xn=None, next_n
     if y is None:
         if mask.shape[-1] < k.shape[2]:
             k, v = k[:, :, : mask.shape[-1]], v[:, :, : mask.shape[-1]]
+        if causal and rows_ok and attend is not None:
+            y = _attend_in_parts(q, kc, vc, input_pos, nh, nkv, attend)
         # a causal span's mask follows from its positions: computed in the kernel, not read
-        y = fastpath.prefill_attention(q, k, v, mask, nh, nkv, hd, positions=input_pos if causal else None)
+        if y is None:
+            y = fastpath.prefill_attention(q, k, v, mask, nh, nkv, hd, positions=input_pos if causal else None)
         if y is None:
             y = fastpath.decode_attention(q, k, v, mask, nh, nkv, hd)
         y = y.transpose(1, 2).contiguous().view(bsz, n, nh * hd)
-    hh = nf4gemv.matmul_norm(a.wo, y, fn.weight, fn.eps, epi=nf4gemv.EPI_RESIDUAL, operand=x, few_rows=True)
+    hh = nf4gemv.matmul_norm(a.wo, y, fn.weight, fn.eps, epi=nf4gemv.EPI_RESIDUAL, operand=x, span=True)
     if hh is not None:
         h, hn = hh
     else:
@@ -385,7 +409,7 @@ def prefill_block_chain(block, x, freqs_cis, mask, input_pos, *, xn=None, next_n
     oo = None
     if u is not None and next_norm is not None:
         oo = nf4gemv.matmul_norm(ff.w2, u, next_norm.weight, next_norm.eps, epi=nf4gemv.EPI_RESIDUAL, operand=h,
-                                 few_rows=True)
+                                 span=True)
     if oo is not None:
         out, out_n = oo
     else:

@@ -236,7 +236,7 @@ def matmul(module, x, *, epi: int = EPI_NONE, operand=None, out=None):
 
 
 #: Rows the few-row kernel takes (`ttsp_nf4_gemm_few`), and from how many `matmul` lets it split K: at fewer the
-#: reduce launch costs what the split saves, unless the reduce runs anyway (`matmul_norm(few_rows=True)`).
+#: reduce launch costs what the split saves, unless the reduce runs anyway (`matmul_norm(span=True)`).
 FEW_MIN_ROWS, FEW_SPLIT_ROWS, FEW_MAX_ROWS = 9, 33, 64
 
 
@@ -248,7 +248,7 @@ def _few(lib, fast, x, dt, rows, out, operand, epi, work, norm_weight=None, eps=
 
 
 #: From this many rows `matmul` and `matmul_swiglu` ask for the dense form (the weight dequantised once a call into a
-#: workspace): below it the kernels that read the codes in place are as fast.
+#: workspace): below it the kernels that read the codes in place are faster.
 DENSE_MIN_ROWS = 513
 
 
@@ -261,12 +261,13 @@ def _dense(M: int, K: int, rows: int) -> bool:
 NORM_MAX_M = 4096
 
 
-def matmul_partials(module, x, *, few_rows: bool = False):
+def matmul_partials(module, x, *, span: bool = False):
     """`(work, splits)`: the K-split launch of `matmul(module, x)` without its
     reduce, work the fp32 partial sums [splits, rows, M] for a consumer that
     adds them in split order; None where the shape runs unsplit (or the
-    kernels do not take the call). `few_rows`: split 9 to 32 rows too, whose
-    `matmul` runs unsplit (it would pay a reduce launch; the consumer does not)."""
+    kernels do not take the call). `span`, the prompt block's: split 9 to 32 rows
+    too, whose `matmul` runs unsplit (it would pay a reduce launch; the
+    consumer does not)."""
     import torch
 
     fast = getattr(module, "_nf4_fast", None)
@@ -282,7 +283,7 @@ def matmul_partials(module, x, *, few_rows: bool = False):
     if rows < 2 or _dense(M, K, rows):
         return None
     lib = _lib.lib()
-    few = lib.ttsp_nf4_gemm_few_splits(M, K, rows) if few_rows or FEW_SPLIT_ROWS <= rows <= FEW_MAX_ROWS else 0
+    few = lib.ttsp_nf4_gemm_few_splits(M, K, rows) if span or FEW_SPLIT_ROWS <= rows <= FEW_MAX_ROWS else 0
     splits = few or lib.ttsp_nf4_gemm_splits(M, K, rows)
     if splits < 2:
         return None
@@ -299,14 +300,15 @@ def matmul_partials(module, x, *, few_rows: bool = False):
     return work, splits
 
 
-def matmul_norm(module, x, norm_weight, eps: float, *, epi: int = EPI_NONE, operand=None, few_rows: bool = False):
+def matmul_norm(module, x, norm_weight, eps: float, *, epi: int = EPI_NONE, operand=None, span: bool = False):
     """`(y, rms_norm(y))` for several rows with the norm folded into the
     split-K reduce, or None where that form does not serve the call (one row,
     an unsplit shape, M over NORM_MAX_M); y is `matmul(module, x, epi=epi,
     operand=operand)` and the second output is `fusedops.rms_norm(y,
-    norm_weight, eps)`, both bit for bit. `few_rows` serves 9 to 32 rows too,
-    whose `matmul` runs unsplit: y is then the sum of K splits (the norm's
-    launch adds them), rounded as a split's reduce rounds."""
+    norm_weight, eps)`, both bit for bit. `span`, the prompt block's: 9 to 32
+    rows too, whose `matmul` runs unsplit (y is then the sum of K splits, which
+    the norm's launch adds), and from 65 rows `ttsp_nf4_gemm_splits`' splits,
+    whose order of sums longer spans keep."""
     import torch
 
     fast = getattr(module, "_nf4_fast", None)
@@ -330,8 +332,8 @@ def matmul_norm(module, x, norm_weight, eps: float, *, epi: int = EPI_NONE, oper
         if operand.device != x.device or not operand.is_contiguous() or operand.data_ptr() % 16:
             return None
     lib = _lib.lib()
-    few = lib.ttsp_nf4_gemm_few_splits(M, K, rows) if few_rows or FEW_SPLIT_ROWS <= rows <= FEW_MAX_ROWS else 0
-    splits = few or lib.ttsp_nf4_gemm_splits(M, K, rows)
+    few = lib.ttsp_nf4_gemm_few_splits(M, K, rows) if span or FEW_SPLIT_ROWS <= rows <= FEW_MAX_ROWS else 0
+    splits = few or (lib.ttsp_nf4_gemm_splits if span else lib.ttsp_nf4_gemm_tile_splits)(M, K, rows)
     if splits not in (2, 4, 8):
         return None
     out = torch.empty((rows, M), dtype=x.dtype, device=x.device)
