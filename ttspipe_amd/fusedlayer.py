@@ -56,26 +56,26 @@ def stats() -> dict:
     return {**_stats, "ready": _lib.gpu_present() and _installed}
 
 
-def _eligible(block, x, mask, input_pos) -> bool:
+def _eligible(a, ff, x, mask, input_pos) -> bool:
     import torch
 
     from ttspipe_amd import nf4gemv
 
-    a, ff = block.attention, block.feed_forward
     if x.dim() != 3 or x.shape[0] != 1 or x.shape[1] != 1:
         return False
     if x.dtype not in (torch.float16, torch.bfloat16) or x.device.type != "cuda" or not x.is_contiguous():
         return False
-    if mask is None or input_pos is None or input_pos.numel() != 1 or a.kv_cache is None:
+    cache, nkv = a.kv_cache, a.n_local_heads
+    if mask is None or input_pos is None or input_pos.numel() != 1 or cache is None:
         return False
     if input_pos.dtype != torch.long or input_pos.device != x.device:
         return False
-    if a.head_dim != HEAD_DIM or a.n_head % a.n_local_heads or a.n_head // a.n_local_heads > 16:
+    if a.head_dim != HEAD_DIM or a.n_head % nkv or a.n_head // nkv > 16:
         return False
-    kc, vc = a.kv_cache.k_cache, a.kv_cache.v_cache
+    kc, vc = cache.k_cache, cache.v_cache
     if kc.dtype != x.dtype or vc.dtype != x.dtype or not (kc.is_contiguous() and vc.is_contiguous()):
         return False
-    if kc.shape[0] != 1 or kc.shape[1] != a.n_local_heads or kc.shape[3] != HEAD_DIM:
+    if kc.shape[0] != 1 or kc.shape[1] != nkv or kc.shape[3] != HEAD_DIM:
         return False
     for linear in (a.wqkv, a.wo, ff.w1, ff.w2, ff.w3):
         if getattr(linear, "bias", None) is not None or not nf4gemv.prepare(linear):
@@ -93,16 +93,19 @@ def decode_block(block, x, freqs_cis, mask, input_pos, *, workspace=None):
 
     from ttspipe_amd import fusedops, nf4gemv
 
-    if not _lib.gpu_present() or not _eligible(block, x, mask, input_pos):
+    if not _lib.gpu_present():
+        return None
+    a, ff = block.attention, block.feed_forward
+    if not _eligible(a, ff, x, mask, input_pos):
         return None
     ftype = _lib.dtype_code(freqs_cis.dtype) if freqs_cis is not None else None
     if ftype is None or not freqs_cis.is_contiguous() or freqs_cis.numel() != HEAD_DIM:
         return None
-    a = block.attention
     nh, nkv = a.n_head, a.n_local_heads
-    max_len = a.kv_cache.k_cache.shape[2]
+    kc, vc = a.kv_cache.k_cache, a.kv_cache.v_cache
+    max_len = kc.shape[2]
     nchunk = -(-min(mask.shape[-1], max_len) // CHUNK)
-    ws = workspace if workspace is not None else make_workspace(block, x, nchunk)
+    ws = workspace if workspace is not None else _Workspace(nh, nkv, x, ff.w1.out_features, nchunk)
     dt = _lib.dtype_code(x.dtype)
     lib = _lib.lib()
     st = _lib.stream()
@@ -117,13 +120,14 @@ def decode_block(block, x, freqs_cis, mask, input_pos, *, workspace=None):
     qn = getattr(a, "q_norm", None) if a.attention_qk_norm else None
     kn = getattr(a, "k_norm", None) if a.attention_qk_norm else None
     eps = float(qn.eps if qn is not None and qn.eps is not None else 1e-6)
-    h = _attn_wo(a, qkv, qn, kn, eps, freqs_cis, ftype, input_pos, x, ws, nchunk, dt, st)
-    if h is not None:  # attention and wo (+ residual) in one launch (short caches)
-        return _ffn(block, h, ws, x.shape)
+    if nchunk == 1:
+        h = _attn_wo(a, qkv, qn, kn, eps, freqs_cis, ftype, input_pos, x, ws, nchunk, dt, st)
+        if h is not None:  # attention and wo (+ residual) in one launch (short caches)
+            return _ffn(block, h, ws, x.shape)
     rc = lib.ttsp_attn_decode_qkv(
         qkv.data_ptr(), _lib.ptr(None if qn is None else qn.weight), _lib.ptr(None if kn is None else kn.weight),
-        eps, freqs_cis.data_ptr(), ftype, input_pos.data_ptr(), a.kv_cache.k_cache.data_ptr(),
-        a.kv_cache.v_cache.data_ptr(), ws["pm"].data_ptr(), ws["pl"].data_ptr(), ws["pacc"].data_ptr(),
+        eps, freqs_cis.data_ptr(), ftype, input_pos.data_ptr(), kc.data_ptr(),
+        vc.data_ptr(), ws["pm"].data_ptr(), ws["pl"].data_ptr(), ws["pacc"].data_ptr(),
         ws["y"].data_ptr(), nh, nkv, max_len, nchunk, float(HEAD_DIM**-0.5), dt, st)
     _lib.check(rc, "ttsp_attn_decode_qkv")
     h = nf4gemv.matmul(a.wo, ws["y"], epi=nf4gemv.EPI_RESIDUAL, operand=x, out=ws["h"])
@@ -177,30 +181,39 @@ def _ffn(block, h, ws, shape):
     return out.view(shape)
 
 
+class _Workspace(dict):
+    """The buffers of one `decode_block` call, each allocated when first asked
+    for (the common route takes seven of the eleven)."""
+
+    def __init__(self, nh, nkv, x, inter, nchunk):
+        D, HD = x.shape[-1], HEAD_DIM
+        self._kind = x.dtype, x.device
+        # name: (shape, fp32)
+        self._shapes = {
+            "xn": ((1, 1, D), False), "qkv": ((1, (nh + 2 * nkv) * HD), False), "q": ((nh * HD,), False),
+            "pm": ((nh * nchunk,), True), "pl": ((nh * nchunk,), True), "pacc": ((nh * nchunk * HD,), True),
+            "y": ((1, 1, nh * HD), False), "h": ((1, D), False), "hn": ((1, 1, D), False), "g1": ((1, inter), False),
+            "g": ((1, 1, inter), False),
+        }
+
+    def __missing__(self, name):
+        import torch
+
+        shape, fp32 = self._shapes[name]
+        dtype, device = self._kind
+        t = self[name] = torch.empty(shape, dtype=torch.float32 if fp32 else dtype, device=device)
+        return t
+
+
 def make_workspace(block, x, nchunk: int, *, with_out: bool = False) -> dict:
     """Buffers one `decode_block` call uses (reusable across calls of the same shape)."""
     import torch
 
     a, ff = block.attention, block.feed_forward
-    nh, nkv, D = a.n_head, a.n_local_heads, x.shape[-1]
-    inter = ff.w1.out_features
-    kw = dict(dtype=x.dtype, device=x.device)
-    f32 = dict(dtype=torch.float32, device=x.device)
-    ws = {
-        "xn": torch.empty((1, 1, D), **kw),
-        "qkv": torch.empty((1, (nh + 2 * nkv) * HEAD_DIM), **kw),
-        "q": torch.empty(nh * HEAD_DIM, **kw),
-        "pm": torch.empty(nh * nchunk, **f32),
-        "pl": torch.empty(nh * nchunk, **f32),
-        "pacc": torch.empty(nh * nchunk * HEAD_DIM, **f32),
-        "y": torch.empty((1, 1, nh * HEAD_DIM), **kw),
-        "h": torch.empty((1, D), **kw),
-        "hn": torch.empty((1, 1, D), **kw),
-        "g1": torch.empty((1, inter), **kw),
-        "g": torch.empty((1, 1, inter), **kw),
-    }
+    lazy = _Workspace(a.n_head, a.n_local_heads, x, ff.w1.out_features, nchunk)
+    ws = {name: lazy[name] for name in lazy._shapes}
     if with_out:
-        ws["out"] = torch.empty((1, D), **kw)
+        ws["out"] = torch.empty((1, x.shape[-1]), dtype=x.dtype, device=x.device)
     return ws
 
 

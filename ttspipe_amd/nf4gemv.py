@@ -179,39 +179,42 @@ def matmul(module, x, *, epi: int = EPI_NONE, operand=None, out=None):
     fast = getattr(module, "_nf4_fast", None)
     if fast is None:
         return None
-    dt = _lib.dtype_code(x.dtype)
-    if dt not in (_lib.DT_F16, _lib.DT_BF16) or x.device.type != "cuda":
+    dtype, device = x.dtype, x.device
+    dt = _lib.dtype_code(dtype)
+    if dt not in (_lib.DT_F16, _lib.DT_BF16) or device.type != "cuda":
         return None
     K, M = fast["K"], fast["M"]
-    if x.shape[-1] != K:
+    shape = x.shape
+    if shape[-1] != K:
         return None
-    flat = x.reshape(-1, K)
+    flat = x  # only its rows' address is used
     if not flat.is_contiguous() or flat.data_ptr() % 16:
-        flat = flat.contiguous()
+        flat = flat.reshape(-1, K).contiguous()
         if flat.data_ptr() % 16:
             return None
-    rows = flat.shape[0]
+    rows = flat.numel() // K
     if rows == 0:
-        return x.new_empty(*x.shape[:-1], M)
+        return x.new_empty(*shape[:-1], M)
     if epi != EPI_NONE:
-        if operand is None or operand.numel() != rows * M or operand.dtype != x.dtype:
+        if operand is None or operand.numel() != rows * M or operand.dtype != dtype:
             return None
-        if operand.device != x.device or not operand.is_contiguous():
+        if operand.device != device or not operand.is_contiguous():
             return None
-    if out is None:
-        out = torch.empty((rows, M), dtype=x.dtype, device=x.device)
-    elif out.dtype != x.dtype or out.numel() != rows * M or not out.is_contiguous():
+    given = out is not None
+    if not given:
+        out = torch.empty((*shape[:-1], M), dtype=dtype, device=device)
+    elif out.dtype != dtype or out.numel() != rows * M or not out.is_contiguous():
         return None
     lib = _lib.lib()
     dense = lib.ttsp_nf4_gemm_dense_splits(M, K, rows) if rows >= DENSE_MIN_ROWS else 0
     few = lib.ttsp_nf4_gemm_few_splits(M, K, rows) if FEW_SPLIT_ROWS <= rows <= FEW_MAX_ROWS else 0
     splits = lib.ttsp_nf4_gemm_tile_splits(M, K, rows) if rows > 1 and not dense and not few else 1
     if few:
-        work = torch.empty(few * rows * M, dtype=torch.float32, device=x.device) if few > 1 else None
+        work = torch.empty(few * rows * M, dtype=torch.float32, device=device) if few > 1 else None
         rc = _few(lib, fast, flat, dt, rows, out, operand, epi, work)
     elif dense:
         # the dequantised weight, then (K split) the partial sums
-        work = torch.empty(2 * M * K + (4 * dense * rows * M if dense > 1 else 0), dtype=torch.uint8, device=x.device)
+        work = torch.empty(2 * M * K + (4 * dense * rows * M if dense > 1 else 0), dtype=torch.uint8, device=device)
         rc = lib.ttsp_nf4_gemm_dense(
             flat.data_ptr(), dt, fast["w"], fast["a8"], fast["amax"], fast["code2"], fast["offset"],
             fast["lut"].data_ptr(), out.data_ptr(), _lib.ptr(operand) if epi else 0, epi, M, K, rows,
@@ -219,7 +222,7 @@ def matmul(module, x, *, epi: int = EPI_NONE, operand=None, out=None):
     elif splits > 1:
         # K split over workgroups (too few output tiles to fill the GPU): fp32
         # partials in a workspace, summed in split order by a second kernel
-        work = torch.empty(splits * rows * M, dtype=torch.float32, device=x.device)
+        work = torch.empty(splits * rows * M, dtype=torch.float32, device=device)
         rc = lib.ttsp_nf4_gemm_split(
             flat.data_ptr(), dt, fast["w"], fast["a8"], fast["amax"], fast["code2"], fast["offset"],
             fast["lut"].data_ptr(), out.data_ptr(), _lib.ptr(operand) if epi else 0, epi, M, K, rows,
@@ -232,7 +235,7 @@ def matmul(module, x, *, epi: int = EPI_NONE, operand=None, out=None):
     if rc:
         raise RuntimeError(f"ttsp_nf4_gemm failed: hipError_t {rc}")
     _stats["fast"] += 1
-    return out.view(*x.shape[:-1], M)
+    return out.view(*shape[:-1], M) if given else out
 
 
 #: Rows the few-row kernel takes (`ttsp_nf4_gemm_few`), and from how many `matmul` lets it split K: at fewer the
@@ -394,7 +397,10 @@ def matmul_fused(module, x, *, norm_weight=None, eps: float = 1e-6, module3=None
         return None
     if rows > 1 and _lib.lib().ttsp_gemv_rows_shape(M, K, rows, None, None, None):
         return None
-    if not gemv_fits(M, K):
+    fits = fast.get("gemv_fits")
+    if fits is None:
+        fits = fast["gemv_fits"] = gemv_fits(M, K)
+    if not fits:
         return None
     fast3 = None
     if module3 is not None:
@@ -415,8 +421,9 @@ def matmul_fused(module, x, *, norm_weight=None, eps: float = 1e-6, module3=None
             return None
         if operand.device != x.device or not operand.is_contiguous():
             return None
-    if out is None:
-        out = torch.empty((rows, M), dtype=x.dtype, device=x.device)
+    given = out is not None
+    if not given:
+        out = torch.empty((*x.shape[:-1], M), dtype=x.dtype, device=x.device)
     elif out.dtype != x.dtype or out.numel() != rows * M or not out.is_contiguous():
         return None
     f3 = fast3 or {"w": 0, "a8": 0, "amax": 0, "code2": 0, "offset": 0.0}
@@ -428,7 +435,7 @@ def matmul_fused(module, x, *, norm_weight=None, eps: float = 1e-6, module3=None
         if rc:
             raise RuntimeError(f"ttsp_nf4_gemv_fused_rows failed: hipError_t {rc}")
         _stats["fast"] += 2 if fast3 is not None else 1
-        return out.view(*x.shape[:-1], M)
+        return out.view(*x.shape[:-1], M) if given else out
     rc = _lib.lib().ttsp_nf4_gemv_fused(
         x.data_ptr(), dt, _lib.ptr(norm_weight), float(eps),
         fast["w"], fast["a8"], fast["amax"], fast["code2"], fast["offset"],
@@ -438,7 +445,7 @@ def matmul_fused(module, x, *, norm_weight=None, eps: float = 1e-6, module3=None
     if rc:
         raise RuntimeError(f"ttsp_nf4_gemv_fused failed: hipError_t {rc}")
     _stats["fast"] += 2 if fast3 is not None else 1
-    return out.view(*x.shape[:-1], M)
+    return out.view(*x.shape[:-1], M) if given else out
 
 
 def matmul_swiglu(module1, module3, x, *, out=None):
