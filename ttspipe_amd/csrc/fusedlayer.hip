@@ -38,7 +38,9 @@ namespace ttsp {
 // in split order and rounded as the split GEMM's own reduce does.
 constexpr int QKV_WAVES = 4;
 
-template <int DT, bool P = false>
+// HPW: neighbouring heads a wave takes, their loads in flight together (each
+// head is a chain of loads, sums and stores that one wave waits for).
+template <int DT, bool P, int HPW>
 __global__ __launch_bounds__(64 * QKV_WAVES) void qk_rope_kv_kernel(
     const uint16_t* __restrict__ QKV, const uint16_t* __restrict__ QW,
     const uint16_t* __restrict__ KW, float eps, const void* __restrict__ F, int ftype,
@@ -46,44 +48,61 @@ __global__ __launch_bounds__(64 * QKV_WAVES) void qk_rope_kv_kernel(
     uint16_t* __restrict__ VC, int nh, int nkv, int max_len, int qkv_rs, const float* __restrict__ YP = nullptr,
     int splits = 0) {
   const int lane = threadIdx.x & 63;
-  const int head = blockIdx.x * QKV_WAVES + (threadIdx.x >> 6);
-  const int row = blockIdx.y;
-  if (head >= nh + 2 * nkv) return;
+  const int head0 = (blockIdx.x * QKV_WAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * HPW;
+  const int row = blockIdx.y, total = nh + 2 * nkv;
+  if (head0 >= total) return;
   const long long pos = POS[row];
   if (pos < 0 || pos >= max_len) return;  // no cache slot to write: leave everything untouched
-  float lo, hi;
-  if constexpr (P) {
-    const size_t o = (size_t)row * qkv_rs + (size_t)head * HD, zs = (size_t)gridDim.y * qkv_rs;
-    lo = YP[o + lane];
-    hi = YP[o + lane + 64];
-    for (int z = 1; z < splits; ++z) {
-      lo += YP[z * zs + o + lane];
-      hi += YP[z * zs + o + lane + 64];
-    }
-    lo = Elem<DT>::load(Elem<DT>::store(lo));
-    hi = Elem<DT>::load(Elem<DT>::store(hi));
-  }
-  const uint16_t* src = P ? nullptr : QKV + (size_t)row * qkv_rs + (size_t)head * HD;
-  if (head >= nh + nkv) {
-    uint16_t* v = VC + ((long long)(head - nh - nkv) * max_len + pos) * HD;
-    v[lane] = P ? (uint16_t)Elem<DT>::store(lo) : src[lane];
-    v[lane + 64] = P ? (uint16_t)Elem<DT>::store(hi) : src[lane + 64];
-    return;
-  }
-  const bool is_q = head < nh;
-  const uint16_t* w = is_q ? QW : KW;
   const RopeF f = load_rope((const uint8_t*)F + (size_t)row * HD * (ftype == DT_F32 ? 4 : 2), ftype, lane);
-  if constexpr (!P) {
-    lo = Elem<DT>::load(src[lane]);
-    hi = Elem<DT>::load(src[lane + 64]);
+  float lo[HPW], hi[HPW];
+  uint16_t hl[HPW], hh[HPW];
+  // the norm weights, of the kinds of head this wave has, once
+  const uint16_t* const qw = head0 < nh ? QW : nullptr;
+  const uint16_t* const kw = head0 + HPW > nh && head0 < nh + nkv ? KW : nullptr;
+  const uint16_t qwl = qw ? qw[lane] : 0, qwh = qw ? qw[lane + 64] : 0;
+  const uint16_t kwl = kw ? kw[lane] : 0, kwh = kw ? kw[lane + 64] : 0;
+#pragma unroll
+  for (int u = 0; u < HPW; ++u) {
+    const int head = min(head0 + u, total - 1);
+    if constexpr (P) {
+      const size_t o = (size_t)row * qkv_rs + (size_t)head * HD, zs = (size_t)gridDim.y * qkv_rs;
+      lo[u] = YP[o + lane];
+      hi[u] = YP[o + lane + 64];
+      for (int z = 1; z < splits; ++z) {
+        lo[u] += YP[z * zs + o + lane];
+        hi[u] += YP[z * zs + o + lane + 64];
+      }
+    } else {
+      const uint16_t* src = QKV + (size_t)row * qkv_rs + (size_t)head * HD;
+      hl[u] = src[lane];
+      hh[u] = src[lane + 64];
+    }
   }
-  const uint16_t nwl = w ? w[lane] : 0, nwh = w ? w[lane + 64] : 0;
-  head_norm_rope<DT>(lo, hi, w != nullptr, nwl, nwh, eps, f, lane);
-  uint16_t* dst = is_q ? Q + (size_t)row * nh * HD + (size_t)head * HD
-                       : KC + ((long long)(head - nh) * max_len + pos) * HD;
-  dst[lane] = Elem<DT>::store(lo);
-  dst[lane + 64] = Elem<DT>::store(hi);
+#pragma unroll
+  for (int u = 0; u < HPW; ++u) {
+    const int head = head0 + u;
+    if (head >= total) return;
+    if constexpr (P) hl[u] = Elem<DT>::store(lo[u]), hh[u] = Elem<DT>::store(hi[u]);
+    if (head >= nh + nkv) {
+      uint16_t* v = VC + ((long long)(head - nh - nkv) * max_len + pos) * HD;
+      v[lane] = hl[u];
+      v[lane + 64] = hh[u];
+      continue;
+    }
+    const bool is_q = head < nh;
+    float l = Elem<DT>::load(hl[u]), h = Elem<DT>::load(hh[u]);
+    head_norm_rope<DT>(l, h, (is_q ? QW : KW) != nullptr, is_q ? qwl : kwl, is_q ? qwh : kwh, eps, f, lane);
+    uint16_t* dst = is_q ? Q + (size_t)row * nh * HD + (size_t)head * HD
+                         : KC + ((long long)(head - nh) * max_len + pos) * HD;
+    dst[lane] = Elem<DT>::store(l);
+    dst[lane + 64] = Elem<DT>::store(h);
+  }
 }
+
+// From this many rows a wave takes four heads: fewer, longer waves. 2048 rows
+// of 48 heads took 26.4 us with one head a wave, 20.1 with four; up to 32
+// rows one head a wave puts more of them on the chip at once.
+constexpr int QKV_HPW = 4, QKV_HPW_ROWS = 64;
 
 template <int DT>
 __global__ __launch_bounds__(1024) void attn_partial_kernel(
@@ -516,7 +535,7 @@ extern "C" int ttsp_qk_rope_kv(const void* QKV, const void* QW, const void* KW, 
   if (nh <= 0 || nkv <= 0 || max_len <= 0 || ftype < 0 || ftype > 2 || (uintptr_t)F % 4)
     return (int)hipErrorInvalidValue;
 #define TTSP_QK(DTV)                                                                            \
-  hipLaunchKernelGGL(qk_rope_kv_kernel<DTV>, dim3((nh + 2 * nkv + QKV_WAVES - 1) / QKV_WAVES), dim3(64 * QKV_WAVES), \
+  hipLaunchKernelGGL((qk_rope_kv_kernel<DTV, false, 1>), dim3((nh + 2 * nkv + QKV_WAVES - 1) / QKV_WAVES), dim3(64 * QKV_WAVES), \
                      0, stream,                                                                 \
                      (const uint16_t*)QKV, (const uint16_t*)QW, (const uint16_t*)KW, eps, F, ftype, \
                      POS, (uint16_t*)Q, (uint16_t*)KC, (uint16_t*)VC, nh, nkv, max_len, 0)
@@ -534,14 +553,21 @@ extern "C" int ttsp_qk_rope_kv_rows(const void* QKV, long long qkv_row_stride, c
   if (nh <= 0 || nkv <= 0 || max_len <= 0 || ftype < 0 || ftype > 2 || rows <= 0 || rows > 65535 ||
       qkv_row_stride < (long long)(nh + 2 * nkv) * HD || qkv_row_stride > (1LL << 30) || (uintptr_t)F % 4)
     return (int)hipErrorInvalidValue;
-#define TTSP_QKR(DTV)                                                                            \
-  hipLaunchKernelGGL(qk_rope_kv_kernel<DTV>, dim3((nh + 2 * nkv + QKV_WAVES - 1) / QKV_WAVES, rows),          \
+#define TTSP_QKR(DTV, HPWV)                                                                      \
+  hipLaunchKernelGGL((qk_rope_kv_kernel<DTV, false, HPWV>),                                      \
+                     dim3((nh + 2 * nkv + QKV_WAVES * HPWV - 1) / (QKV_WAVES * HPWV), rows),     \
                      dim3(64 * QKV_WAVES), 0, stream,                                           \
                      (const uint16_t*)QKV, (const uint16_t*)QW, (const uint16_t*)KW, eps, F, ftype, \
                      POS, (uint16_t*)Q, (uint16_t*)KC, (uint16_t*)VC, nh, nkv, max_len, (int)qkv_row_stride)
-  if (dtype == DT_F16) TTSP_QKR(DT_F16);
-  else if (dtype == DT_BF16) TTSP_QKR(DT_BF16);
+#define TTSP_QKRD(DTV)                              \
+  do {                                              \
+    if (rows >= QKV_HPW_ROWS) TTSP_QKR(DTV, QKV_HPW); \
+    else TTSP_QKR(DTV, 1);                          \
+  } while (0)
+  if (dtype == DT_F16) TTSP_QKRD(DT_F16);
+  else if (dtype == DT_BF16) TTSP_QKRD(DT_BF16);
   else return (int)hipErrorInvalidValue;
+#undef TTSP_QKRD
 #undef TTSP_QKR
   TTSP_RETURN_LAUNCH();
 }
@@ -554,13 +580,20 @@ extern "C" int ttsp_qk_rope_kv_rows_partials(const float* YP, int splits, const 
       splits < 2 || splits > 8 || (uintptr_t)F % 4)
     return (int)hipErrorInvalidValue;
   const int qkv_rs = (nh + 2 * nkv) * HD;
-#define TTSP_QKP(DTV)                                                                                           \
-  hipLaunchKernelGGL((qk_rope_kv_kernel<DTV, true>), dim3((nh + 2 * nkv + QKV_WAVES - 1) / QKV_WAVES, rows),      \
+#define TTSP_QKP(DTV, HPWV)                                                                                     \
+  hipLaunchKernelGGL((qk_rope_kv_kernel<DTV, true, HPWV>),                                                      \
+                     dim3((nh + 2 * nkv + QKV_WAVES * HPWV - 1) / (QKV_WAVES * HPWV), rows),                    \
                      dim3(64 * QKV_WAVES), 0, stream, nullptr, (const uint16_t*)QW, (const uint16_t*)KW, eps, F, \
                      ftype, POS, (uint16_t*)Q, (uint16_t*)KC, (uint16_t*)VC, nh, nkv, max_len, qkv_rs, YP, splits)
-  if (dtype == DT_F16) TTSP_QKP(DT_F16);
-  else if (dtype == DT_BF16) TTSP_QKP(DT_BF16);
+#define TTSP_QKPD(DTV)                              \
+  do {                                              \
+    if (rows >= QKV_HPW_ROWS) TTSP_QKP(DTV, QKV_HPW); \
+    else TTSP_QKP(DTV, 1);                          \
+  } while (0)
+  if (dtype == DT_F16) TTSP_QKPD(DT_F16);
+  else if (dtype == DT_BF16) TTSP_QKPD(DT_BF16);
   else return (int)hipErrorInvalidValue;
+#undef TTSP_QKPD
 #undef TTSP_QKP
   TTSP_RETURN_LAUNCH();
 }
