@@ -347,22 +347,33 @@ __global__ __launch_bounds__(64 * W * KG) void nf4_gemm_tile_kernel(
   }
   if (YP) {
     if (kg) return;
+    // each wave's 32 x 32 blocks through LDS of its own, so that a store writes
+    // whole 128-byte pieces of 8 rows, not 32 bytes of 32 (512 rows, traced:
+    // 6144 x 2560 in 2 splits 30.1 -> 27.3 us, 2560 x 4096 in 4 26.3 -> 22.4,
+    // 2560 x 9728 in 4 42.2 -> 40.6)
+    constexpr int PP = 36;  // floats a staged row
+    static_assert(4 * 32 * PP * 4 <= KG * STAGE, "four waves' blocks exceed a ring stage");
+    float* const ws = reinterpret_cast<float*>((wave & 4 ? &ring2[0][0] : &ring1[0][0]) + (wave & 3) * (32 * PP * 4));
     float* yp = YP + (size_t)blockIdx.z * N * M;
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
-      const int n = n0 + 32 * b + (lane & 31);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int m = mw + 8 * g + 4 * (lane >> 5);
-        const size_t o = (size_t)n * M + m;
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<float4*>(ws + (lane & 31) * PP + 8 * g + 4 * (lane >> 5)) =
+            make_float4(acc[b][4 * g], acc[b][4 * g + 1], acc[b][4 * g + 2], acc[b][4 * g + 3]);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int nl = 8 * j + (lane >> 3), n = n0 + 32 * b + nl, m = mw + 4 * (lane & 7);
+        const float4 v = *reinterpret_cast<const float4*>(ws + nl * PP + 4 * (lane & 7));
         if (n >= N || m >= M) continue;
+        const size_t o = (size_t)n * M + m;
         if ((M & 3) == 0) {
-          *reinterpret_cast<float4*>(yp + o) =
-              make_float4(acc[b][4 * g], acc[b][4 * g + 1], acc[b][4 * g + 2], acc[b][4 * g + 3]);
+          *reinterpret_cast<float4*>(yp + o) = v;
         } else {
           for (int c = 0; c < 4; ++c)
-            if (m + c < M) yp[o + c] = c == 0 ? acc[b][4 * g] : c == 1 ? acc[b][4 * g + 1] : c == 2 ? acc[b][4 * g + 2]
-                                                                                  : acc[b][4 * g + 3];
+            if (m + c < M) yp[o + c] = c == 0 ? v.x : c == 1 ? v.y : c == 2 ? v.z : v.w;
         }
       }
     }
