@@ -251,29 +251,40 @@ __global__ __launch_bounds__(64 * C::NW) void nf4_gemm_dense_kernel(
   }
 
   // accumulator r of lane l is (weight row 8 (r / 4) + 4 (l / 32) + r % 4, activation row l % 32)
-  if (YP) {  // (M % 4 == 0: the plan)
-    TTSP_WAIT_VM_LGKM0(0);  // the unread refills land before the workgroup's LDS is given back
-    float* yp = YP + (size_t)blockIdx.z * N * M;
-#pragma unroll
-    for (int b = 0; b < C::TN; ++b) {
-      const int n = n0 + (wn * C::TN + b) * 32 + (lane & 31);
-      const int mb = m0 + wm * C::TM * 32 + 4 * (lane >> 5);
-      float* row = yp + (size_t)n * M + mb;
-#pragma unroll
-      for (int a = 0; a < C::TM; ++a)
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-          if (n < N && mb + 32 * a + 8 * g < M)
-            *reinterpret_cast<float4*>(row + 32 * a + 8 * g) =
-                make_float4(acc[a][b][4 * g], acc[a][b][4 * g + 1], acc[a][b][4 * g + 2], acc[a][b][4 * g + 3]);
-    }
-    return;
-  }
   TTSP_WAIT_VM_LGKM0(0);
   __syncthreads();
   constexpr int PITCH = C::TM * 64 + 16, WB = 32 * PITCH, PERST = C::STAGE / WB;
   static_assert(C::NW <= 2 * PERST, "output staging exceeds the ring");
   uint8_t* const stg = wave < PERST ? ring0 + wave * WB : ring1 + (wave - PERST) * WB;
+  if (YP) {  // (M % 4 == 0: the plan)
+    // each 32 x 32 block through the wave's own LDS, so that a store writes
+    // whole 128-byte pieces of 8 rows, not 32 bytes of 32 (with the reduce, us:
+    // 2560 x 9728 in 4 splits at 1500 rows 104.2 -> 100.4, 1024 x 3072 at 1200
+    // 26.7 -> 24.2, 2560 x 4096 at 1024 44.9 -> 42.6)
+    constexpr int PP = 36;  // floats a staged row
+    static_assert(32 * PP * 4 <= WB, "a block exceeds the wave's staging");
+    float* const ws = reinterpret_cast<float*>(stg);
+    float* yp = YP + (size_t)blockIdx.z * N * M;
+#pragma unroll
+    for (int b = 0; b < C::TN; ++b)
+#pragma unroll
+      for (int a = 0; a < C::TM; ++a) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          *reinterpret_cast<float4*>(ws + (lane & 31) * PP + 8 * g + 4 * (lane >> 5)) =
+              make_float4(acc[a][b][4 * g], acc[a][b][4 * g + 1], acc[a][b][4 * g + 2], acc[a][b][4 * g + 3]);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int nl = 8 * j + (lane >> 3), n = n0 + (wn * C::TN + b) * 32 + nl;
+          const int m = m0 + (wm * C::TM + a) * 32 + 4 * (lane & 7);
+          const float4 v = *reinterpret_cast<const float4*>(ws + nl * PP + 4 * (lane & 7));
+          if (n < N && m < M) *reinterpret_cast<float4*>(yp + (size_t)n * M + m) = v;
+        }
+      }
+    return;
+  }
   const int ep = SW ? 2 : epi & 3;
   const bool vec = (M & 7) == 0 && (epi & 8);
   constexpr int CPR = C::TM * (SW ? 2 : 4);  // 16-byte output chunks of a row
