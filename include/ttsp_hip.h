@@ -429,9 +429,6 @@ int ttsp_prefill_max_groups(void);
  * a long cached prefix still spreads over the CUs. Host only. Replaces: nothing (the reference's SDPA picks its own split,
  * app/engine/fastpath.py:244-268). */
 int ttsp_prefill_attention_splits(int S, int nkv, int L);
-/* The splits that are fastest where the caller may choose: at most
- * ttsp_prefill_attention_splits'. ttsp_prefill_attention_split and _causal take any. */
-int ttsp_prefill_attention_plan(int S, int nkv, int L);
 
 /* ttsp_prefill_attention with the keys split into `splits` (1..16) ranges of
  * whole 32-key blocks over separate workgroups, each writing its unnormalised

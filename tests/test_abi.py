@@ -433,19 +433,3 @@ def test_swiglu_gemm_plan_on_the_host():
                                     None) == 1
     assert lib.ttsp_nf4_gemm_swiglu(p, 1, p, p, p, p, 0.0, p, None, p, p, 0.0, p, p, 9728, 2560, 512, 64, 256,
                                     None) == 1  # one weight nested, the other plain
-
-
-@pytest.mark.parametrize("S", [1, 32, 64, 200, 300, 390, 512, 700, 2048])
-@pytest.mark.parametrize("nkv", [1, 2, 8])
-@pytest.mark.parametrize("prefix", [0, 700, 1610, 8000])
-def test_attention_plan_stays_within_one_round(S, nkv, prefix):
-    """The split plan's count, or the most that keeps one round of 256 workgroups."""
-    from ttspipe_amd import _lib
-
-    lib = _lib.load()
-    L = S + prefix
-    plan, sp = lib.ttsp_prefill_attention_splits(S, nkv, L), lib.ttsp_prefill_attention_plan(S, nkv, L)
-    wg = nkv * -(-S // 32)
-    assert 1 <= sp <= plan
-    assert sp == 1 or wg * sp <= 256
-    assert sp == plan or wg * (sp + 1) > 256

@@ -159,6 +159,20 @@ def test_any_key_split_gives_the_unsplit_result(S, prefix, nh, nkv):
         assert relative_error(got, one) < 2 * TOL, sp  # each within TOL of fp64
 
 
+@pytest.mark.parametrize("S,prefix,nh,nkv", [(390, 1610, 32, 8), (200, 824, 32, 8), (700, 3396, 16, 8)])
+def test_prefill_attention_takes_the_plans_key_splits(S, prefix, nh, nkv):
+    """`fastpath.prefill_attention` runs `ttsp_prefill_attention_splits`' splits,
+    bit for bit (a split's largest key has probability 1 exactly, so fewer
+    splits than the plan's would round more)."""
+    from ttspipe_amd import _lib
+
+    splits = _lib.load().ttsp_prefill_attention_splits(S, nkv, S + prefix)
+    assert splits > 1
+    q, k, v, mask = _setup(S, prefix, nh, nkv, torch.bfloat16, seed=31)
+    y = _run(q, k, v, mask, nh, nkv)[0].float().cpu().numpy()
+    assert np.array_equal(y, _split_call(q, k, v, mask, nh, nkv, splits))
+
+
 @pytest.mark.parametrize("S,prefix", [(64, 1500), (512, 0), (200, 700)])
 def test_key_split_over_the_whole_cache_splits_the_live_keys(S, prefix):
     """K/V and the mask over the whole cache (4096 positions), as a captured

@@ -98,7 +98,6 @@ SIGNATURES: dict[str, list] = {
                                _vp],
     "ttsp_prefill_max_groups": [],
     "ttsp_prefill_attention_splits": [_i, _i, _i],
-    "ttsp_prefill_attention_plan": [_i, _i, _i],
     "ttsp_prefill_attention_split": [_vp, _ll, _ll, _vp, _ll, _ll, _vp, _ll, _ll, _vp, _ll, _vp, _i, _i, _i, _i, _f,
                                      _i, _vp, _i, _vp],
     "ttsp_prefill_attention_causal": [_vp, _ll, _ll, _vp, _ll, _ll, _vp, _ll, _ll, _vp, _vp, _i, _i, _i, _i, _f, _i,

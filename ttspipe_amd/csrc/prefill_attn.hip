@@ -590,20 +590,6 @@ static int prefill_splits(int S, int nkv, int L) {
   return sp;
 }
 
-// The splits a caller with a choice takes: at most prefill_splits', and no
-// more than one round of workgroups (each pays ~4 us before its first step).
-// Measured (32 query, 8 kv heads, masked, us, prefill_splits' count against
-// this): 390 rows over 1610 cached 42.8 (4) -> 36.4 (2), 200 over 1000 31.4
-// (8) -> 22.6 (4), 300 over 1800 40.9 (4) -> 30.4 (3), 700 over 1200 53.9 (2)
-// -> 42.8 (1). (Fewer, longer splits of a short run help over a long live
-// prefix, 64 rows over 2000 21.5 -> 18.9 with 8 for 16, but cost a prompt's
-// bucket, whose window is the whole cache and whose live prefix is short.)
-static int prefill_plan(int S, int nkv, int L) {
-  const long long wg = (long long)nkv * ((S + PA_QB - 1) / PA_QB);
-  const int sp = prefill_splits(S, nkv, L);
-  return sp > 1 ? (int)max(1LL, min((long long)sp, 256 / wg)) : sp;
-}
-
 }  // namespace ttsp
 
 using namespace ttsp;
@@ -731,11 +717,6 @@ extern "C" int ttsp_prefill_attention(const void* Q, long long q_seq_stride, lon
 extern "C" int ttsp_prefill_attention_splits(int S, int nkv, int L) {
   if (S <= 0 || nkv <= 0 || L <= 0) return 1;
   return prefill_splits(S, nkv, L);
-}
-
-extern "C" int ttsp_prefill_attention_plan(int S, int nkv, int L) {
-  if (S <= 0 || nkv <= 0 || L <= 0) return 1;
-  return prefill_plan(S, nkv, L);
 }
 
 extern "C" int ttsp_prefill_attention_split(const void* Q, long long q_seq_stride, long long q_head_stride,

@@ -69,10 +69,9 @@ def prefill_attention(q, k, v, mask, n_head, n_local_heads, head_dim, out=None, 
     supply that tensor), so the caller's `transpose(1, 2).contiguous()` is free;
     None when declined. A query whose mask row allows no key gets NaN, as the
     reference's softmax over all -inf scores. A short run over a long cache
-    splits its keys over several workgroups (`ttsp_prefill_attention_plan`,
-    never more than `ttsp_prefill_attention_splits`) through an fp32 workspace:
-    `work=` may supply one of at least `prefill_work_floats(...)` elements,
-    else it is allocated per call.
+    splits its keys over several workgroups (`ttsp_prefill_attention_splits`)
+    through an fp32 workspace: `work=` may supply one of at least
+    `prefill_work_floats(...)` elements, else it is allocated per call.
     `positions` (int64 (S,), contiguous): the causal mask at those positions
     (row i allows keys 0 .. positions[i], none at or past L) is computed in
     the kernel instead of read, and `mask` is not read (it may be None); the
@@ -93,7 +92,7 @@ def prefill_attention(q, k, v, mask, n_head, n_local_heads, head_dim, out=None, 
     elif out.shape != (1, seqlen, n_head * head_dim) or out.dtype != q.dtype or not out.is_contiguous():
         raise ValueError("out must be a contiguous (1, S, n_head * head_dim) tensor of q's dtype")
     lib = _lib.lib()
-    splits = lib.ttsp_prefill_attention_plan(seqlen, n_local_heads, L)
+    splits = lib.ttsp_prefill_attention_splits(seqlen, n_local_heads, L)
     need = prefill_work_floats(seqlen, n_head, splits)
     if splits > 1 and work is None:
         work = torch.empty(need, dtype=torch.float32, device=q.device)
