@@ -740,6 +740,41 @@ def test_wide_spans_merge_runs_of_the_largest_bucket():
         assert all(b <= WIDE_SPANS * top for _, _, b in wide)
 
 
+@pytest.mark.parametrize("max_len", [40, 320, 600, 1100, 2304, 4096])
+def test_prefill_sizes_cover_every_prompt(max_len):
+    """`capture_prefill`'s default list holds every span length that a prompt
+    which fits the cache is run in, and none that does not fit."""
+    from ttspipe_amd.dualar import _wide_spans, prefill_sizes, prefill_spans
+
+    sizes = prefill_sizes(max_len)
+    assert len(set(sizes)) == len(sizes) and max(sizes) <= max_len
+    for n in range(1, max_len + 1):
+        spans = prefill_spans(n)
+        if spans[-1][0] + spans[-1][2] <= max_len:
+            assert {b for _, _, b in _wide_spans(spans)} <= set(sizes), n
+
+
+@pytest.mark.gpu
+def test_default_captures_leave_nothing_for_a_long_prompt(two_layers, monkeypatch):
+    """After `capture_prefill()` and `capture_prefill(first=True)` prompts of up
+    to 1900 tokens replay only: no capture is left inside a request."""
+    m = two_layers
+    initial = _kv_state(m, m.cfg.max_seq_len)
+    m.capture_prefill()
+    m.capture_prefill(first=True)
+    for (k, v), blk in zip(initial, m.layers):  # captures put the rows they write back
+        assert torch.equal(k, blk.attention.kv_cache.k_cache) and torch.equal(v, blk.attention.kv_cache.v_cache)
+
+    def no_capture(*args, **kwargs):
+        raise AssertionError(f"captured {args} inside a prefill")
+
+    monkeypatch.setattr(m, "capture_prefill", no_capture)
+    for start, n in ((0, 1900), (0, 600), (300, 1500), (100, 1024), (0, 20)):
+        assert m.prefill(_tokens(m, n, n), start)
+    torch.cuda.synchronize()
+    _set_kv(m, initial)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("start,n", [(0, 1024), (0, 900), (200, 1000)])
 def test_wide_span_prefill_matches_its_narrow_spans(roomy, monkeypatch, start, n):

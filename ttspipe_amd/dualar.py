@@ -114,6 +114,13 @@ def _wide_spans(spans):
     return out
 
 
+def prefill_sizes(max_len: int):
+    """The span lengths `SyntheticDualAR.prefill` replays graphs of, for a cache
+    of `max_len` positions: the buckets, and the runs of the largest one."""
+    top = PREFILL_BUCKETS[-1]
+    return [b for b in (*PREFILL_BUCKETS, *(top * i for i in range(2, WIDE_SPANS + 1))) if b <= max_len]
+
+
 SMALL = DualARConfig(dim=512, n_layer=3, n_head=4, n_local_heads=2, intermediate_size=1024,
                      vocab_size=512, fast_dim=256, fast_n_layer=2, fast_n_head=2, fast_n_local_heads=1,
                      fast_intermediate_size=512, num_codebooks=4, codebook_size=512, max_seq_len=320,
@@ -595,7 +602,9 @@ class SyntheticDualAR:
         self._check(rc, "ttsp_argmax")
 
     def capture_prefill(self, buckets=None, first: bool = False) -> None:
-        """One graph per padded span length (after an eager warm-up of each);
+        """One graph per padded span length (after an eager warm-up of each;
+        default every length a prompt that fits the cache is run in, so that a
+        program that captures both sets at its start captures nothing later);
         `first`: the graphs for a span at position 0, whose attention window
         ends with the span (`prefill_first_graphs`), else the whole-cache ones
         (`prefill_graphs`).
@@ -608,7 +617,7 @@ class SyntheticDualAR:
         import torch
 
         graphs = self.prefill_first_graphs if first else self.prefill_graphs
-        for b in buckets or PREFILL_BUCKETS:
+        for b in buckets or prefill_sizes(self.cfg.max_seq_len):
             if b in graphs or b > self.cfg.max_seq_len:
                 continue
             width = b if first else None
@@ -631,9 +640,9 @@ class SyntheticDualAR:
     def prefill(self, tokens, start: int, graphed: bool = True) -> bool:
         """KV entries for `tokens` (n_tokens, n) int32 at [start, start + n),
         in spans of the largest bucket (up to `WIDE_SPANS` of them run as one)
-        and a last span padded to a bucket (the padding repeats the last real token; its KV entries land past the
-        prompt, where decoding overwrites them before reading them); the last
-        real position's token in `prefill_token`. False (nothing done) when
+        and a last span padded to a bucket (the padding repeats the last real
+        token; its KV entries land past the prompt, where decoding overwrites
+        them before reading them); the last real position's token in `prefill_token`. False (nothing done) when
         the padded span runs past the cache (reference: graphs.py:304-335).
         A span at position 0 attends over its own positions only (the window
         of the reference's causal mask there), not the whole cache."""
