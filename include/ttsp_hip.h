@@ -161,6 +161,10 @@ int ttsp_nf4_gemm_few(const void* X, int x_dtype, const uint8_t* W, const uint8_
  * work: 16-byte aligned, 2 * M * K bytes of dense weights, then (splits > 1)
  * splits * N * M fp32 partial sums. Other arguments as ttsp_nf4_gemm's. */
 int ttsp_nf4_gemm_dense_splits(int M, int K, int N);
+/* The K splits (ttsp_nf4_gemm_splits' or ttsp_nf4_gemm_tile_splits') of a
+ * 512-row product whose bits ttsp_nf4_gemm_dense keeps at 1024, 1536 and 2048
+ * rows; 0 where it keeps none. Host-only. */
+int ttsp_nf4_gemm_span_splits(int M, int K);
 int ttsp_nf4_gemm_dense(const void* X, int x_dtype, const uint8_t* W, const uint8_t* A8, const float* AMAX,
                         const float* CODE2, float offset, const float* LUT, void* Y, const void* R, int epi, int M,
                         int K, int N, int blocksize, int blocksize2, void* work, void* stream);

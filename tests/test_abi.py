@@ -433,3 +433,23 @@ def test_swiglu_gemm_plan_on_the_host():
                                     None) == 1
     assert lib.ttsp_nf4_gemm_swiglu(p, 1, p, p, p, p, 0.0, p, None, p, p, 0.0, p, p, 9728, 2560, 512, 64, 256,
                                     None) == 1  # one weight nested, the other plain
+
+
+def test_span_splits_name_the_products_that_keep_the_512_row_order():
+    """`ttsp_nf4_gemm_span_splits`: the 512-row splits of the model's layer; none
+    where the 512-row launch adds its K in halves (few 64 x 128 tiles) or the
+    dense form does not serve the weight."""
+    from ttspipe_amd import _lib
+
+    lib = _lib.load()
+    for M, K, splits in ((6144, 2560, 2), (2560, 4096, 4), (9728, 2560, 1), (2560, 9728, 4)):
+        assert lib.ttsp_nf4_gemm_span_splits(M, K) == splits == lib.ttsp_nf4_gemm_splits(M, K, 512)
+    for M, K in ((4096, 2560), (1024, 3072), (2048, 2048), (1540, 2560), (512, 512), (1024, 1024)):
+        assert lib.ttsp_nf4_gemm_span_splits(M, K) == 0
+    for M in range(64, 8000, 320):
+        for K in (512, 1024, 2560, 3072, 4096):
+            parts = lib.ttsp_nf4_gemm_splits(M, K, 512)
+            kept = lib.ttsp_nf4_gemm_span_splits(M, K)
+            assert kept in (0, parts)
+            if kept:
+                assert -(-M // 64) * 4 * parts > 256 and M * K >= 2**21

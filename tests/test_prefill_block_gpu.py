@@ -785,6 +785,7 @@ def test_wide_span_prefill_matches_its_narrow_spans(roomy, monkeypatch, start, n
     from ttspipe_amd import dualar
 
     m = roomy
+    monkeypatch.setattr(m, "merge_spans", True)  # (not of itself: its small weights' tiles change with the rows)
     toks = _tokens(m, n, 11 + n)
     initial = _kv_state(m, m.cfg.max_seq_len)
     got = {}
@@ -812,6 +813,34 @@ def two_layers():
     from ttspipe_amd.dualar import DualARConfig, SyntheticDualAR
 
     return SyntheticDualAR(dataclasses.replace(DualARConfig(), n_layer=2))
+
+
+@pytest.mark.gpu
+def test_spans_merge_only_where_that_keeps_their_bits(two_layers, monkeypatch):
+    """A model whose products add in another order over more rows (1024 wide:
+    its 512-row tiles add each split's K in halves) runs its 512-row spans one
+    by one: KV rows and logits do not depend on WIDE_SPANS."""
+    import dataclasses
+
+    from ttspipe_amd import dualar
+    from ttspipe_amd.dualar import SMALL, SyntheticDualAR
+
+    m = SyntheticDualAR(dataclasses.replace(SMALL, max_seq_len=1300, dim=1024, n_head=8, n_local_heads=2,
+                                            intermediate_size=3072))
+    assert two_layers.merge_spans and not m.merge_spans
+    n = 1000
+    toks = _tokens(m, n, 17)
+    initial = _kv_state(m, m.cfg.max_seq_len)
+    got = []
+    for wide in (1, 4):
+        monkeypatch.setattr(dualar, "WIDE_SPANS", wide)
+        _set_kv(m, initial)
+        assert m.prefill(toks, 0, graphed=False)
+        torch.cuda.synchronize()
+        got.append((_kv_state(m, n), m.logits.clone()))
+    for (ka, va), (kb, vb) in zip(got[0][0], got[1][0]):
+        assert torch.equal(ka, kb) and torch.equal(va, vb)
+    assert torch.equal(got[0][1], got[1][1])
 
 
 @pytest.mark.gpu

@@ -423,10 +423,11 @@ struct DensePlan {
 
 long long tiles(int M, int N, int bm, int bn) { return (long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
 
-// The sums' order: the K splits the tile kernel takes at 512 rows, each summed
-// along K and then added in order, whether as splits here or as runs inside a
-// workgroup. A prompt's spans then give the same bits run together as one by
-// one. Estimated us: rounds of 256 workgroups, each its K-steps (measured 0.72
+// The sums' order: the K splits ttsp_nf4_gemm_splits gives at 512 rows, each
+// summed along K and then added in order, whether as splits here or as runs
+// inside a workgroup. Where the 512-row product adds that way too
+// (ttsp_nf4_gemm_span_splits), a prompt's spans give the same bits run together
+// as one by one. Estimated us: rounds of 256 workgroups, each its K-steps (measured 0.72
 // us a 256 x 128 step, 1.05 a 192 x 256 step) and ~5 us of first loads and
 // epilogue; splits add the partial sums' traffic and a launch. The least wins.
 DensePlan dense_plan(int M, int K, int N, double* us_out = nullptr) {
@@ -459,6 +460,7 @@ int dense_form(const DensePlan& p, const void* X, const uint16_t* W, void* Y, co
 }  // namespace
 
 double tile_estimate(int M, int K, int N);
+bool tile_halves(int M, int N, int splits);
 int gemm_reduce(int dt, const float* YP, int splits, void* Y, const void* R, int epi, int M, int N, hipStream_t st);
 
 constexpr int DENSE_MIN_N = 513;
@@ -490,6 +492,18 @@ extern "C" int ttsp_nf4_gemm_dense_splits(int M, int K, int N) {
   double us = 0.0;
   const DensePlan plan = dense_plan(M, K, N, &us);
   return N >= 1024 || us + 3.0 + (double)M * K * 2.5 / 5.2e6 < tile_estimate(M, K, N) ? plan.splits : 0;
+}
+
+// The K splits of a 512-row product whose bits the dense form keeps at every
+// run of 512-row spans (1024, 1536 and 2048 rows); 0 where there are none: a
+// weight it does not serve at all of them, or one whose 512-row product adds
+// its K in halves (nf4_gemm_tile.hip's two-group form: few tiles, such as 4096
+// x 2560 or 1024 x 3072).
+extern "C" int ttsp_nf4_gemm_span_splits(int M, int K) {
+  for (int n = 1024; n <= 2048; n += 512)
+    if (!ttsp_nf4_gemm_dense_splits(M, K, n)) return 0;
+  const int parts = ttsp_nf4_gemm_splits(M, K, 512);
+  return tile_halves(M, 512, parts) ? 0 : parts;
 }
 
 // Y = epilogue(X . W^T). `work` (16-byte aligned) holds M * K dense weights,

@@ -431,11 +431,17 @@ int launch_tile(const void* X, const TileMat& a, const TileMat& b, const float* 
   TTSP_RETURN_LAUNCH();
 }
 
+}  // namespace
+
+bool tile_halves(int M, int N, int splits);
+
+namespace {
+
 template <int DT>
 int tile_form(const void* X, const TileMat& a, const float* LUT, void* Y, const void* R, int epi, int M, int K, int N,
               int bs_shift, int bs2_shift, int splits, float* YP, hipStream_t st) {
   const long long nt = (long long)((N + BN - 1) / BN) * splits;
-  if ((M + 63) / 64 * nt <= 256)
+  if (tile_halves(M, N, splits))
     return launch_tile<DT, 2, 2, 16, false>(X, a, a, LUT, Y, R, epi, M, K, N, bs_shift, bs2_shift, splits, YP, st);
   if ((M + 255) / 256 * nt >= 128)
     return launch_tile<DT, 8, 1, 32, false>(X, a, a, LUT, Y, R, epi, M, K, N, bs_shift, bs2_shift, splits, YP, st);
@@ -443,6 +449,12 @@ int tile_form(const void* X, const TileMat& a, const float* LUT, void* Y, const 
 }
 
 }  // namespace
+
+// Whether gemm_tile adds a split's sums as two K halves (tile_form's first
+// form) instead of in one run along K.
+bool tile_halves(int M, int N, int splits) {
+  return (long long)((M + 63) / 64) * ((N + BN - 1) / BN) * splits <= 256;
+}
 
 // splits > 1 writes fp32 partials to YP [splits][N][M] (the caller reduces
 // them and applies the epilogue), each split a whole even number of K-steps;

@@ -95,30 +95,35 @@ def prefill_spans(n: int):
 #: (2048 rows): the linears take a long span's rows in one product, which
 #: dequantises each weight once (1900 tokens after none, 12 layers: 11.7 ms in
 #: four spans of 512, 7.7 ms in one of 2048). More would only grow the
-#: activations: past 2048 rows the products gain nothing. The products keep
-#: the order of the 512-row spans' sums and the attention runs per 512 rows,
-#: so a prompt's bits do not depend on how its spans are run together (a stack
-#: of layers can blow a difference in one rounding up to a different row).
+#: activations: past 2048 rows the products gain nothing. Only for a model whose
+#: products then keep the order of the 512-row spans' sums
+#: (`SyntheticDualAR.merge_spans`; the benchmark's widths do), and with the
+#: attention 512 rows a launch: a prompt's bits do not depend on how its spans
+#: are run (a stack of layers can blow a difference in one rounding up to a
+#: different row).
 WIDE_SPANS = 4
 
 
-def _wide_spans(spans):
+def _wide_spans(spans, most: int | None = None):
     """`prefill_spans`' list with each run of largest-bucket spans merged, up to
-    `WIDE_SPANS` to one: the same padded positions in fewer spans."""
+    `most` (`WIDE_SPANS`) to one: the same padded positions in fewer spans."""
     top, out = PREFILL_BUCKETS[-1], []
+    most = WIDE_SPANS if most is None else most
     for off, size, b in spans:
-        if out and b == top and out[-1][2] % top == 0 and out[-1][2] < WIDE_SPANS * top:
+        if out and b == top and out[-1][2] % top == 0 and out[-1][2] < most * top:
             out[-1] = (out[-1][0], out[-1][1] + size, out[-1][2] + b)
         else:
             out.append((off, size, b))
     return out
 
 
-def prefill_sizes(max_len: int):
+def prefill_sizes(max_len: int, most: int | None = None):
     """The span lengths `SyntheticDualAR.prefill` replays graphs of, for a cache
-    of `max_len` positions: the buckets, and the runs of the largest one."""
+    of `max_len` positions: the buckets, and runs of up to `most`
+    (`WIDE_SPANS`) of the largest one."""
     top = PREFILL_BUCKETS[-1]
-    return [b for b in (*PREFILL_BUCKETS, *(top * i for i in range(2, WIDE_SPANS + 1))) if b <= max_len]
+    most = WIDE_SPANS if most is None else most
+    return [b for b in (*PREFILL_BUCKETS, *(top * i for i in range(2, most + 1))) if b <= max_len]
 
 
 SMALL = DualARConfig(dim=512, n_layer=3, n_head=4, n_local_heads=2, intermediate_size=1024,
@@ -317,6 +322,10 @@ class SyntheticDualAR:
                                   cfg.intermediate_size, cfg.max_seq_len, True)
         self.fast_layers = make_blocks("fast_layers", cfg.fast_n_layer, cfg.fast_dim, cfg.fast_n_head,
                                        cfg.fast_n_local_heads, cfg.fast_intermediate_size, cfg.fast_max_len, False)
+        # whether runs of largest-bucket spans keep their bits in one span
+        self.merge_spans = all(
+            fusedlayer.spans_keep_order(blk, nxt.attention_norm if nxt is not None else None)
+            for blk, nxt in zip(self.layers, [*self.layers[1:], None]))
         self.output = make_linear("output")
         self.fast_project_in = make_linear("fast_project_in")
         self.fast_output = make_linear("fast_output")
@@ -617,7 +626,7 @@ class SyntheticDualAR:
         import torch
 
         graphs = self.prefill_first_graphs if first else self.prefill_graphs
-        for b in buckets or prefill_sizes(self.cfg.max_seq_len):
+        for b in buckets or prefill_sizes(self.cfg.max_seq_len, None if self.merge_spans else 1):
             if b in graphs or b > self.cfg.max_seq_len:
                 continue
             width = b if first else None
@@ -639,7 +648,8 @@ class SyntheticDualAR:
 
     def prefill(self, tokens, start: int, graphed: bool = True) -> bool:
         """KV entries for `tokens` (n_tokens, n) int32 at [start, start + n),
-        in spans of the largest bucket (up to `WIDE_SPANS` of them run as one)
+        in spans of the largest bucket (with `merge_spans` up to `WIDE_SPANS` of
+        them run as one)
         and a last span padded to a bucket (the padding repeats the last real
         token; its KV entries land past the prompt, where decoding overwrites
         them before reading them); the last real position's token in `prefill_token`. False (nothing done) when
@@ -652,7 +662,7 @@ class SyntheticDualAR:
         spans = prefill_spans(n)
         if not spans or start + spans[-1][0] + spans[-1][2] > self.cfg.max_seq_len:
             return False
-        for off, size, b in _wide_spans(spans):
+        for off, size, b in _wide_spans(spans, None if self.merge_spans else 1):
             first = start + off == 0
             if graphed:
                 graphs = self.prefill_first_graphs if first else self.prefill_graphs

@@ -436,6 +436,34 @@ def prefill_block_chain(block, x, freqs_cis, mask, input_pos, *, xn=None, next_n
     return out, out_n
 
 
+def spans_keep_order(block, next_norm=None) -> bool:
+    """Whether `prefill_block_chain` gives 512-row spans the same bits run
+    together (`attend`: 512 rows a launch) as one by one: where the attention
+    kernel takes the heads and every product of 1024 to 2048 rows adds its K as
+    its 512-row form in the block does."""
+    from ttspipe_amd import nf4gemv
+
+    a, ff = block.attention, block.feed_forward
+    lib = _lib.lib()
+    if a.head_dim != HEAD_DIM or a.n_head // a.n_local_heads > lib.ttsp_prefill_max_groups():
+        return False
+
+    def keeps(linear, summed: bool, norm=None) -> bool:
+        # summed: the block adds the partial sums of ttsp_nf4_gemm_splits itself (with the next norm); else `matmul`
+        if not nf4gemv.prepare(linear):
+            return False
+        M, K = linear._nf4_fast["M"], linear._nf4_fast["K"]
+        if summed and norm is not None:
+            summed = M <= nf4gemv.NORM_MAX_M and M % 8 == 0 and norm.weight.data_ptr() % 16 == 0
+        parts = lib.ttsp_nf4_gemm_splits(M, K, 512)
+        if not summed or parts == 1:
+            parts = lib.ttsp_nf4_gemm_tile_splits(M, K, 512)
+        return lib.ttsp_nf4_gemm_span_splits(M, K) == parts
+
+    return (keeps(a.wqkv, True) and keeps(a.wo, True, block.ffn_norm) and keeps(ff.w1, False) and keeps(ff.w3, False)
+            and keeps(ff.w2, next_norm is not None, next_norm))
+
+
 def install() -> bool:
     """Patch `TransformerBlock.forward`: one-position calls go to `decode_block`,
     multi-position calls to `prefill_block`, anything either declines to the
