@@ -161,6 +161,8 @@ int ttsp_nf4_gemm_few(const void* X, int x_dtype, const uint8_t* W, const uint8_
  * work: 16-byte aligned, 2 * M * K bytes of dense weights, then (splits > 1)
  * splits * N * M fp32 partial sums. Other arguments as ttsp_nf4_gemm's. */
 int ttsp_nf4_gemm_dense_splits(int M, int K, int N);
+/* 1 where it serves the shape and is estimated faster than the tile kernel. Host-only. */
+int ttsp_nf4_gemm_dense_pays(int M, int K, int N);
 /* The K splits (ttsp_nf4_gemm_splits' or ttsp_nf4_gemm_tile_splits') of a
  * 512-row product whose bits ttsp_nf4_gemm_dense keeps at 1024, 1536 and 2048
  * rows; 0 where it keeps none. Host-only. */

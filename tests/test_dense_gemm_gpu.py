@@ -41,6 +41,47 @@ def test_dense_plan_covers_long_prompts_only():
             assert sp < 2 or M % 4 == 0
 
 
+def test_dense_form_only_where_it_pays():
+    """`ttsp_nf4_gemm_dense_pays`: large weights over many rows, not the small
+    ones whose tiles are faster (1024 x 3072 at 2048 rows 26 against 38 us), and
+    never where the form does not serve; below 1024 rows served means paying."""
+    from ttspipe_amd import _lib
+
+    pays = _lib.load().ttsp_nf4_gemm_dense_pays
+    for M, K, rows in ((9728, 2560, 1024), (9728, 2560, 2048), (6144, 2560, 2048), (2560, 9728, 2048), (2560, 9728, 800)):
+        assert pays(M, K, rows) == 1
+    for M, K, rows in ((1024, 3072, 1024), (1024, 3072, 2048), (1536, 2560, 1024), (2048, 2048, 1024), (3072, 1024, 1200),
+                       (9728, 2560, 600), (512, 512, 2048), (9728, 2560, 512)):
+        assert pays(M, K, rows) == 0
+    for M in (256, 1024, 1540, 4096, 9730):
+        for K in (512, 1024, 2560, 4096):
+            for rows in (513, 700, 1023, 1024, 1500, 3000):
+                sp = _plan(M, K, rows)
+                assert pays(M, K, rows) <= (sp > 0) and (rows >= 1024 or pays(M, K, rows) == (sp > 0))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1024, 1500])
+def test_matmul_takes_the_dense_form_where_it_pays(nf4, rows):
+    """A small weight's rows run the tiles unless the caller keeps the merged
+    spans' order (`wide`); both within the bar of each other's rounding."""
+    from ttspipe_amd import _lib
+
+    M, K = 1024, 3072
+    lib, lin = _lib.load(), to_linear(random_layer(M, K, True, seed=9), torch.bfloat16)
+    assert nf4.prepare(lin) and _plan(M, K, rows) and not lib.ttsp_nf4_gemm_dense_pays(M, K, rows)
+    x = from_bits(randn_bits(rows * K, torch.bfloat16, seed=3), torch.bfloat16).view(rows, K)
+    fast, out = lin._nf4_fast, torch.empty(rows, M, dtype=torch.bfloat16, device="cuda")
+    splits = lib.ttsp_nf4_gemm_tile_splits(M, K, rows)
+    work = torch.empty(splits * rows * M, device="cuda")
+    rc = lib.ttsp_nf4_gemm_split(x.data_ptr(), _lib.DT_BF16, fast["w"], fast["a8"], fast["amax"], fast["code2"],
+                                 fast["offset"], fast["lut"].data_ptr(), out.data_ptr(), 0, 0, M, K, rows, 64, 256,
+                                 work.data_ptr(), splits, _lib.stream())
+    assert rc == 0 and torch.equal(nf4.matmul(lin, x), out)
+    wide = nf4.matmul(lin, x, wide=True)
+    assert float((wide.float() - out.float()).norm() / out.float().norm()) < 2**-8
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("shape,rows,splits,nested,dtype,epi", [
     ((9728, 2560), 1025, 1, True, torch.bfloat16, 0),    # one activation row in the last tile
@@ -67,7 +108,8 @@ def test_dense_gemm_against_fp64(nf4, orc, shape, rows, splits, nested, dtype, e
     x = from_bits(xb, dtype).view(rows, K)
     rb = randn_bits(rows * M, dtype, seed=5)
     guard = torch.full((rows + 1, M), 7.0, dtype=dtype, device="cuda")
-    y = nf4.matmul(lin, x, epi=epi, operand=from_bits(rb, dtype).view(rows, M) if epi else None, out=guard[:rows])
+    y = nf4.matmul(lin, x, epi=epi, operand=from_bits(rb, dtype).view(rows, M) if epi else None, out=guard[:rows],
+                   wide=True)
     assert bool((guard[rows] == 7.0).all())
     sample = np.unique(np.r_[0:rows:61, rows - 1])
     ref = orc.nf4_gemm_ref(xb.reshape(rows, K)[sample], dt, **oracle_args(layer), M=M, K=K, N=sample.size, bs=64,

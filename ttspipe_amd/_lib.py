@@ -64,6 +64,7 @@ SIGNATURES: dict[str, list] = {
     "ttsp_nf4_gemm_few": [_vp, _i, _vp, _vp, _vp, _vp, _f, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _f, _vp,
                           _vp],
     "ttsp_nf4_gemm_dense_splits": [_i, _i, _i],
+    "ttsp_nf4_gemm_dense_pays": [_i, _i, _i],
     "ttsp_nf4_gemm_span_splits": [_i, _i],
     "ttsp_nf4_gemm_dense": [_vp, _i, _vp, _vp, _vp, _vp, _f, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp, _vp],
     "ttsp_nf4_gemm_dense_swiglu_fits": [_i, _i, _i],

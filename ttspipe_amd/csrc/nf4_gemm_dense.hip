@@ -480,18 +480,30 @@ static bool dense_fits(int M, int K, int N, int mats) {
 
 using namespace ttsp;
 
+// Whether the dense form is faster than the tile kernel by their estimates,
+// counting here the dequantisation's bytes at ~5.2 TB/s and its launch (us,
+// dense against tiles: 9728 x 2560 at 700 rows 50 / 43, at 1024 64 / 79, at
+// 2048 113 / 128; 2048 x 2560 at 1024 29.5 / 22.2, at 2048 35.7 / 35.9; 1024 x
+// 3072 at 2048 37.8 / 26.2). Over 48 weights of 1024 x 2048 to 9728 x 9728 at
+// 1024 to 2048 rows the estimates' choice was within 1 % of the faster form in
+// all but a few, and 8 % off at the worst.
+static bool dense_pays(int M, int K, int N) {
+  double us = 0.0;
+  dense_plan(M, K, N, &us);
+  return us + 3.0 + (double)M * K * 2.5 / 5.2e6 < tile_estimate(M, K, N);
+}
+
 // The K splits `ttsp_nf4_gemm_dense` takes a product in, 0 where it does not
-// serve it: small products, and below 1024 rows where the tile kernel's
-// estimate is lower, counting here the dequantisation's bytes at ~5.2 TB/s and
-// its launch (9728 x 2560 at 700 rows one round of tiles, 43 us against 50; at
-// 1024 two rounds, ~86 against 66; at 2048 114 against the 220 of the kernels
-// before both). From 1024 rows, a prompt's long spans, always: the order of
-// the sums is then the 512-row spans'.
+// serve it: small products, and below 1024 rows where it does not pay. From
+// 1024 rows a prompt's merged spans take it for its order of sums
+// (ttsp_nf4_gemm_span_splits), other callers where ttsp_nf4_gemm_dense_pays.
 extern "C" int ttsp_nf4_gemm_dense_splits(int M, int K, int N) {
   if (!dense_fits(M, K, N, 1) || (long long)M * K < (1ll << 21) || (double)M * K * N < 2.5e9) return 0;
-  double us = 0.0;
-  const DensePlan plan = dense_plan(M, K, N, &us);
-  return N >= 1024 || us + 3.0 + (double)M * K * 2.5 / 5.2e6 < tile_estimate(M, K, N) ? plan.splits : 0;
+  return N >= 1024 || dense_pays(M, K, N) ? dense_plan(M, K, N).splits : 0;
+}
+
+extern "C" int ttsp_nf4_gemm_dense_pays(int M, int K, int N) {
+  return ttsp_nf4_gemm_dense_splits(M, K, N) && dense_pays(M, K, N) ? 1 : 0;
 }
 
 // The K splits of a 512-row product whose bits the dense form keeps at every

@@ -319,6 +319,7 @@ def prefill_block_chain(block, x, freqs_cis, mask, input_pos, *, xn=None, next_n
     # a span of up to FUSED_MAX_ROWS rows takes the GEMV with each row's
     # RMSNorm folded in, as the decode step does: no norm launch runs
     fold = n <= nf4gemv.FUSED_MAX_ROWS
+    wide = attend is not None  # merged spans: the products keep their order of sums
     qkv = None
     if xn is None and fold:
         qkv = nf4gemv.matmul_fused(a.wqkv, x, norm_weight=an.weight, eps=an.eps)
@@ -336,9 +337,9 @@ def prefill_block_chain(block, x, freqs_cis, mask, input_pos, *, xn=None, next_n
     # rotary / KV kernel, which adds them as the split's own reduce would
     part = None
     if qkv is None and rows_ok and a.wqkv._nf4_fast["M"] == (nh + 2 * nkv) * hd:
-        part = nf4gemv.matmul_partials(a.wqkv, xn, span=True)
+        part = nf4gemv.matmul_partials(a.wqkv, xn, span=True, wide=wide)
     if part is None and qkv is None:
-        qkv = nf4gemv.matmul(a.wqkv, xn)
+        qkv = nf4gemv.matmul(a.wqkv, xn, wide=wide)
         if qkv is None:
             return None
     y = None
@@ -397,11 +398,11 @@ def prefill_block_chain(block, x, freqs_cis, mask, input_pos, *, xn=None, next_n
         if y is None:
             y = fastpath.decode_attention(q, k, v, mask, nh, nkv, hd)
         y = y.transpose(1, 2).contiguous().view(bsz, n, nh * hd)
-    hh = nf4gemv.matmul_norm(a.wo, y, fn.weight, fn.eps, epi=nf4gemv.EPI_RESIDUAL, operand=x, span=True)
+    hh = nf4gemv.matmul_norm(a.wo, y, fn.weight, fn.eps, epi=nf4gemv.EPI_RESIDUAL, operand=x, span=True, wide=wide)
     if hh is not None:
         h, hn = hh
     else:
-        h = nf4gemv.matmul(a.wo, y, epi=nf4gemv.EPI_RESIDUAL, operand=x)
+        h = nf4gemv.matmul(a.wo, y, epi=nf4gemv.EPI_RESIDUAL, operand=x, wide=wide)
         hn = None
     u = None
     if hh is None and fold and h is not None:  # w1 and w3 with the FFN norm folded in: one launch, else two
@@ -415,18 +416,18 @@ def prefill_block_chain(block, x, freqs_cis, mask, input_pos, *, xn=None, next_n
         hn = fusedops.rms_norm(h, fn.weight, fn.eps)
     # w1 and w3 with the SwiGLU gate in one launch where it serves the shape, else two
     if u is None and hn is not None:
-        u = nf4gemv.matmul_swiglu(ff.w1, ff.w3, hn)
+        u = nf4gemv.matmul_swiglu(ff.w1, ff.w3, hn, wide=wide)
     if u is None and hn is not None:
-        g = nf4gemv.matmul(ff.w1, hn)
-        u = None if g is None else nf4gemv.matmul(ff.w3, hn, epi=nf4gemv.EPI_SILU_GATE, operand=g)
+        g = nf4gemv.matmul(ff.w1, hn, wide=wide)
+        u = None if g is None else nf4gemv.matmul(ff.w3, hn, epi=nf4gemv.EPI_SILU_GATE, operand=g, wide=wide)
     oo = None
     if u is not None and next_norm is not None:
         oo = nf4gemv.matmul_norm(ff.w2, u, next_norm.weight, next_norm.eps, epi=nf4gemv.EPI_RESIDUAL, operand=h,
-                                 span=True)
+                                 span=True, wide=wide)
     if oo is not None:
         out, out_n = oo
     else:
-        out = None if u is None else nf4gemv.matmul(ff.w2, u, epi=nf4gemv.EPI_RESIDUAL, operand=h)
+        out = None if u is None else nf4gemv.matmul(ff.w2, u, epi=nf4gemv.EPI_RESIDUAL, operand=h, wide=wide)
         out_n = None
         if out is not None and next_norm is not None and not fold:  # (a short span's next block folds it)
             out_n = fusedops.rms_norm(out, next_norm.weight, next_norm.eps)

@@ -164,7 +164,7 @@ def prepare(module) -> bool:
     return True
 
 
-def matmul(module, x, *, epi: int = EPI_NONE, operand=None, out=None):
+def matmul(module, x, *, epi: int = EPI_NONE, operand=None, out=None, wide: bool = False):
     """Return x times the layer's weight transposed (fp16 or bf16 rows, any
     count), or None when the kernels cannot take this call.
 
@@ -206,7 +206,7 @@ def matmul(module, x, *, epi: int = EPI_NONE, operand=None, out=None):
     elif out.dtype != dtype or out.numel() != rows * M or not out.is_contiguous():
         return None
     lib = _lib.lib()
-    dense = lib.ttsp_nf4_gemm_dense_splits(M, K, rows) if rows >= DENSE_MIN_ROWS else 0
+    dense = _dense(M, K, rows, wide)
     few = lib.ttsp_nf4_gemm_few_splits(M, K, rows) if FEW_SPLIT_ROWS <= rows <= FEW_MAX_ROWS else 0
     splits = lib.ttsp_nf4_gemm_tile_splits(M, K, rows) if rows > 1 and not dense and not few else 1
     if few:
@@ -255,8 +255,14 @@ def _few(lib, fast, x, dt, rows, out, operand, epi, work, norm_weight=None, eps=
 DENSE_MIN_ROWS = 513
 
 
-def _dense(M: int, K: int, rows: int) -> bool:
-    return rows >= DENSE_MIN_ROWS and _lib.lib().ttsp_nf4_gemm_dense_splits(M, K, rows) > 0
+def _dense(M: int, K: int, rows: int, wide: bool) -> int:
+    """The dense form's K splits, 0 where the call does not take it. `wide` (a
+    prompt's merged spans): wherever it serves, for its order of sums, else
+    where it pays."""
+    if rows < DENSE_MIN_ROWS:
+        return 0
+    lib = _lib.lib()
+    return lib.ttsp_nf4_gemm_dense_splits(M, K, rows) if wide or lib.ttsp_nf4_gemm_dense_pays(M, K, rows) else 0
 
 
 #: Widest output row whose RMSNorm the split-K reduce folds in (eight 8-value
@@ -264,13 +270,13 @@ def _dense(M: int, K: int, rows: int) -> bool:
 NORM_MAX_M = 4096
 
 
-def matmul_partials(module, x, *, span: bool = False):
+def matmul_partials(module, x, *, span: bool = False, wide: bool = False):
     """`(work, splits)`: the K-split launch of `matmul(module, x)` without its
     reduce, work the fp32 partial sums [splits, rows, M] for a consumer that
     adds them in split order; None where the shape runs unsplit (or the
     kernels do not take the call). `span`, the prompt block's: split 9 to 32 rows
     too, whose `matmul` runs unsplit (it would pay a reduce launch; the
-    consumer does not)."""
+    consumer does not). `wide`: as `matmul`'s, which then takes the call."""
     import torch
 
     fast = getattr(module, "_nf4_fast", None)
@@ -283,7 +289,7 @@ def matmul_partials(module, x, *, span: bool = False):
     if x.shape[-1] != K or not x.is_contiguous() or x.data_ptr() % 16:
         return None
     rows = x.numel() // K
-    if rows < 2 or _dense(M, K, rows):
+    if rows < 2 or _dense(M, K, rows, wide):
         return None
     lib = _lib.lib()
     few = lib.ttsp_nf4_gemm_few_splits(M, K, rows) if span or FEW_SPLIT_ROWS <= rows <= FEW_MAX_ROWS else 0
@@ -303,7 +309,8 @@ def matmul_partials(module, x, *, span: bool = False):
     return work, splits
 
 
-def matmul_norm(module, x, norm_weight, eps: float, *, epi: int = EPI_NONE, operand=None, span: bool = False):
+def matmul_norm(module, x, norm_weight, eps: float, *, epi: int = EPI_NONE, operand=None, span: bool = False,
+                wide: bool = False):
     """`(y, rms_norm(y))` for several rows with the norm folded into the
     split-K reduce, or None where that form does not serve the call (one row,
     an unsplit shape, M over NORM_MAX_M); y is `matmul(module, x, epi=epi,
@@ -311,7 +318,8 @@ def matmul_norm(module, x, norm_weight, eps: float, *, epi: int = EPI_NONE, oper
     norm_weight, eps)`, both bit for bit. `span`, the prompt block's: 9 to 32
     rows too, whose `matmul` runs unsplit (y is then the sum of K splits, which
     the norm's launch adds), and from 65 rows `ttsp_nf4_gemm_splits`' splits,
-    whose order of sums longer spans keep."""
+    whose order of sums longer spans keep. `wide`: as `matmul`'s, which then
+    takes the call."""
     import torch
 
     fast = getattr(module, "_nf4_fast", None)
@@ -324,7 +332,7 @@ def matmul_norm(module, x, norm_weight, eps: float, *, epi: int = EPI_NONE, oper
     if x.shape[-1] != K or not x.is_contiguous() or x.data_ptr() % 16 or M % 8 or M > NORM_MAX_M:
         return None
     rows = x.numel() // K
-    if rows < 2 or _dense(M, K, rows):
+    if rows < 2 or _dense(M, K, rows, wide):
         return None
     if (norm_weight.dtype != x.dtype or norm_weight.numel() != M or not norm_weight.is_contiguous()
             or norm_weight.data_ptr() % 16 or norm_weight.device != x.device):
@@ -448,7 +456,7 @@ def matmul_fused(module, x, *, norm_weight=None, eps: float = 1e-6, module3=None
     return out.view(*x.shape[:-1], M) if given else out
 
 
-def matmul_swiglu(module1, module3, x, *, out=None):
+def matmul_swiglu(module1, module3, x, *, out=None, wide: bool = False):
     """silu(x W1^T) * (x W3^T) for several rows in one launch, rounded as the
     two-launch form `matmul(w3, x, epi=EPI_SILU_GATE, operand=matmul(w1, x))`
     and with its bits; None where one launch does not serve the shape (it
@@ -471,7 +479,7 @@ def matmul_swiglu(module1, module3, x, *, out=None):
         return None
     rows = x.numel() // K
     lib = _lib.lib()
-    dense = rows >= DENSE_MIN_ROWS and lib.ttsp_nf4_gemm_dense_swiglu_fits(M, K, rows)
+    dense = _dense(M, K, rows, wide) and lib.ttsp_nf4_gemm_dense_swiglu_fits(M, K, rows)
     if not dense and not lib.ttsp_nf4_gemm_swiglu_fits(M, K, rows, f1["bs"], f1["bs2"], int(f1["nested"])):
         return None
     if out is None:
