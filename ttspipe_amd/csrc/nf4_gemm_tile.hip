@@ -21,8 +21,12 @@
 //
 // Forms (bf16, nested, us, the kernels replaced against this):
 // * 64 rows a workgroup with both K halves (W 2, KG 2), where those tiles fit
-//   one to a CU: 9728 x 2560 at 100 rows 27.0 -> 20.0, 6144 x 2560 at 256
-//   26.6 -> 19.6, 2560 x 9728 at 100 (4 splits) 28.2 -> 24.
+//   one to a CU: 9728 x 2560 at 100 rows 27.0 -> 19.6, 6144 x 2560 at 256
+//   26.6 -> 19.1, 2560 x 9728 at 100 (4 splits) 28.2 -> 22.8. One copy of the
+//   code table: its few waves gain less from 16 copies than writing them costs
+//   (at 16 copies 19.8, 19.5 and 23.2; 1024 x 1024 at 256 rows, where a short K
+//   leaves the prologue most of the launch, 10.9 against 10.4, and in 2 splits
+//   slower than the kernel before).
 // * 256 rows (W 8) where at least half the CUs get one: one code table serves
 //   eight waves, so it can hold 32 copies (64 KB: a lookup's 64 lanes then
 //   touch every bank the minimum number of times), -5 % against one copy.
@@ -442,7 +446,7 @@ int tile_form(const void* X, const TileMat& a, const float* LUT, void* Y, const 
               int bs_shift, int bs2_shift, int splits, float* YP, hipStream_t st) {
   const long long nt = (long long)((N + BN - 1) / BN) * splits;
   if (tile_halves(M, N, splits))
-    return launch_tile<DT, 2, 2, 16, false>(X, a, a, LUT, Y, R, epi, M, K, N, bs_shift, bs2_shift, splits, YP, st);
+    return launch_tile<DT, 2, 2, 1, false>(X, a, a, LUT, Y, R, epi, M, K, N, bs_shift, bs2_shift, splits, YP, st);
   if ((M + 255) / 256 * nt >= 128)
     return launch_tile<DT, 8, 1, 32, false>(X, a, a, LUT, Y, R, epi, M, K, N, bs_shift, bs2_shift, splits, YP, st);
   return launch_tile<DT, 4, 1, 32, false>(X, a, a, LUT, Y, R, epi, M, K, N, bs_shift, bs2_shift, splits, YP, st);
