@@ -38,6 +38,24 @@ def test_few_row_split_plan():
     assert _splits(1 << 20, 1 << 14, 16) == 0  # byte offsets past 2^31
 
 
+def test_long_rows_are_split_at_17_to_32_rows():
+    """Past 10240 codes a product of 17 to 32 rows takes the plan's K splits
+    (and w1 / w3 two launches, which then split), up to there none."""
+    from ttspipe_amd import _lib
+
+    lib = _lib.load()
+    for M in (256, 1024, 2560):
+        for rows in (17, 24, 32):
+            for K in (2560, 9728, 10240):
+                assert lib.ttsp_nf4_gemm_splits(M, K, rows) == 1
+                assert lib.ttsp_nf4_gemm_swiglu_fits(M, K, rows, 64, 256, 1) == 1
+            for K in (10368, 16384, 40960):
+                sp = lib.ttsp_nf4_gemm_splits(M, K, rows)
+                assert sp == lib.ttsp_nf4_gemm_tile_splits(M, K, rows) and K % (128 * sp) == 0
+                assert sp > 1 or K % 256  # (10368 = 81 x 128: no even split)
+                assert lib.ttsp_nf4_gemm_swiglu_fits(M, K, rows, 64, 256, 1) == 0
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("shape,rows,nested,bs,bs2,dtype", [
     ((9728, 2560), 9, True, 64, 256, torch.bfloat16),     # the fewest rows: 7 of 16 loaded rows repeat
@@ -48,7 +66,10 @@ def test_few_row_split_plan():
     ((1022, 4096), 64, False, 256, 0, torch.float16),     # a split with M % 4 == 2
     ((33, 128), 24, True, 64, 256, torch.bfloat16),       # two K-steps for four waves; a tile with one row
     ((64, 384), 40, True, 128, 32, torch.float16),        # six K-steps over four waves
-    ((96, 16384), 20, True, 64, 256, torch.bfloat16),     # 64 steps a wave
+    ((96, 16384), 20, True, 64, 256, torch.bfloat16),     # eight splits by the plan
+    ((96, 10240), 32, True, 64, 256, torch.float16),      # the longest unsplit row: 40 steps a wave
+    ((70, 24576), 17, False, 128, 0, torch.bfloat16),     # eight splits, M % 4 == 2
+    ((64, 10368), 31, True, 64, 256, torch.bfloat16),     # past it, no even split: unsplit
 ])
 def test_few_rows_against_fp64(nf4, orc, shape, rows, nested, bs, bs2, dtype):
     """`matmul` and, where it splits, `matmul_partials` and `matmul_norm`:

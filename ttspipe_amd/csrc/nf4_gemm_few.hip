@@ -346,6 +346,9 @@ int few_rows(const void* X, const FewMat& a, const FewMat& b, const float* LUT, 
 }  // namespace
 
 constexpr int FEW_MIN_N = 9, FEW_MAX_N = 64, FEW_PAIR_MAX_N = 32;
+// The longest row of an unsplit product of 17 to 32 rows; longer ones take the
+// plan's K splits.
+constexpr int FEW_UNSPLIT_MAX_K = 10240;
 
 // Whether the kernel takes the shape: byte offsets of X and W and the scale
 // indices below 2^31.
@@ -354,12 +357,16 @@ bool few_takes(int M, int K, int N) {
   return (long long)N * K * 2 < (1ll << 31) && (long long)M * K / 2 < (1ll << 31);
 }
 
-// Whether an unsplit product of N rows runs here: from 17 rows always; at 9 to
+// Whether an unsplit product of N rows runs here: from 17 rows always, but at
+// 17 to 32 of a longer K than FEW_UNSPLIT_MAX_K, whose four waves a workgroup
+// would each add a long run (256 x 40960 at 32 rows 57.9 us, 20.3 in 4 splits;
+// 1024 x 16384 25.7 and 12.9; at 2560 x 4096 the two are within 0.6 us); at 9 to
 // 16 the skinny kernel's 16-row tiles make more workgroups of a small matrix
 // (2560 x 4096 at 16 rows 7.7 against 8.3 us here, 1024 x 3072 6.5 against
 // 6.6; 9728 x 2560 12.7 against 9.4, 6144 x 2560 9.4 against 6.5).
 bool few_unsplit(int M, int K, int N) {
-  return few_takes(M, K, N) && (N > 16 || ((M + 31) / 32 >= 192 && K <= 4096));
+  if (!few_takes(M, K, N)) return false;
+  return N > 16 ? N > 32 || K <= FEW_UNSPLIT_MAX_K : (M + 31) / 32 >= 192 && K <= 4096;
 }
 
 // K splits where the sums' reduce costs nothing extra (it also writes the next
