@@ -123,6 +123,13 @@ def test_sampler_row_lengths(V):
     assert checked >= 4
 
 
+@pytest.mark.parametrize("V", [2, 256, 511, 512, 513, 4096, 4097, 8192, 8193, 16384, 16385])
+def test_sampler_at_the_edges_of_its_register_counts(V):
+    """The rows at which a thread's key registers change (2, 16, 32, 64, 128 of
+    them), one entry to either side, against the oracle."""
+    test_sampler_row_lengths(V)
+
+
 def test_sampler_declines_rows_longer_than_it_holds():
     from ttspipe_amd import fusedsample
 

@@ -34,7 +34,7 @@
 //      a butterfly over (score, index) picks the draw.
 // Bound by the serial chain of these steps. With the keys in LDS (read again
 // in each of the 16 rounds, and by index for the candidates) a 4096-entry row
-// took 38 us; now 12.
+// took 38 us; now 12 (500 entries 11.3 -> 7.4, 8193 70.5 -> 30.9, 32768 264 -> 82).
 #include "ttsp_common.h"
 
 namespace ttsp {
@@ -64,7 +64,9 @@ __device__ __forceinline__ T wave_scan(T v, int lane) {
   return v;
 }
 
-// SL: key registers a thread (V <= 256 SL).
+// SL: key registers a thread (V <= 256 SL). A register past the row costs its
+// share of every count, so there are five: 64 entries took 9.2 us with 16 and
+// take 6.3 with 2 (7.6 before), 8193 took 71.4 with 128 and take 29.5 with 64.
 template <int DT, int SL>
 __global__ __launch_bounds__(SMP_THREADS) void sample_topk_kernel(const uint16_t* __restrict__ L, int V,
                                                                   const uint16_t* __restrict__ TEMP,
@@ -136,14 +138,17 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_topk_kernel(const uint16_t
   __syncthreads();
   if (wave < 2) {  // one wave a list: lane l sums its NC / 64 entries
     int* const list = wave ? ceq : cgt;
-    constexpr int PER = NC / 64;
+    constexpr int PER = NC > 64 ? NC / 64 : 1;
     int v[PER], s = 0;
 #pragma unroll
-    for (int e = 0; e < PER; ++e) v[e] = list[lane * PER + e], s += v[e];
+    for (int e = 0; e < PER; ++e) v[e] = NC >= 64 || lane < NC ? list[lane * PER + e] : 0, s += v[e];
     const int inc = wave_scan(s, lane);
     int at = inc - s;
 #pragma unroll
-    for (int e = 0; e < PER; ++e) list[lane * PER + e] = at, at += v[e];
+    for (int e = 0; e < PER; ++e) {
+      if (NC >= 64 || lane < NC) list[lane * PER + e] = at;
+      at += v[e];
+    }
     if (wave == 0 && lane == 63) total_s = inc;
   }
   __syncthreads();
@@ -167,13 +172,13 @@ __global__ __launch_bounds__(SMP_THREADS) void sample_topk_kernel(const uint16_t
   __syncthreads();
   if (wave != 0) return;
 
-  // 4. rank counting (one wave from here on)
+  // 4. rank counting (one wave from here on): key and index in one word, which
+  // is larger for the larger key or the lower index (V <= 2^15)
   const int me = lane < k ? cand[lane] : 0, mk = lane < k ? candk[lane] : 0;
+  const uint32_t word = ((uint32_t)mk << 16) | (0xffffu - (uint32_t)me);
   int rank = 0;
-  for (int j = 0; j < k; ++j) {
-    const int o = __builtin_amdgcn_readlane(me, j), ok = __builtin_amdgcn_readlane(mk, j);
-    rank += ok > mk || (ok == mk && o < me);
-  }
+#pragma unroll 4
+  for (int j = 0; j < k; ++j) rank += (uint32_t)__builtin_amdgcn_readlane((int)word, j) > word;
   __builtin_amdgcn_wave_barrier();
   if (lane < k) cand[rank] = me, candk[rank] = mk;
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -212,8 +217,10 @@ void launch_sample(const uint16_t* L, int V, const uint16_t* TEMP, const uint16_
                    const float* U, int* OUT, hipStream_t st) {
 #define TTSP_SMP(SLV) \
   hipLaunchKernelGGL((sample_topk_kernel<DT, SLV>), dim3(1), dim3(SMP_THREADS), 0, st, L, V, TEMP, TOPP, TOPK, U, OUT)
-  if (V <= 16 * SMP_THREADS) TTSP_SMP(16);
+  if (V <= 2 * SMP_THREADS) TTSP_SMP(2);
+  else if (V <= 16 * SMP_THREADS) TTSP_SMP(16);
   else if (V <= 32 * SMP_THREADS) TTSP_SMP(32);
+  else if (V <= 64 * SMP_THREADS) TTSP_SMP(64);
   else TTSP_SMP(128);
 #undef TTSP_SMP
 }
