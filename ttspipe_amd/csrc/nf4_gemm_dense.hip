@@ -290,6 +290,8 @@ __global__ __launch_bounds__(64 * C::NW) void nf4_gemm_dense_kernel(
   constexpr int CPR = C::TM * (SW ? 2 : 4);  // 16-byte output chunks of a row
 #pragma unroll
   for (int b = 0; b < C::TN; ++b) {
+    // the block's rows are written and read by different lanes of the wave
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
     for (int a = 0; a < C::TM; ++a)
 #pragma unroll
@@ -297,6 +299,7 @@ __global__ __launch_bounds__(64 * C::NW) void nf4_gemm_dense_kernel(
         *reinterpret_cast<uint2*>(stg + (lane & 31) * PITCH + a * 64 + g * 16 + (lane >> 5) * 8) =
             make_uint2(pack2<DT>(acc[a][b][4 * g], acc[a][b][4 * g + 1]),
                        pack2<DT>(acc[a][b][4 * g + 2], acc[a][b][4 * g + 3]));
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll 1
     for (int e = lane; e < 32 * CPR; e += 64) {
       const int nl = e / CPR, ch = e % CPR;
