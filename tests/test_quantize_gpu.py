@@ -72,3 +72,20 @@ def test_quantize_forms_the_kernel_leaves_to_torch():
         assert quant._kernel_serves(p, p.view(-1), 64)
     a, b = quant.quantize_4bit(w[2:2050], 64), quant.quantize_4bit(w[2:2050].clone(), 64)  # misaligned, aligned
     assert torch.equal(a[0], b[0]) and torch.equal(a[1].absmax, b[1].absmax)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nested", [True, False])
+def test_quantize_without_the_library_runs_the_torch_steps(monkeypatch, tmp_path, nested):
+    """A weight on the GPU is quantised to the same bytes where the library is
+    not built (or not shipped)."""
+    from ttspipe_amd import _lib
+
+    w = torch.randn(64, 128, generator=torch.Generator(device="cuda").manual_seed(3), device="cuda").bfloat16()
+    packed, state = quant.quantize_4bit(w, 64, compress_statistics=nested)
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib, "LIB_PATH", tmp_path / "libttsp_hip.so")
+    packed_t, state_t = quant.quantize_4bit(w, 64, compress_statistics=nested)
+    assert torch.equal(packed, packed_t)
+    _same(state.absmax, state_t.absmax)
+    _same(state.offset, state_t.offset)

@@ -146,6 +146,11 @@ def lib() -> ctypes.CDLL:
     return load()
 
 
+def built() -> bool:
+    """Whether the library is there to load (for calls that have another way)."""
+    return _lib is not None or LIB_PATH.exists()
+
+
 _gpu = False  # a GPU was seen (one that is there stays)
 
 

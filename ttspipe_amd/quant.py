@@ -154,12 +154,15 @@ def _constant(name: str, device):
 def _kernel_serves(A, flat, blocksize: int) -> bool:
     """Whether the quantisation kernel takes this weight: plain fp16 / bf16 /
     fp32 values on the current GPU, blocks of 64 to 512 (8 to 64 lanes of a
-    wave), nothing that follows the operations (gradients, wrapped tensors)."""
+    wave), nothing that follows the operations (gradients, wrapped tensors).
+    Loading a model needs no kernel: without the library torch's steps run."""
+    from ttspipe_amd import _lib
+
     return (A.device.type == "cuda" and type(A) in (torch.Tensor, torch.nn.Parameter) and 64 <= blocksize <= 512
             and A.dtype in (torch.float16, torch.bfloat16, torch.float32) and flat.numel() > 0
             and not (A.requires_grad and torch.is_grad_enabled())
             and not torch._C._functorch.is_functorch_wrapped_tensor(A)
-            and A.device.index == torch.cuda.current_device() and flat.data_ptr() % 16 == 0)
+            and A.device.index == torch.cuda.current_device() and flat.data_ptr() % 16 == 0 and _lib.built())
 
 
 def _quantize_4bit_kernel(A, flat, blocksize: int, compress_statistics: bool):
