@@ -89,3 +89,41 @@ def test_quantize_without_the_library_runs_the_torch_steps(monkeypatch, tmp_path
     assert torch.equal(packed, packed_t)
     _same(state.absmax, state_t.absmax)
     _same(state.offset, state_t.offset)
+
+
+@pytest.mark.gpu
+def test_quantize_reads_a_lazily_negated_weight_as_its_values():
+    w = torch.randn(64, 128, generator=torch.Generator(device="cuda").manual_seed(5), device="cuda")
+    lazy = torch._neg_view(w)
+    assert lazy.is_neg() and lazy.data_ptr() == w.data_ptr()
+    packed, state = quant.quantize_4bit(lazy)
+    packed_n, state_n = quant.quantize_4bit((-w).contiguous())
+    assert torch.equal(packed, packed_n)
+    _same(state.absmax, state_n.absmax)
+
+
+@pytest.mark.gpu
+def test_quantize_steps_are_seen_by_modes_and_tangents():
+    """Under a dispatch mode every step goes through it, and a forward-mode
+    tangent reaches the scales: the torch steps run, with the same bytes."""
+    from torch.autograd import forward_ad
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Names(TorchDispatchMode):
+        seen: list = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    w = torch.randn(64, 128, generator=torch.Generator(device="cuda").manual_seed(7), device="cuda")
+    packed, state = quant.quantize_4bit(w)
+    with Names() as names:
+        packed_m, state_m = quant.quantize_4bit(w)
+    assert any("bucketize" in s for s in names.seen)
+    assert torch.equal(packed, packed_m) and torch.equal(state.absmax, state_m.absmax)
+    with forward_ad.dual_level():
+        packed_d, state_d = quant.quantize_4bit(forward_ad.make_dual(w, torch.ones_like(w)))
+        absmax, tangent = forward_ad.unpack_dual(state_d.absmax)
+        assert torch.equal(packed, packed_d) and torch.equal(state.absmax, absmax)
+        assert torch.equal(tangent, w.view(-1, 64).gather(1, w.view(-1, 64).abs().argmax(1, keepdim=True))[:, 0].sign())

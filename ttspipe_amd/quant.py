@@ -146,22 +146,28 @@ def _constant(name: str, device):
     key = (name, device)
     t = _constants.get(key)
     if t is None:
-        t = torch.tensor(NF4_CODE, dtype=torch.float32) if name == "nf4" else create_dynamic_map()
+        t = torch.tensor(NF4_CODE, dtype=torch.float32, device="cpu") if name == "nf4" else create_dynamic_map()
         t = _constants[key] = t.to(device)
     return t.clone()
+
+
+def _ops_are_followed() -> bool:
+    return (torch.autograd.forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack() > 0
+            or torch.compiler.is_compiling() or torch.jit.is_tracing())
 
 
 def _kernel_serves(A, flat, blocksize: int) -> bool:
     """Whether the quantisation kernel takes this weight: plain fp16 / bf16 /
     fp32 values on the current GPU, blocks of 64 to 512 (8 to 64 lanes of a
-    wave), nothing that follows the operations (gradients, wrapped tensors).
-    Loading a model needs no kernel: without the library torch's steps run."""
+    wave), held in memory as they are (no lazy negation, no zero tensor without
+    storage), and nothing that follows the operations (gradients, forward-mode
+    tangents, wrapped tensors, dispatch modes, tracing). Loading a model needs no kernel: without the library torch's steps run."""
     from ttspipe_amd import _lib
 
-    return (A.device.type == "cuda" and type(A) in (torch.Tensor, torch.nn.Parameter) and 64 <= blocksize <= 512
+    return (A.device.type == "cuda" and not _ops_are_followed() and type(A) in (torch.Tensor, torch.nn.Parameter) and 64 <= blocksize <= 512
             and A.dtype in (torch.float16, torch.bfloat16, torch.float32) and flat.numel() > 0
             and not (A.requires_grad and torch.is_grad_enabled())
-            and not torch._C._functorch.is_functorch_wrapped_tensor(A)
+            and not torch._C._functorch.is_functorch_wrapped_tensor(A) and not A.is_neg() and not A._is_zerotensor()
             and A.device.index == torch.cuda.current_device() and flat.data_ptr() % 16 == 0 and _lib.built())
 
 
