@@ -435,6 +435,22 @@ def test_swiglu_gemm_plan_on_the_host():
                                     None) == 1  # one weight nested, the other plain
 
 
+@pytest.mark.parametrize("N,K", [(3, 2560), (12, 2560), (24, 2560), (24, 20480), (48, 2560), (100, 2560), (512, 2560),
+                                 (1200, 2560), (1, 40960)])
+def test_misaligned_matrices_are_refused(N, K):
+    """Every product kernel but the GEMV loads X and W 16 bytes at a time: an
+    address off that boundary is hipErrorInvalidValue before any launch (the
+    addresses here are never read)."""
+    from ttspipe_amd import _lib
+
+    lib, p = _lib.load(), 1 << 20
+    for x, w in ((p + 2, p), (p + 8, p), (p, p + 4)):
+        assert lib.ttsp_nf4_gemm(x, 1, w, p, p, p, 0.0, p, p, None, 0, 1024, K, N, 64, 256, None) == 1
+        sp = lib.ttsp_nf4_gemm_splits(1024, K, N)
+        if N > 1 and sp > 1:
+            assert lib.ttsp_nf4_gemm_split(x, 1, w, p, p, p, 0.0, p, p, None, 0, 1024, K, N, 64, 256, p, sp, None) == 1
+
+
 def test_span_splits_name_the_products_that_keep_the_512_row_order():
     """`ttsp_nf4_gemm_span_splits`: the 512-row splits of the model's layer; none
     where the 512-row launch adds its K in halves (few 64 x 128 tiles) or the

@@ -241,7 +241,7 @@ int gemm_mfma(const void* X, int dt, const uint8_t* W, const uint8_t* A8, const 
               int bs2_shift, int splits, float* YP, hipStream_t st, bool reduce = true) {
   if (K % (2 * KT)) return (int)hipErrorInvalidValue;
   if (splits > 1 && (!YP || (K / KT) % (2 * splits))) return (int)hipErrorInvalidValue;
-  const bool few = few_takes(M, K, N) && (uintptr_t)X % 16 == 0 && (uintptr_t)W % 16 == 0;
+  const bool few = few_takes(M, K, N);
   if (int rc = few ? gemm_few(X, dt, W, A8, AMAX, CODE2, offset, LUT, Y, R, epi, M, K, N, bs_shift, bs2_shift, splits,
                               YP, st)
                    : gemm_tile(X, dt, W, A8, AMAX, CODE2, offset, LUT, Y, R, epi, M, K, N, bs_shift, bs2_shift, splits,
@@ -330,7 +330,7 @@ extern "C" int ttsp_nf4_gemm(const void* X, int x_dtype, const uint8_t* W, const
                          &bs2_shift))
     return rc;
   // (one row whose K the GEMV cannot hold, K > 32768, takes the tiled kernel below)
-  if (few_unsplit(M, K, N) && (uintptr_t)X % 16 == 0 && (uintptr_t)W % 16 == 0)
+  if (few_unsplit(M, K, N))
     return gemm_few(X, x_dtype, W, A8, AMAX, CODE2, offset, LUT, Y, R, epi, M, K, N, bs_shift, bs2_shift, 1, nullptr,
                     stream);
   if (N >= 2 && skinny(K, N))

@@ -467,6 +467,7 @@ int gemm_tile(const void* X, int dt, const uint8_t* W, const uint8_t* A8, const 
               float offset, const float* LUT, void* Y, const void* R, int epi, int M, int K, int N, int bs_shift,
               int bs2_shift, int splits, float* YP, hipStream_t st) {
   if (splits < 1 || K % (2 * KT * splits) || (splits > 1 && !YP)) return (int)hipErrorInvalidValue;
+  if ((uintptr_t)X % 16 || (uintptr_t)W % 16) return (int)hipErrorInvalidValue;  // 16-byte loads to LDS
   const TileMat a{W, A8, AMAX, CODE2, offset};
   const bool al16 = (uintptr_t)Y % 16 == 0 && (!(epi & 3) || (uintptr_t)R % 16 == 0);
   const int e = (epi & 3) | (al16 ? 8 : 0);
@@ -483,6 +484,7 @@ int gemm_tile_swiglu(const void* X, int dt, const uint8_t* W1, const uint8_t* A8
                      const float* CODE2_1, float offset_1, const uint8_t* W3, const uint8_t* A8_3, const float* AMAX_3,
                      const float* CODE2_3, float offset_3, const float* LUT, void* Y, int M, int K, int N, int bs_shift,
                      int bs2_shift, hipStream_t st) {
+  if ((uintptr_t)X % 16 || (uintptr_t)W1 % 16 || (uintptr_t)W3 % 16) return (int)hipErrorInvalidValue;
   const TileMat a{W1, A8_1, AMAX_1, CODE2_1, offset_1}, b{W3, A8_3, AMAX_3, CODE2_3, offset_3};
   const int e = (uintptr_t)Y % 16 == 0 ? 8 : 0;
   if (dt == DT_BF16)
