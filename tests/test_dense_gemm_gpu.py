@@ -83,6 +83,32 @@ def test_matmul_takes_the_dense_form_where_it_pays(nf4, rows):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,K,rows", [(9728, 2560, 1100), (2560, 9728, 1100)])
+def test_without_room_for_the_workspace_the_tiles_run(nf4, monkeypatch, M, K, rows):
+    """A product whose dequantised weight does not fit the memory left runs the
+    kernels that read the codes in place (the pair as two launches): within the
+    roundings of the dense form, through the same calls."""
+    lin, lin3 = (to_linear(random_layer(M, K, True, seed=s), torch.bfloat16) for s in (1, 2))
+    assert nf4.prepare(lin) and nf4.prepare(lin3) and _plan(M, K, rows)
+    x = from_bits(randn_bits(rows * K, torch.bfloat16, seed=3), torch.bfloat16).view(rows, K)
+    dense, pair = nf4.matmul(lin, x), nf4.matmul_swiglu(lin, lin3, x)
+    empty = torch.empty
+
+    def limited(*size, **kw):
+        if kw.get("dtype") is torch.uint8:
+            raise torch.OutOfMemoryError("no room")
+        return empty(*size, **kw)
+
+    monkeypatch.setattr(torch, "empty", limited)
+    tiles = nf4.matmul(lin, x)
+    assert float((tiles.float() - dense.float()).norm() / dense.float().norm()) < 2**-8
+    assert nf4.matmul_swiglu(lin, lin3, x) is None
+    if pair is not None:
+        two = nf4.matmul(lin3, x, epi=nf4.EPI_SILU_GATE, operand=tiles)
+        assert float((two.float() - pair.float()).norm() / pair.float().norm()) < 2**-7
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("shape,rows,splits,nested,dtype,epi", [
     ((9728, 2560), 1025, 1, True, torch.bfloat16, 0),    # one activation row in the last tile
     ((9730, 2560), 900, 1, False, torch.float16, 0),     # M % 4 == 2: element-wise stores

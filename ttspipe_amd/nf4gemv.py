@@ -207,14 +207,16 @@ def matmul(module, x, *, epi: int = EPI_NONE, operand=None, out=None, wide: bool
         return None
     lib = _lib.lib()
     dense = _dense(M, K, rows, wide)
+    if dense:
+        # the dequantised weight, then (K split) the partial sums
+        work = _dense_work(2 * M * K + (4 * dense * rows * M if dense > 1 else 0), device)
+        dense = dense if work is not None else 0
     few = lib.ttsp_nf4_gemm_few_splits(M, K, rows) if FEW_SPLIT_ROWS <= rows <= FEW_MAX_ROWS else 0
     splits = lib.ttsp_nf4_gemm_tile_splits(M, K, rows) if rows > 1 and not dense and not few else 1
     if few:
         work = torch.empty(few * rows * M, dtype=torch.float32, device=device) if few > 1 else None
         rc = _few(lib, fast, flat, dt, rows, out, operand, epi, work)
     elif dense:
-        # the dequantised weight, then (K split) the partial sums
-        work = torch.empty(2 * M * K + (4 * dense * rows * M if dense > 1 else 0), dtype=torch.uint8, device=device)
         rc = lib.ttsp_nf4_gemm_dense(
             flat.data_ptr(), dt, fast["w"], fast["a8"], fast["amax"], fast["code2"], fast["offset"],
             fast["lut"].data_ptr(), out.data_ptr(), _lib.ptr(operand) if epi else 0, epi, M, K, rows,
@@ -253,6 +255,17 @@ def _few(lib, fast, x, dt, rows, out, operand, epi, work, norm_weight=None, eps=
 #: From this many rows `matmul` and `matmul_swiglu` ask for the dense form (the weight dequantised once a call into a
 #: workspace): below it the kernels that read the codes in place are faster.
 DENSE_MIN_ROWS = 513
+
+
+def _dense_work(nbytes: int, device):
+    """The dense form's workspace, or None where it does not fit the GPU's memory
+    beside what is there: the call then takes the kernels that need none."""
+    import torch
+
+    try:
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        return None
 
 
 def _dense(M: int, K: int, rows: int, wide: bool) -> int:
@@ -480,6 +493,9 @@ def matmul_swiglu(module1, module3, x, *, out=None, wide: bool = False):
     rows = x.numel() // K
     lib = _lib.lib()
     dense = _dense(M, K, rows, wide) and lib.ttsp_nf4_gemm_dense_swiglu_fits(M, K, rows)
+    if dense:
+        work = _dense_work(4 * M * K, x.device)  # both dequantised weights
+        dense = work is not None
     if not dense and not lib.ttsp_nf4_gemm_swiglu_fits(M, K, rows, f1["bs"], f1["bs2"], int(f1["nested"])):
         return None
     if out is None:
@@ -490,7 +506,6 @@ def matmul_swiglu(module1, module3, x, *, out=None, wide: bool = False):
             f3["w"], f3["a8"], f3["amax"], f3["code2"], f3["offset"], f1["lut"].data_ptr(), out.data_ptr(),
             M, K, rows, f1["bs"], f1["bs2"])
     if dense:
-        work = torch.empty(4 * M * K, dtype=torch.uint8, device=x.device)  # both dequantised weights
         rc = lib.ttsp_nf4_gemm_dense_swiglu(*args, work.data_ptr(), _lib.stream())
     else:
         rc = lib.ttsp_nf4_gemm_swiglu(*args, _lib.stream())
