@@ -844,17 +844,24 @@ def test_spans_merge_only_where_that_keeps_their_bits(two_layers, monkeypatch):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("start,n", [(0, 1900), (0, 1000), (0, 1500), (700, 1024)])
+@pytest.mark.parametrize("start,n", [(0, 1900), (0, 1000), (0, 1500), (700, 1024), (100, 1900)])
 def test_wide_spans_keep_the_bits_of_narrow_ones(two_layers, monkeypatch, start, n):
     """At the model's widths a prompt's KV rows and logits are the same bits
-    whether its 512-row spans run one by one or 2, 3 or 4 together."""
+    whether its 512-row spans run one by one or 2, 3 or 4 together (the last one
+    whole or padded). Each run finds other values in the cache rows from its
+    start on, so a row it skips, or reads before it is written, differs."""
     from ttspipe_amd import dualar
 
     m = two_layers
     toks = _tokens(m, n, 3 + n)
+    initial = _kv_state(m, m.cfg.max_seq_len)
     got = []
-    for wide in (1, 4):
+    for wide, stale in ((1, 900.0), (4, -700.0)):
         monkeypatch.setattr(dualar, "WIDE_SPANS", wide)
+        _set_kv(m, initial)
+        for blk in m.layers:
+            blk.attention.kv_cache.k_cache[:, :, start:] = stale
+            blk.attention.kv_cache.v_cache[:, :, start:] = stale
         assert m.prefill(toks, start, graphed=False)
         torch.cuda.synchronize()
         got.append((_kv_state(m, start + n), m.logits.clone()))
@@ -862,3 +869,4 @@ def test_wide_spans_keep_the_bits_of_narrow_ones(two_layers, monkeypatch, start,
     for i, ((ka, va), (kb, vb)) in enumerate(zip(kva, kvb)):
         assert torch.equal(ka, kb) and torch.equal(va, vb), f"layer {i}"
     assert torch.equal(la, lb)
+    _set_kv(m, initial)
