@@ -53,6 +53,22 @@ def gemv_rows_shape(M: int, K: int, N: int):
     return (J.value, KS.value, RPW.value) if rc == 0 else None
 
 
+def split_product(lin, x, splits: int, epi: int = 0, operand=None):
+    """`ttsp_nf4_gemm_split` of a prepared layer in `splits` K splits (a count
+    the entry takes for these rows), whatever count `nf4gemv.matmul` would ask for."""
+    from ttspipe_amd import _lib
+
+    f, rows = lin._nf4_fast, x.numel() // lin._nf4_fast["K"]
+    y = torch.empty(rows, f["M"], dtype=x.dtype, device=x.device)
+    work = torch.empty(splits * rows * f["M"], device=x.device)
+    rc = _lib.load().ttsp_nf4_gemm_split(
+        x.data_ptr(), _lib.dtype_code(x.dtype), f["w"], f["a8"], f["amax"], f["code2"], f["offset"],
+        f["lut"].data_ptr(), y.data_ptr(), _lib.ptr(operand), epi, f["M"], f["K"], rows, f["bs"], f["bs2"],
+        work.data_ptr(), splits, _lib.stream())
+    assert rc == 0, f"ttsp_nf4_gemm_split in {splits}: {rc}"
+    return y
+
+
 def first_mismatch(a: np.ndarray, b: np.ndarray) -> str:
     idx = np.flatnonzero(a != b)
     if idx.size == 0:

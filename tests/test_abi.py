@@ -74,8 +74,8 @@ def test_gemv_shape_covers_every_row_and_column(M, K):
     assert J * KS * 64 >= K // 8 and (J - 1) * KS * 64 < K // 8  # no wholly idle chunk slot
 
 
-def _dl_split(M, K, N):
-    """The direct-to-LDS kernel's split for 256 to 512 rows, or None: 4 where K
+def _span_split(M, K, N):
+    """The plan's split by its rule for large shapes of 256 to 512 rows, or None: 4 where K
     has 64 or more steps and there are at least 75 64 x 128 tiles; with fewer
     steps none from 512 tiles and 2 from 300."""
     steps, t = K // 64, -(-M // 64) * -(-N // 128)
@@ -97,8 +97,8 @@ def test_gemm_split_plan(M, K, N):
     """The K split a prefill GEMM takes (host-only query): none for N <= 32 or
     when the 64 x 128 output tiles already fill the GPU; otherwise each split
     covers an even number of at least 8 K-steps of 64 codes. 33 to 64 rows:
-    4 splits where that allows, else 2. 256 to 512 rows where the
-    direct-to-LDS kernel takes the launch: its split. More rows otherwise: up
+    4 splits where that allows, else 2. Large shapes of 256 to 512 rows: 4, 2
+    or none by K and tiles. More rows otherwise: up
     to 128 tiles the largest such split whose workgroups fit one to a CU;
     between 128 and 256 tiles, 4 splits when each keeps more than 16 K-steps."""
     from ttspipe_amd import _lib
@@ -110,9 +110,9 @@ def test_gemm_split_plan(M, K, N):
     t = -(-M // 64) * -(-N // 128)
     if sp > 1:
         assert steps % (2 * sp) == 0 and steps // sp >= 8
-    dl = _dl_split(M, K, N) if N > 64 else None
-    if dl is not None:
-        assert sp == dl
+    span = _span_split(M, K, N) if N > 64 else None
+    if span is not None:
+        assert sp == span
         return
     if N <= 32 or t >= 256:
         assert sp == 1
@@ -406,9 +406,9 @@ def test_fast_steps_rejects_bad_arguments_before_any_launch():
 
 def test_swiglu_gemm_plan_on_the_host():
     """`ttsp_nf4_gemm_swiglu_fits`: one launch where both GEMMs of the pair
-    would run the direct-to-LDS kernel unsplit (up to 512 rows, >= 512 tiles
+    would run the tile kernel unsplit (256 to 512 rows, >= 512 tiles
     of 64 x 128 with fewer than 64 K-steps: 385-512 rows of 9728 x 2560) or
-    the few-row kernel (3-32 rows), nowhere else; the entry rejects a
+    the skinny or few-row kernel (3-32 rows), nowhere else; the entry rejects a
     shape it does not serve before any launch."""
     from ttspipe_amd import _lib
 
@@ -421,7 +421,7 @@ def test_swiglu_gemm_plan_on_the_host():
                  (1536, 1024, 512, 64, 256, 1), (9728, 2560, 512, 64, 16, 1), (9728, 2560, 512, 32, 256, 1),
                  (9728, 2560, 512, 96, 256, 0), (9728, 2500, 512, 64, 256, 1)):
         assert fits(*args) == 0, args
-    # 3-32 rows where both GEMMs run the few-row kernel unsplit: its pair form
+    # 3-32 rows where both GEMMs run the skinny or the few-row kernel unsplit: its pair form
     for rows in (3, 4, 8, 16, 17, 32):
         assert fits(9728, 2560, rows, 64, 256, 1) == 1, rows
         assert fits(2560, 9728, rows, 64, 256, 0) == 1, rows

@@ -16,7 +16,8 @@ import torch
 
 from oracle import oracle as o
 from tests.conftest import beyond_rounding_error, relative_error
-from tests.gpuutil import bits, dt_code, first_mismatch, from_bits, gemv_rows_shape, gemv_shape, randn_bits
+from tests.gpuutil import (bits, dt_code, first_mismatch, from_bits, gemv_rows_shape, gemv_shape, randn_bits,
+                           split_product)
 from tests.nf4data import dequant_numpy, oracle_args, random_layer, to_linear
 
 pytestmark = pytest.mark.gpu
@@ -302,8 +303,8 @@ def test_several_positions_within_bar(nf4, orc, shape, rows, dtype):
 
 @pytest.mark.parametrize("rows", [3, 16, 17, 40])
 def test_few_rows_over_a_long_row(nf4, orc, rows):
-    """K = 16384: up to 16 rows the few-row kernel splits K over 16 waves; more
-    rows than its limit for that K go to the tiled GEMM. Both within the bar."""
+    """K = 16384: up to 16 rows the skinny kernel splits K over 16 waves; more
+    rows go to the few-row kernel in K splits. Both within the bar."""
     M, K, dtype = 272, 16384, torch.bfloat16
     layer = random_layer(M, K, True, seed=rows + 7)
     lin = to_linear(layer, dtype)
@@ -392,7 +393,7 @@ def test_prefill_gemm_bucket_rows(nf4, orc, name, shape, rows):
 def test_gemm_epilogues(nf4, orc, epi, rows, shape):
     """Residual and SwiGLU-gate epilogues of the GEMM (24 rows: unsplit; 512
     rows at 2560 x 9728: the K-split plan, where the reduce kernel applies
-    them; 512 rows at 9728 x 2560: the unsplit direct-to-LDS kernel, which
+    them; 512 rows at 9728 x 2560: the unsplit tile kernel, which
     applies them itself) against the closed forms round(R + round(y)) and
     round(round(silu(R)) * round(y)) evaluated on the oracle's fp64 product,
     within the 2e-3 bar beyond the output's own rounding. An epilogue with its
@@ -401,7 +402,7 @@ def test_gemm_epilogues(nf4, orc, epi, rows, shape):
 
     (M, K), dtype = shape, torch.float16
     if rows == 512:
-        assert _lib.load().ttsp_nf4_gemm_splits(M, K, rows) == (4 if M == 2560 else 1)
+        assert _lib.load().ttsp_nf4_gemm_tile_splits(M, K, rows) == (4 if M == 2560 else 1)
     layer = random_layer(M, K, True, seed=31)
     lin = to_linear(layer, dtype)
     xb = randn_bits(rows * K, dtype, seed=32, scale=0.5)
@@ -429,7 +430,7 @@ def test_split_gemm_with_rows_not_a_multiple_of_four(nf4, orc, rows):
     from ttspipe_amd import _lib
 
     M, K, dtype = 1540, 2560, torch.bfloat16
-    splits = _lib.load().ttsp_nf4_gemm_splits(M, K, rows)
+    splits = _lib.load().ttsp_nf4_gemm_tile_splits(M, K, rows)
     assert splits > 1
     layer = random_layer(M, K, True, seed=1540)
     lin = to_linear(layer, dtype)
@@ -447,9 +448,10 @@ def test_split_gemm_with_rows_not_a_multiple_of_four(nf4, orc, rows):
 @pytest.mark.parametrize("shape,rows,splits", [((9728, 2560), 512, 1), ((6144, 2560), 512, 2),
                                                ((2560, 4096), 256, 4), ((9730, 2560), 500, 1),
                                                ((9730, 2560), 300, 2)])
-def test_direct_lds_gemm_launches(nf4, orc, shape, rows, splits, nested, dtype):
-    """Every launch the plan gives the direct-to-LDS kernel (unsplit, 2 and 4
-    K-splits) with bf16 and fp16 activations and nested and plain scales,
+def test_span_gemm_launches(nf4, orc, shape, rows, splits, nested, dtype):
+    """Every split count the plan gives 256 to 512 rows of large shapes (unsplit,
+    2 and 4 K-splits), launched in it and as `matmul` takes it (2 splits run
+    unsplit where no norm follows, 4 of 64 to 127 K-steps as 2), with bf16 and fp16 activations and nested and plain scales,
     including ragged tiles (9730 weight rows: M % 4 == 2, a partial 64-row
     tile; 500 and 300 activation rows: a partial 128-row tile), against the
     oracle's fp64 product within the bar."""
@@ -460,35 +462,42 @@ def test_direct_lds_gemm_launches(nf4, orc, shape, rows, splits, nested, dtype):
     layer = random_layer(M, K, nested, seed=M + rows)
     lin = to_linear(layer, dtype)
     xb = randn_bits(rows * K, dtype, seed=rows + 3)
-    y = lin(from_bits(xb, dtype).view(rows, K))
+    x = from_bits(xb, dtype).view(rows, K)
     dt = dt_code(dtype)
     sample = np.concatenate([np.arange(0, rows, 41), [rows - 1]])  # the last row sits in the partial tile
     ref = orc.nf4_gemm_ref(xb.reshape(rows, K)[sample], dt, **oracle_args(layer), M=M, K=K, N=sample.size, bs=64)
-    got = o.to_f32(bits(y), dt).reshape(rows, M)[sample]
-    assert beyond_rounding_error(got, ref, dt) < 2e-3
+    alone = lin(x)
+    for y in (alone, split_product(lin, x, splits)):
+        got = o.to_f32(bits(y), dt).reshape(rows, M)[sample]
+        assert beyond_rounding_error(got, ref, dt) < 2e-3
+    taken = _lib.load().ttsp_nf4_gemm_tile_splits(M, K, rows)
+    assert taken == {2: 1, 4: 2}.get(splits, splits)
+    assert np.array_equal(bits(alone), bits(split_product(lin, x, taken)))
 
 
 @pytest.mark.parametrize("shape,rows,bs2", [((9728, 2560), 512, 16), ((2560, 4096), 256, 16),
                                             ((6144, 2560), 512, 32)])
-def test_direct_lds_gemm_small_second_level_groups(nf4, orc, shape, rows, bs2):
+def test_span_gemm_small_second_level_groups(nf4, orc, shape, rows, bs2):
     """Nested scales with second-level groups of 16 or 32 blocks (1,024 or
-    2,048 codes) at launches the plan gives the direct-to-LDS kernel: where a
-    workgroup's K range (2,560 codes unsplit) could cross two group
-    boundaries the launch falls back to the 64 x 128 kernel; where it spans
-    at most one (1,024 codes a split for 16-block groups, 1,280 for 32) the
-    kernel switches the group's absmax mid-range. Against the oracle."""
+    2,048 codes): the tile kernel resolves each step's scales with its own
+    group's absmax, over a whole K range (2,560 codes unsplit) and a split's
+    (1,024 and 1,280 codes). Against the oracle, in the plan's splits and those
+    `matmul` takes."""
+    from ttspipe_amd import _lib
+
     M, K = shape
     dtype = torch.bfloat16
     layer = random_layer(M, K, True, seed=M + bs2, bs2=bs2)
     lin = to_linear(layer, dtype)
     xb = randn_bits(rows * K, dtype, seed=rows + bs2)
-    y = lin(from_bits(xb, dtype).view(rows, K))
+    x = from_bits(xb, dtype).view(rows, K)
     dt = dt_code(dtype)
     sample = np.concatenate([np.arange(0, rows, 37), [rows - 1]])
     ref = orc.nf4_gemm_ref(xb.reshape(rows, K)[sample], dt, **oracle_args(layer), M=M, K=K, N=sample.size, bs=64,
                            bs2=bs2)
-    got = o.to_f32(bits(y), dt).reshape(rows, M)[sample]
-    assert beyond_rounding_error(got, ref, dt) < 2e-3
+    for y in (lin(x), split_product(lin, x, _lib.load().ttsp_nf4_gemm_splits(M, K, rows))):
+        got = o.to_f32(bits(y), dt).reshape(rows, M)[sample]
+        assert beyond_rounding_error(got, ref, dt) < 2e-3
 
 
 # ------------------------------------------------------------ fused forms (one launch)
@@ -728,10 +737,9 @@ def test_swiglu_few_rows_equals_the_two_launches(nf4, shape, rows, nested, dtype
 @pytest.mark.parametrize("shape,rows,bs2", [((2560, 9728), 512, 256), ((9728, 2560), 256, 256),
                                             ((9728, 2560), 512, 16), ((1536, 1024), 512, 256)])
 def test_swiglu_gemm_declines_what_one_launch_does_not_serve(nf4, shape, rows, bs2):
-    """Shapes whose GEMMs the plan splits along K, row counts below the
-    direct-to-LDS kernel's, second-level groups a workgroup's K range could
-    cross twice, and tile counts below its unsplit rule: None (the caller runs
-    the two launches)."""
+    """Shapes whose GEMMs the plan splits along K, second-level groups shorter
+    than K, and tile counts below the unsplit rule: None (the caller runs the
+    two launches)."""
     M, K = shape
     w1 = to_linear(random_layer(M, K, True, seed=3, bs2=bs2), torch.bfloat16)
     w3 = to_linear(random_layer(M, K, True, seed=4, bs2=bs2), torch.bfloat16)
@@ -741,6 +749,7 @@ def test_swiglu_gemm_declines_what_one_launch_does_not_serve(nf4, shape, rows, b
 
 @pytest.mark.parametrize("shape,rows,splits,epi,nested,dtype", [
     ((2560, 4096), 512, 4, 1, True, torch.bfloat16),   # wo of a 512-row span
+    ((2560, 4096), 256, 4, 1, True, torch.float16),    # and of a 256-row one
     ((2560, 9728), 512, 4, 1, True, torch.bfloat16),   # w2 of a 512-row span
     ((2560, 9728), 64, 4, 1, False, torch.float16),
     ((1024, 4096), 128, 8, 0, True, torch.float16),
@@ -751,8 +760,9 @@ def test_swiglu_gemm_declines_what_one_launch_does_not_serve(nf4, shape, rows, b
     ((4088, 2048), 64, 4, 0, False, torch.bfloat16)])
 def test_split_gemm_with_the_next_norm_equals_the_two_launches(nf4, shape, rows, splits, epi, nested, dtype):
     """`matmul_norm` (the split-K reduce, its epilogue and the RMSNorm of each
-    output row in one launch) against `matmul` then `fusedops.rms_norm`, bit
-    for bit: 2, 4 and 8 splits, every epilogue, fp16 and bf16, plain and
+    output row in one launch) against `matmul` then `fusedops.rms_norm`, and
+    with `span` (from 65 rows the plan's splits, `splits`) against the launch in
+    that many splits and the norm, bit for bit: 2, 4 and 8 splits, every epilogue, fp16 and bf16, plain and
     nested scales, a row count that is not a multiple of four, rows of one
     to eight 512-column steps (a wave each) and a ragged last step."""
     from ttspipe_amd import _lib, fusedops
@@ -766,16 +776,19 @@ def test_split_gemm_with_the_next_norm_equals_the_two_launches(nf4, shape, rows,
     r = from_bits(randn_bits(rows * M, dtype, seed=rows + 12), dtype).view(1, rows, M) if epi else None
     g = torch.rand(M, generator=torch.Generator().manual_seed(M)).add(0.5).to(dtype).cuda()
     eps = 1e-5
-    got = nf4.matmul_norm(lin, x, g, eps, epi=epi, operand=r)
-    assert got is not None
-    y, yn = got
-    ref = nf4.matmul(lin, x, epi=epi, operand=r)
-    ref_n = fusedops.rms_norm(ref, g, eps)
-    assert ref_n is not None
-    torch.cuda.synchronize()
-    for a, b in ((y, ref), (yn, ref_n)):
-        ab, bb = bits(a), bits(b)
-        assert np.array_equal(ab, bb), first_mismatch(ab, bb)
+    for span in (False, True):
+        if span and rows <= 64:
+            continue  # (the few-row kernel's own splits: test_few_rows_gpu.py)
+        got = nf4.matmul_norm(lin, x, g, eps, epi=epi, operand=r, span=span)
+        assert got is not None
+        y, yn = got
+        ref = split_product(lin, x, splits, epi, r) if span else nf4.matmul(lin, x, epi=epi, operand=r)
+        ref_n = fusedops.rms_norm(ref, g, eps)
+        assert ref_n is not None
+        torch.cuda.synchronize()
+        for a, b in ((y, ref), (yn, ref_n)):
+            ab, bb = bits(a), bits(b)
+            assert np.array_equal(ab, bb), first_mismatch(ab, bb)
     nb = o.to_f32(bits(ref_n), dt_code(dtype)).reshape(rows, M)
     assert np.all(np.isfinite(nb)) and np.abs(nb).max() > 0
 

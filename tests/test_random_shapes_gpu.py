@@ -21,7 +21,7 @@ import torch
 
 from oracle import oracle as o
 from tests.conftest import beyond_rounding_error
-from tests.gpuutil import bits, dt_code, first_mismatch, from_bits, gemv_shape, randn_bits
+from tests.gpuutil import bits, dt_code, first_mismatch, from_bits, gemv_shape, randn_bits, split_product
 from tests.nf4data import oracle_args, random_layer, to_linear
 
 pytestmark = pytest.mark.gpu
@@ -101,9 +101,9 @@ def test_matmul_random_shapes_within_bar(nf4, orc, case):
     assert splits  # (recorded for the failure message of a future plan change)
 
 
-def _dl_shapes(n: int, seed: int, splits: int):
-    """(M, K, bs, nested, dtype, rows) the launch plan gives the direct-to-LDS
-    kernel with `splits` K splits: 4 where K has 64 or more 64-code steps and
+def _span_shapes(n: int, seed: int, splits: int):
+    """(M, K, bs, nested, dtype, rows) of 256 to 512 rows that the split plan
+    gives `splits` K splits by its rule for large shapes: 4 where K has 64 or more 64-code steps and
     there are at least 75 64 x 128 tiles; with fewer steps unsplit from 512
     tiles and 2 splits from 300."""
     rng = np.random.default_rng(seed)
@@ -132,29 +132,34 @@ def _dl_shapes(n: int, seed: int, splits: int):
 
 
 @pytest.mark.parametrize("splits", [1, 2, 4])
-def test_direct_lds_gemm_random_shapes_within_bar(nf4, orc, splits):
-    """Six random shapes per launch form of the direct-to-LDS kernel
+def test_tile_gemm_random_shapes_within_bar(nf4, orc, splits):
+    """Six random shapes per split count of the plan at 256 to 512 rows
     (unsplit, 2 and 4 K-splits): ragged weight and activation rows, block
     sizes 64 to 256, plain and nested scales (whose second-level group may
     change inside a workgroup's K range), bf16 and fp16; a sample of rows
-    against the oracle's fp64 product within the bar."""
+    against the oracle's fp64 product within the bar, in the plan's splits (as
+    a prompt block adds them) and in those `matmul` takes."""
     from ttspipe_amd import _lib
-    from tests.test_abi import _dl_split
+    from tests.test_abi import _span_split
 
-    for i, (M, K, bs, nested, dtype, rows) in enumerate(_dl_shapes(6, 2700 + splits, splits)):
+    for i, (M, K, bs, nested, dtype, rows) in enumerate(_span_shapes(6, 2700 + splits, splits)):
         where = f"M={M} K={K} rows={rows} bs={bs} nested={nested} {dtype}"
-        assert _dl_split(M, K, rows) == splits, where
+        assert _span_split(M, K, rows) == splits, where
         assert _lib.load().ttsp_nf4_gemm_splits(M, K, rows) == splits, where
         layer = random_layer(M, K, nested, seed=splits * 100 + i + 7, bs=bs)
         lin = to_linear(layer, dtype)
         xb = randn_bits(rows * K, dtype, seed=rows + i + 11)
-        y = lin(from_bits(xb, dtype).view(rows, K))
+        x = from_bits(xb, dtype).view(rows, K)
         dt = dt_code(dtype)
         sample = np.unique(np.concatenate([np.linspace(0, rows - 1, 5).astype(int), [rows - 1]]))
         ref = orc.nf4_gemm_ref(xb.reshape(rows, K)[sample], dt, **oracle_args(layer), M=M, K=K, N=sample.size,
                                bs=bs, bs2=layer["bs2"] or 256)
-        got = o.to_f32(bits(y), dt).reshape(rows, M)[sample]
-        assert beyond_rounding_error(got, ref, dt) < 2e-3, where
+        alone = lin(x)
+        for y in (alone, split_product(lin, x, splits)):
+            got = o.to_f32(bits(y), dt).reshape(rows, M)[sample]
+            assert beyond_rounding_error(got, ref, dt) < 2e-3, where
+        taken = _lib.load().ttsp_nf4_gemm_tile_splits(M, K, rows)
+        assert np.array_equal(bits(alone), bits(split_product(lin, x, taken))), f"{where}: not in {taken} splits"
 
 
 @pytest.mark.parametrize("case", range(6))

@@ -70,6 +70,32 @@ def test_tile_gemm_against_fp64(nf4, orc, shape, rows, nested, bs, bs2, dtype, e
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,rows,nested,dtype", [(6144, 385, True, torch.bfloat16), (6144, 400, False, torch.float16),
+                                                 (6144, 512, True, torch.bfloat16), (6146, 511, True, torch.float16)])
+def test_span_partial_sums_against_fp64(nf4, orc, M, rows, nested, dtype):
+    """A prompt block's wqkv: `matmul_partials(span=True)` in the plan's two
+    splits of 2560 codes, its sums added in order against the fp64 product,
+    ragged M and rows. The bar on the fp32 sums themselves, 1e-5 of the largest:
+    160 roundings of 2^-24 in a random walk are 8e-7 of a sum's deviation, 5
+    times that over 1e5 of them."""
+    from ttspipe_amd import _lib
+
+    K, dt = 2560, dt_code(dtype)
+    assert _lib.load().ttsp_nf4_gemm_splits(M, K, rows) == 2
+    layer = random_layer(M, K, nested, seed=M + rows)
+    lin = to_linear(layer, dtype)
+    assert nf4.prepare(lin)
+    xb = randn_bits(rows * K, dtype, seed=rows, scale=0.5)
+    work, splits = nf4.matmul_partials(lin, from_bits(xb, dtype).view(rows, K), span=True)
+    assert splits == 2
+    sample = np.unique(np.r_[0:rows:29, rows - 1])
+    ref = orc.nf4_gemm_ref(xb.reshape(rows, K)[sample], dt, **oracle_args(layer), M=M, K=K, N=sample.size, bs=64,
+                           bs2=256).astype(np.float64).reshape(sample.size, M)
+    got = (work[0] + work[1]).cpu().numpy().astype(np.float64)[sample]
+    assert np.abs(got - ref).max() < 1e-5 * np.abs(ref).max()
+
+
+@pytest.mark.gpu
 def test_tile_gemm_is_reproducible(nf4):
     """Twenty runs of each form give the same bits (a stage refilled while
     another wave still reads it would not)."""
