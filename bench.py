@@ -358,14 +358,17 @@ def bench_gemm(rows: int = 512, copies: int = 4, reps: int = 20):
     dev = torch.device("cuda", 0)
     lut = torch.tensor(NF4_CODE, dtype=torch.float32, device=dev)
     res, total_s, total_flop = [], 0.0, 0
-    # the seven projections of the reference's table, then wqkv as the
-    # prefill block runs it (q, k and v rows of one weight, one launch)
-    for i, (name, M, K) in enumerate(LAYER + [("qkv", 6144, 2560)]):
+    # the seven projections of the reference's table, then wqkv (q, k and v rows
+    # of one weight, one launch) and wo as the prefill block runs them
+    for i, (name, M, K) in enumerate(LAYER + [("qkv", 6144, 2560), ("wo", 2560, 4096)]):
         lins = [Linear(M, K, True, seed=500 + 10 * i + c, device=dev) for c in range(copies)]
         x = torch.randn(rows, K, device=dev).to(torch.bfloat16)
         y = torch.empty(rows, M, dtype=torch.bfloat16, device=dev)
-        # the K split nf4gemv.matmul uses for this shape (fp32 partials in a workspace)
-        splits = lib.ttsp_nf4_gemm_splits(M, K, rows)
+        # the K split nf4gemv.matmul uses for this shape (fp32 partials in a
+        # workspace); the block's wqkv and wo, whose sums its head-norm kernel
+        # and the next norm's reduce add, take the plan's
+        plan = lib.ttsp_nf4_gemm_splits if name in ("qkv", "wo") else lib.ttsp_nf4_gemm_tile_splits
+        splits = plan(M, K, rows)
         work = torch.empty(splits * rows * M, dtype=torch.float32, device=dev)
 
         def body():
@@ -386,7 +389,7 @@ def bench_gemm(rows: int = 512, copies: int = 4, reps: int = 20):
         flop = 2 * rows * M * K
         res.append({"name": name, "M": M, "K": K, "k_splits": splits, "us": round(sec * 1e6, 2),
                     "tflops": round(flop / sec / 1e12, 1)})
-        if name != "qkv":
+        if name not in ("qkv", "wo"):
             total_s += sec
             total_flop += flop
         del lins
@@ -427,7 +430,7 @@ def bench_gemm(rows: int = 512, copies: int = 4, reps: int = 20):
             100 * total_flop / layer / 1e12 / MFMA_PEAK_TFLOPS, 2)
         # the prefill block's four launches: wqkv, wo, the SwiGLU pair, w2
         us = {r["name"]: r["us"] * 1e-6 for r in res}
-        block = us["qkv"] + us["o"] + sec + us["down"]
+        block = us["qkv"] + us["wo"] + sec + us["down"]
         out["prefill_block_launches_us"] = round(block * 1e6, 1)
         out["pct_of_mfma_peak_prefill_block_launches"] = round(
             100 * total_flop / block / 1e12 / MFMA_PEAK_TFLOPS, 2)
