@@ -137,10 +137,10 @@ __global__ __launch_bounds__(64 * NRM_CH) void nf4_gemm_reduce_norm_kernel(const
 // K-steps) whose workgroups fit one to a CU: a split's fp32 partial sums cost
 // a write and a read of splits x N x M floats, so a second pass of workgroups
 // only pays where each split keeps a long K run. Between 128 and 256 tiles 4
-// splits pay only past 16 K-steps each. 256 to 512 rows: dl_plan below. 33 to
+// splits pay only past 16 K-steps each. 256 to 512 rows: span_plan below. 33 to
 // 64 rows: 4 ways where each split keeps 8 or more K-steps, else 2 (callers
-// with a choice take ttsp_nf4_gemm_few's plan, which is faster). Up to 64 rows
-// otherwise the few-row or the skinny kernel, never split.
+// with a choice take ttsp_nf4_gemm_few's plan, which is faster). Up to 32 rows
+// the few-row or the skinny kernel unsplit, but for K past their longest rows.
 constexpr int SKINNY_MAX_N = 16;
 int skinny_max_k();
 bool few_unsplit(int M, int K, int N);
@@ -162,9 +162,9 @@ int gemm_tile(const void* X, int dt, const uint8_t* W, const uint8_t* A8, const 
 // 256 to 512 rows: 4 K-splits where K has 64 or more steps and there are at
 // least 75 64 x 128 tiles; with fewer steps none from 512 tiles and 2 from 300.
 // 0: no rule here.
-constexpr int DL_MIN_N = 256, DL_MAX_N = 512;
-static int dl_plan(int M, int K, int N) {
-  if (N < DL_MIN_N || N > DL_MAX_N) return 0;
+constexpr int SPAN_MIN_N = 256, SPAN_MAX_N = 512;
+static int span_plan(int M, int K, int N) {
+  if (N < SPAN_MIN_N || N > SPAN_MAX_N) return 0;
   const int steps = K / KT;
   const long long t = gemm_tiles(M, N, 64, 128);
   if (steps >= 64) return t >= 75 && steps % 8 == 0 && steps / 4 <= 64 ? 4 : 0;
@@ -178,7 +178,7 @@ static int gemm_plan(int M, int K, int N) {
     for (int sp = 4; sp >= 2; sp /= 2)
       if (steps % (2 * sp) == 0 && steps / sp >= 8) return sp;
   if (skinny(K, N) || few_unsplit(M, K, N)) return 1;
-  if (const int dl = dl_plan(M, K, N)) return dl;
+  if (const int span = span_plan(M, K, N)) return span;
   const long long t = gemm_tiles(M, N, 64, 128);
   if (t >= 256) return 1;
   int splits = 1;
@@ -285,11 +285,13 @@ static bool swiglu_skinny(int M, int K, int N) {
 }
 
 // Whether the SwiGLU pair fits one launch of the tile kernel: where each of
-// its two GEMMs runs that kernel unsplit and over whole K (more than 256 64 x
-// 128 tiles), so that the one launch gives their bits. (Second-level groups
-// shorter than K keep two launches, as before the scales were resolved per step.)
+// its two GEMMs runs that kernel unsplit and over whole K (256 to 512 rows of
+// at least 512 64 x 128 tiles and K below 4096), so that the one launch gives
+// their bits. One launch against w1 and then w3 with the gate: 9728 x 2560 at
+// 385 rows 78 / 87 us, at 512 79 / 86. (Second-level groups shorter than K take
+// two launches; the kernel would serve them.)
 static bool swiglu_fits(int M, int K, int N, int bs_shift, int bs2_shift, bool nested) {
-  if (M <= 0 || K <= 0 || K % 128 || N <= 64 || dl_plan(M, K, N) != 1) return false;
+  if (M <= 0 || K <= 0 || K % 128 || N <= 64 || span_plan(M, K, N) != 1) return false;
   return !(nested && (long long)K > (1LL << (bs_shift + bs2_shift)));
 }
 
@@ -316,7 +318,7 @@ static int gemm_args(const void* X, const uint8_t* W, const uint8_t* A8, const f
 // One entry for every row count: up to GEMV_ROWS_N rows take the
 // bandwidth-bound GEMV (or, past the rows it holds, the kernels below), up
 // to 64 rows the skinny or the few-row MFMA kernel (weights streamed once),
-// more rows the tiled MFMA kernel (weights read once per BN rows), unsplit.
+// more rows the tile kernel (weights read once per 128 rows), unsplit.
 extern "C" int ttsp_nf4_gemm(const void* X, int x_dtype, const uint8_t* W, const uint8_t* A8,
                              const float* AMAX, const float* CODE2, float offset, const float* LUT,
                              void* Y, const void* R, int epi, int M, int K, int N, int blocksize,
@@ -346,20 +348,21 @@ extern "C" int ttsp_nf4_gemm_splits(int M, int K, int N) {
 
 // The splits a caller with a workspace should take from 65 rows:
 // ttsp_nf4_gemm_splits', but from 256 rows unsplit instead of 2 ways where no
-// norm follows in the reduce (M past its widest row): 9728 x 2560 at 256 rows
-// 28.0 us against 32 and a 10 us reduce, 6144 x 2560 at 512 28.7 against 30.3
-// and 7 (sums that another kernel adds keep the two splits); and 2 instead of
-// 4 where a split still has 32 K-steps or more but fewer than 64 (2560 x 4096:
-// 18.1 against 18.1 us at 256 rows, 26.9 against 26.5 at 512, half the sums to
-// reduce).
+// norm follows in the reduce (M past its widest row; with the reduce, us, 1
+// split against 2: 9728 x 2560 at 256 rows 27.6 / 31.8, 6144 x 2560 at 512 27.9
+// / 33.7, 7168 x 2048 at 385 24.8 / 31.7; sums that another kernel adds keep
+// the two splits); and 2 instead of 4 where a split still has 32 K-steps or
+// more but fewer than 64: half the sums to reduce, which a wide weight feels (2
+// splits against 4: 2560 x 4096 at 256 rows 22.9 / 22.5, at 385 26.9 / 25.6, at
+// 512 27.6 / 27.4; 5120 x 5120 at 512 45.2 / 57.4, 14336 x 4096 88.6 / 111.7).
 namespace ttsp {
 
 int tile_splits(int M, int K, int N) {
   if (M <= 0 || K <= 0 || N <= 1 || K % 128) return 1;
-  const int dl = dl_plan(M, K, N), plan = gemm_plan(M, K, N);
-  if (N <= 64 || !dl) return plan;
-  if (M > 64 * 8 * NRM_CH && dl == 2) return 1;
-  return dl == 4 && K / KT < 128 && K / KT % 4 == 0 ? 2 : plan;
+  const int span = span_plan(M, K, N), plan = gemm_plan(M, K, N);
+  if (N <= 64 || !span) return plan;
+  if (M > 64 * 8 * NRM_CH && span == 2) return 1;
+  return span == 4 && K / KT < 128 && K / KT % 4 == 0 ? 2 : plan;
 }
 
 // Estimated us of the tile kernel from 65 rows: rounds of 256 workgroups, each

@@ -361,9 +361,12 @@ bool few_takes(int M, int K, int N) {
 // 17 to 32 of a longer K than FEW_UNSPLIT_MAX_K, whose four waves a workgroup
 // would each add a long run (256 x 40960 at 32 rows 57.9 us, 20.3 in 4 splits;
 // 1024 x 16384 25.7 and 12.9; at 2560 x 4096 the two are within 0.6 us); at 9 to
-// 16 the skinny kernel's 16-row tiles make more workgroups of a small matrix
-// (2560 x 4096 at 16 rows 7.7 against 8.3 us here, 1024 x 3072 6.5 against
-// 6.6; 9728 x 2560 12.7 against 9.4, 6144 x 2560 9.4 against 6.5).
+// 16 the skinny kernel's 16-row tiles make more workgroups of a small matrix.
+// Measured at 16 rows, skinny against this kernel, us: 1024 x 2560 6.5 / 6.7,
+// 2560 x 4096 8.4 / 8.7, 4096 x 2560 6.9 / 6.9; past 4096 rows the skinny one
+// takes a second round: 5120 x 2560 9.7 / 6.9, 6144 x 2560 9.9 / 7.0, 9728 x
+// 2560 12.3 / 9.8, 6144 x 9728 29.0 / 15.5. (The line here, 6144 rows and K up
+// to 4096, is on the safe side of that.)
 bool few_unsplit(int M, int K, int N) {
   if (!few_takes(M, K, N)) return false;
   return N > 16 ? N > 32 || K <= FEW_UNSPLIT_MAX_K : (M + 31) / 32 >= 192 && K <= 4096;

@@ -95,8 +95,6 @@ struct SkinnyW3 {
   float offset;
 };
 
-constexpr int NT = 1;  // 16-row tiles of X
-
 template <int DT, int R, int NW, int MS, bool NESTED, int TG = 1, bool PAIR = false>
 __global__ __launch_bounds__(64 * NW * TG) void nf4_skinny_kernel(
     const uint16_t* __restrict__ X, const uint8_t* __restrict__ W, const uint8_t* __restrict__ A8,
@@ -107,11 +105,11 @@ __global__ __launch_bounds__(64 * NW * TG) void nf4_skinny_kernel(
   // [e][j]; after the loop the same memory holds each wave's partial sums
   constexpr int NWT = NW * TG;  // waves a workgroup
   constexpr int S = PAIR ? 2 * R : R;  // tile slots: slot r < R of W, slot R + r of W3 (same rows)
-  static_assert(NWT * S * NT * 64 * sizeof(f32x4) <= SK_LDS, "partial sums exceed the table's LDS");
+  static_assert(NWT * S * 64 * sizeof(f32x4) <= SK_LDS, "partial sums exceed the table's LDS");
   __shared__ __align__(16) unsigned char lds[SK_LDS];
   __shared__ __align__(16) float code2_s[NESTED ? (PAIR ? 512 : 256) : 4];
   float2 (*lut2)[SK_REP] = reinterpret_cast<float2 (*)[SK_REP]>(lds);
-  f32x4 (*part)[S * NT][64] = reinterpret_cast<f32x4 (*)[S * NT][64]>(lds);
+  f32x4 (*part)[S][64] = reinterpret_cast<f32x4 (*)[S][64]>(lds);
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int grp = TG > 1 ? wave / NW : 0, wk = TG > 1 ? wave % NW : wave;  // row-tile group, K run
@@ -147,16 +145,12 @@ __global__ __launch_bounds__(64 * NW * TG) void nf4_skinny_kernel(
   if constexpr (NESTED && PAIR)
 #pragma unroll
     for (int i = 0; i < 4; ++i) c2v3[i] = w3.CODE2[4 * lane + i];
-  u32x4 xq[SK_PF][NT][4];
-  auto load_x = [&](u32x4 (&xs)[NT][4], int step) {
+  u32x4 xq[SK_PF][4];
+  auto load_x = [&](u32x4 (&xs)[4], int step) {
     const int st = min(step, max(s1 - 1, 0));
+    const u32x4* xr = reinterpret_cast<const u32x4*>(X + (size_t)min(m, N - 1) * K + 128 * st + 32 * q);
 #pragma unroll
-    for (int c = 0; c < NT; ++c) {
-      const int n = min(16 * c + m, N - 1);
-      const u32x4* xr = reinterpret_cast<const u32x4*>(X + (size_t)n * K + 128 * st + 32 * q);
-#pragma unroll
-      for (int t = 0; t < 4; ++t) xs[c][t] = xr[t];
-    }
+    for (int t = 0; t < 4; ++t) xs[t] = xr[t];
   };
   // (a wave with an empty run - K < 128 NW - loads step 0 and adds nothing)
   const int slast = max(s1 - 1, 0);
@@ -186,11 +180,9 @@ __global__ __launch_bounds__(64 * NW * TG) void nf4_skinny_kernel(
     __builtin_amdgcn_sched_barrier(0);
   }
 
-  f32x4 acc[S][NT];
+  f32x4 acc[S];
 #pragma unroll
-  for (int r = 0; r < S; ++r)
-#pragma unroll
-    for (int c = 0; c < NT; ++c) acc[r][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int r = 0; r < S; ++r) acc[r] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
   // the tables, while the operands stream: wave w writes entries w, w + NW,
   // ..., four a store instruction (lane l: entry base + l / 16, copies
@@ -216,17 +208,15 @@ __global__ __launch_bounds__(64 * NW * TG) void nf4_skinny_kernel(
   __builtin_amdgcn_sched_barrier(0);
   const unsigned char* tab = reinterpret_cast<const unsigned char*>(&lut2[0][0]);
   const uint32_t lane8 = 8u * (uint32_t)(lane & (SK_REP - 1));
-  // rows n >= N of an X tile contribute zeros (their fragments are replaced)
-  bool nvalid[NT];
-#pragma unroll
-  for (int c = 0; c < NT; ++c) nvalid[c] = 16 * c + m < N;
+  // rows n >= N of the X tile contribute zeros (their fragments are replaced)
+  const bool nvalid = m < N;
 
   // Every budgeted step is computed - a branch around a step would let the
   // compiler sink that step's loads into it, after the barrier - and steps
   // past the wave's run add exact zeros (zero scale, zero activations).
 #pragma unroll
   for (int j = 0; j < MS; ++j) {
-    u32x4 (&xs)[NT][4] = xq[j % SK_PF];
+    u32x4 (&xs)[4] = xq[j % SK_PF];
     const bool live = s0 + j < s1;
 #pragma unroll
     for (int r = 0; r < S; ++r) {
@@ -245,11 +235,8 @@ __global__ __launch_bounds__(64 * NW * TG) void nf4_skinny_kernel(
           bw[b] = sk_pack2<DT>(__fmul_rn(pc.x, sc), __fmul_rn(pc.y, sc));
         }
         const u32x4 bop = {bw[0], bw[1], bw[2], bw[3]};
-#pragma unroll
-        for (int c = 0; c < NT; ++c) {
-          const u32x4 xa = live && nvalid[c] ? xs[c][t] : u32x4{0u, 0u, 0u, 0u};
-          acc[r][c] = sk_mfma<DT>(xa, bop, acc[r][c]);
-        }
+        const u32x4 xa = live && nvalid ? xs[t] : u32x4{0u, 0u, 0u, 0u};
+        acc[r] = sk_mfma<DT>(xa, bop, acc[r]);
       }
     }
     if (j + SK_PF < MS) load_x(xs, s0 + j + SK_PF);
@@ -259,43 +246,38 @@ __global__ __launch_bounds__(64 * NW * TG) void nf4_skinny_kernel(
   // tiles r with r % NW == w
   __syncthreads();  // every wave is past its last lookup: the table's memory takes the partial sums
 #pragma unroll
-  for (int r = 0; r < S; ++r)
-#pragma unroll
-    for (int c = 0; c < NT; ++c) part[wave][r * NT + c][lane] = acc[r][c];
+  for (int r = 0; r < S; ++r) part[wave][r][lane] = acc[r];
   __syncthreads();
   const int ep = epi & 3;
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     if (r % NW != wk) continue;
     const int row = row0 + 16 * r + m;
+    f32x4 v = part[grp * NW][r][lane], v3 = {0.0f, 0.0f, 0.0f, 0.0f};
+    if constexpr (PAIR) v3 = part[grp * NW][R + r][lane];
 #pragma unroll
-    for (int c = 0; c < NT; ++c) {
-      f32x4 v = part[grp * NW][r * NT + c][lane], v3 = {0.0f, 0.0f, 0.0f, 0.0f};
-      if constexpr (PAIR) v3 = part[grp * NW][(R + r) * NT + c][lane];
+    for (int w = 1; w < NW; ++w) {
+      const f32x4 o = part[grp * NW + w][r][lane];
 #pragma unroll
-      for (int w = 1; w < NW; ++w) {
-        const f32x4 o = part[grp * NW + w][r * NT + c][lane];
+      for (int i = 0; i < 4; ++i) v[i] = __fadd_rn(v[i], o[i]);
+      if constexpr (PAIR) {
+        const f32x4 o3 = part[grp * NW + w][R + r][lane];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = __fadd_rn(v[i], o[i]);
-        if constexpr (PAIR) {
-          const f32x4 o3 = part[grp * NW + w][(R + r) * NT + c][lane];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) v3[i] = __fadd_rn(v3[i], o3[i]);
-        }
+        for (int i = 0; i < 4; ++i) v3[i] = __fadd_rn(v3[i], o3[i]);
       }
+    }
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int n = 16 * c + 4 * q + i;
-        if (n >= N || row >= M || !own) continue;
-        const size_t o = (size_t)n * M + row;
-        const float y = Elem<DT>::load(Elem<DT>::store(v[i]));
-        float out = y;
-        if constexpr (PAIR)  // W1's output as its launch stores it, then W3's gate epilogue
-          out = __fmul_rn(Elem<DT>::load(Elem<DT>::store(silu_rn(y))), Elem<DT>::load(Elem<DT>::store(v3[i])));
-        else if (ep == 1) out = __fadd_rn(Elem<DT>::load(RES[o]), y);
-        else if (ep == 2) out = __fmul_rn(Elem<DT>::load(Elem<DT>::store(silu_rn(Elem<DT>::load(RES[o])))), y);
-        Y[o] = Elem<DT>::store(out);
-      }
+    for (int i = 0; i < 4; ++i) {
+      const int n = 4 * q + i;
+      if (n >= N || row >= M || !own) continue;
+      const size_t o = (size_t)n * M + row;
+      const float y = Elem<DT>::load(Elem<DT>::store(v[i]));
+      float out = y;
+      if constexpr (PAIR)  // W1's output as its launch stores it, then W3's gate epilogue
+        out = __fmul_rn(Elem<DT>::load(Elem<DT>::store(silu_rn(y))), Elem<DT>::load(Elem<DT>::store(v3[i])));
+      else if (ep == 1) out = __fadd_rn(Elem<DT>::load(RES[o]), y);
+      else if (ep == 2) out = __fmul_rn(Elem<DT>::load(Elem<DT>::store(silu_rn(Elem<DT>::load(RES[o])))), y);
+      Y[o] = Elem<DT>::store(out);
     }
   }
 }

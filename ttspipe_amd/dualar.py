@@ -72,7 +72,8 @@ class DualARConfig:
 #: spans of the largest. The reference pads to 1, 2, 4, 8, 16 or 32 rows
 #: (graphs.py:137; its MMA kernel takes at most 32); the GEMM here takes any
 #: row count, so the buckets go on to 512. A 1-position span runs the decode
-#: block (the GEMV), 2 positions the two-row GEMV, 4-64 the few-row kernel.
+#: block (the GEMV), 2 positions the two-row GEMV, 4 and 8 the skinny kernel,
+#: 16-64 the few-row kernel, 128-512 the tile kernel.
 PREFILL_BUCKETS = (1, 2, 4, 8, 16, 32, 64, 128, 256, 512)
 
 def prefill_spans(n: int):

@@ -172,7 +172,8 @@ def matmul(module, x, *, epi: int = EPI_NONE, operand=None, out=None, wide: bool
     EPI_RESIDUAL gives `operand + y`, EPI_SILU_GATE `silu(operand) * y`, each
     rounded exactly where the separate torch ops would round. `operand` must
     match the output in shape, dtype and device and be contiguous; `out`, if
-    given, is written in place.
+    given, is written in place. `wide` (a prompt's merged spans) keeps the
+    512-row order of sums from 1024 rows (`_dense`).
     """
     import torch
 
@@ -240,9 +241,9 @@ def matmul(module, x, *, epi: int = EPI_NONE, operand=None, out=None, wide: bool
     return out.view(*shape[:-1], M) if given else out
 
 
-#: Rows the few-row kernel takes (`ttsp_nf4_gemm_few`), and from how many `matmul` lets it split K: at fewer the
+#: From how many rows `matmul` lets the few-row kernel (`ttsp_nf4_gemm_few`) split K, and the most it takes: at fewer the
 #: reduce launch costs what the split saves, unless the reduce runs anyway (`matmul_norm(span=True)`).
-FEW_MIN_ROWS, FEW_SPLIT_ROWS, FEW_MAX_ROWS = 9, 33, 64
+FEW_SPLIT_ROWS, FEW_MAX_ROWS = 33, 64
 
 
 def _few(lib, fast, x, dt, rows, out, operand, epi, work, norm_weight=None, eps=0.0, out_n=None):
@@ -474,9 +475,10 @@ def matmul_swiglu(module1, module3, x, *, out=None, wide: bool = False):
     two-launch form `matmul(w3, x, epi=EPI_SILU_GATE, operand=matmul(w1, x))`
     and with its bits; None where one launch does not serve the shape (it
     serves where both GEMMs would run the tile kernel unsplit over whole K, e.g.
-    385 to 512 rows of 9728 x 2560, and where both would run the few-row
-    kernel, 3 to 32 rows, whose pair form reads each row tile of w1 and w3
-    in one workgroup)."""
+    385 to 512 rows of 9728 x 2560, where both would run the dense form
+    unsplit, and from 3 to 32 rows where both would run the skinny or the
+    few-row kernel, whose pair forms read each row tile of w1 and w3 in one
+    workgroup). `wide`: as `matmul`'s."""
     import torch
 
     if not (prepare(module1) and prepare(module3)):
