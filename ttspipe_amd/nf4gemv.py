@@ -207,7 +207,7 @@ def matmul(module, x, *, epi: int = EPI_NONE, operand=None, out=None, wide: bool
     elif out.dtype != dtype or out.numel() != rows * M or not out.is_contiguous():
         return None
     lib = _lib.lib()
-    dense = _dense(M, K, rows, wide)
+    dense = _dense(M, K, rows, wide) if rows >= DENSE_MIN_ROWS else 0
     if dense:
         # the dequantised weight, then (K split) the partial sums
         work = _dense_work(2 * M * K + (4 * dense * rows * M if dense > 1 else 0), device)
