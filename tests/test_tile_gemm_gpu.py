@@ -7,7 +7,7 @@ import torch
 
 from oracle import oracle as o
 from tests.conftest import beyond_rounding_error
-from tests.gpuutil import bits, dt_code, from_bits, randn_bits
+from tests.gpuutil import bits, dt_code, from_bits, randn_bits, split_product
 from tests.nf4data import oracle_args, random_layer, to_linear
 
 
@@ -93,6 +93,33 @@ def test_span_partial_sums_against_fp64(nf4, orc, M, rows, nested, dtype):
                            bs2=256).astype(np.float64).reshape(sample.size, M)
     got = (work[0] + work[1]).cpu().numpy().astype(np.float64)[sample]
     assert np.abs(got - ref).max() < 1e-5 * np.abs(ref).max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,rows", [(1024, 1024, 128), (6144, 2560, 385), (6144, 2560, 512), (2560, 4096, 300)])
+@pytest.mark.parametrize("epi", [1, 2])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_epilogue_over_all_operands_equals_the_reduce_kernels(nf4, M, K, rows, epi, dtype):
+    """The tile kernel's residual and gate, eight values at a time, against the
+    split reduce's, one by one, bit for bit: one-hot rows of X make a product
+    that no order of sums changes, and the operands run over every finite value
+    of the type, both infinities and NaN (which stays a NaN)."""
+    from ttspipe_amd import _lib
+
+    lin = to_linear(random_layer(M, K, True, seed=6), dtype)
+    assert nf4.prepare(lin)
+    x = torch.zeros(rows, K, dtype=dtype, device="cuda")
+    x[torch.arange(rows), (torch.arange(rows) * 37) % K] = 1.0
+    r = torch.arange(rows * M, device="cuda").to(torch.int16).view(dtype).view(rows, M).contiguous()
+    f, lib, out = lin._nf4_fast, _lib.load(), torch.empty(rows, M, dtype=dtype, device="cuda")
+    rc = lib.ttsp_nf4_gemm(x.data_ptr(), _lib.dtype_code(dtype), f["w"], f["a8"], f["amax"], f["code2"], f["offset"],
+                           f["lut"].data_ptr(), out.data_ptr(), r.data_ptr(), epi, M, K, rows, 64, 256, _lib.stream())
+    splits = lib.ttsp_nf4_gemm_splits(M, K, rows)
+    assert rc == 0 and splits > 1
+    ref = split_product(lin, x, splits, epi, r)
+    nan = torch.isnan(ref.float())
+    assert torch.equal(nan, torch.isnan(out.float())) and bool(nan.any()) and not bool(nan.all())
+    assert torch.equal(out.view(torch.int16)[~nan], ref.view(torch.int16)[~nan])
 
 
 @pytest.mark.gpu

@@ -288,7 +288,7 @@ static bool swiglu_skinny(int M, int K, int N) {
 // its two GEMMs runs that kernel unsplit and over whole K (256 to 512 rows of
 // at least 512 64 x 128 tiles and K below 4096), so that the one launch gives
 // their bits. One launch against w1 and then w3 with the gate: 9728 x 2560 at
-// 385 rows 78 / 87 us, at 512 79 / 86. (Second-level groups shorter than K take
+// 385 rows 74 / 78 us, at 512 73.5 / 76. (Second-level groups shorter than K take
 // two launches; the kernel would serve them.)
 static bool swiglu_fits(int M, int K, int N, int bs_shift, int bs2_shift, bool nested) {
   if (M <= 0 || K <= 0 || K % 128 || N <= 64 || span_plan(M, K, N) != 1) return false;

@@ -32,7 +32,7 @@
 //   touch every bank the minimum number of times), -5 % against one copy.
 // * 128 rows (W 4) between: 9728 x 2560 at 256 rows 34.1 -> 28.0.
 // The SwiGLU form takes W 4 with one copy, so that two workgroups fit a CU
-// (9728 x 2560 at 512 rows 86 -> 80; W 8 with 32 copies 86).
+// (9728 x 2560 at 512 rows 86 -> 73; W 8 with 32 copies was slower).
 #include "nf4_mfma.h"
 
 namespace ttsp {
@@ -383,38 +383,66 @@ __global__ __launch_bounds__(64 * W * KG) void nf4_gemm_tile_kernel(
     }
     return;
   }
-  // the rounded tile through the ring, 64 activation rows at a time, stored as
-  // 16-byte pieces of whole rows
-  constexpr int PITCH = BM * 2 + 16, CPR = BMO / 8;
-  constexpr int QB = 64 * PITCH <= KG * STAGE ? 2 : 1;  // 32-row blocks a pass
-  static_assert(32 * QB * PITCH <= KG * STAGE, "the output rows exceed a ring stage");
-  uint8_t* const stg = &ring1[0][0];
+  // the rounded tile through the ring's three stages, stored as 16-byte pieces
+  // of whole rows. The epilogue's operands are requested before the staging
+  // (read piece by piece in the loop they cost a memory round trip a turn) and
+  // the gate's eight silus run interleaved; what is left of the gate is its
+  // arithmetic, 64 silus a thread. us, plain / residual / gate: 9728 x 2560 at
+  // 256 rows 25.7 / 31.2 / 37.0 before, 25.4 / 27.8 / 31.3; 3072 x 1024 at 512
+  // 11.2 / 13.2 / 16.5 before, 10.5 / 11.7 / 13.5.
+  constexpr int PITCH = BM * 2 + 16, CPR = BMO / 8, STEP = NT / CPR, IT = BN / STEP;
+  constexpr int RPS = KG * STAGE / PITCH;  // rows a stage holds
+  static_assert(3 * RPS >= BN && NT % CPR == 0 && BN % STEP == 0, "the tile exceeds the ring");
+  static_assert(KG == 1 || RPS >= BN, "ring0 may still be read (the second group's sums)");
+  auto row_at = [&](int n) {
+    if (RPS >= BN || n < RPS) return &ring1[0][0] + n * PITCH;
+    return n < 2 * RPS ? &ring2[0][0] + (n - RPS) * PITCH : &ring0[0][0] + (n - 2 * RPS) * PITCH;
+  };
   const int ep = SW ? 2 : epi & 3;
-  const bool vec = (M & 7) == 0 && (epi & 8);
+  const int ch = tid % CPR, m = m0 + ch * 8;
+  const bool full = (M & 7) == 0 && (epi & 8) && m + 8 <= M;
+  constexpr int IR = SW ? 1 : IT;
+  u32x4 rr[IR];
 #pragma unroll
-  for (int q = 0; q < 4 / QB; ++q) {
-    if (q) __syncthreads();
-    if (kg == 0) {
+  for (int i = 0; i < IR; ++i) rr[i] = u32x4{0, 0, 0, 0};
+  if (!SW && ep && full) {
 #pragma unroll
-      for (int bb = 0; bb < QB; ++bb)
+    for (int i = 0; i < IR; ++i)
+      rr[i] = *reinterpret_cast<const u32x4*>(R + (size_t)min(n0 + tid / CPR + i * STEP, N - 1) * M + m);
+  }
+  if (kg == 0) {
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const f32x16_v& a = acc[QB * q + bb];
-          *reinterpret_cast<uint2*>(stg + (32 * bb + (lane & 31)) * PITCH + wave * 64 + g * 16 + (lane >> 5) * 8) =
-              make_uint2(pack2<DT>(a[4 * g], a[4 * g + 1]), pack2<DT>(a[4 * g + 2], a[4 * g + 3]));
-        }
+    for (int b = 0; b < 4; ++b) {
+      uint8_t* const row = row_at(32 * b + (lane & 31)) + wave * 64 + (lane >> 5) * 8;
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<uint2*>(row + g * 16) = make_uint2(pack2<DT>(acc[b][4 * g], acc[b][4 * g + 1]),
+                                                             pack2<DT>(acc[b][4 * g + 2], acc[b][4 * g + 3]));
     }
-    __syncthreads();
+  }
+  __syncthreads();
+  if (!SW && !ep && full) {  // nothing to compute: all reads, then all stores
+    u32x4 y[IT];
+#pragma unroll
+    for (int i = 0; i < IT; ++i) y[i] = *reinterpret_cast<const u32x4*>(row_at(tid / CPR + i * STEP) + ch * 16);
+#pragma unroll
+    for (int i = 0; i < IT; ++i) {
+      const int n = n0 + tid / CPR + i * STEP;
+      if (n < N) *reinterpret_cast<u32x4*>(Y + (size_t)n * M + m) = y[i];
+    }
+    return;
+  }
 #pragma unroll 1
-    for (int e = tid; e < 32 * QB * CPR; e += NT) {
-      const int nl = e / CPR, ch = e % CPR;
-      const int n = n0 + 32 * QB * q + nl, m = m0 + ch * 8;
-      if (n >= N || m >= M) continue;
-      const u32x4 y = *reinterpret_cast<const u32x4*>(stg + nl * PITCH + ch * 16 + (SW ? BMO * 2 : 0));
-      u32x4 r = {0, 0, 0, 0};
-      if constexpr (SW) r = *reinterpret_cast<const u32x4*>(stg + nl * PITCH + ch * 16);
-      mm_store8<DT>(Y, R, (size_t)n * M + m, m, M, vec && m + 8 <= M, ep, y, SW, r);
-    }
+  for (int i = 0; i < IT; ++i) {
+    const int nl = tid / CPR + i * STEP, n = n0 + nl;
+    const uint8_t* const src = row_at(nl) + ch * 16;
+    u32x4 r = rr[0];
+#pragma unroll
+    for (int k = 0; k + 1 < IR; ++k) rr[k] = rr[k + 1];
+    if (n >= N || m >= M) continue;
+    const u32x4 y = *reinterpret_cast<const u32x4*>(src + (SW ? BMO * 2 : 0));
+    if constexpr (SW) r = *reinterpret_cast<const u32x4*>(src);
+    mm_store8<DT>(Y, R, (size_t)n * M + m, m, M, full, ep, y, SW || full, r);
   }
 #endif
 }

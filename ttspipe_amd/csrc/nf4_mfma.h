@@ -53,20 +53,46 @@ __device__ __forceinline__ uint16_t mm_epi(float y, uint16_t r, int ep) {
   return Elem<DT>::store(v);
 }
 
+// silu_rn's arithmetic with the range tests of its exp as selects: no branch, so
+// that several run interleaved.
+__device__ __forceinline__ float silu_flat(float a) {
+  const float x = -a;
+  const float n = __builtin_rintf(__fmul_rn(__builtin_amdgcn_fmed3f(x, -87.0f, 88.72283935546875f),
+                                            1.44269502162933349609375f));
+  float r = __builtin_fmaf(n, -0.693359375f, x);
+  r = __builtin_fmaf(n, 2.12194440e-4f, r);
+  const float z = __fmul_rn(r, r);
+  float p = 1.9875691500e-4f;
+  p = __builtin_fmaf(p, r, 1.3981999507e-3f);
+  p = __builtin_fmaf(p, r, 8.3334519073e-3f);
+  p = __builtin_fmaf(p, r, 4.1665795894e-2f);
+  p = __builtin_fmaf(p, r, 1.6666665459e-1f);
+  p = __builtin_fmaf(p, r, 5.0000001201e-1f);
+  p = __builtin_fmaf(p, z, r);
+  p = __builtin_ldexpf(__fadd_rn(p, 1.0f), (int)n);
+  p = x > 88.72283935546875f ? __uint_as_float(0x7f800000u) : x < -87.0f ? 0.0f : p;
+  return __fdiv_rn(a, __fadd_rn(1.0f, p));
+}
+
 // Eight values of an output row (packed, rounded) through the epilogue with
-// their operands, a dword of each a turn: the vectors rotate, so a rolled loop
-// indexes nothing at run time and its code stays small.
+// their operands. A caller keeps it in a rolled loop: eight silus are ~2 KB.
 template <int DT>
 __device__ __forceinline__ u32x4 mm_epi8(u32x4 y, u32x4 r, int ep) {
-#pragma unroll 1
-  for (int q = 0; q < 4; ++q) {
-    const uint32_t a = y.x, b = r.x;
-    const uint32_t w = (uint32_t)mm_epi<DT>(Elem<DT>::load(a), (uint16_t)b, ep) |
-                       ((uint32_t)mm_epi<DT>(Elem<DT>::load(a >> 16), (uint16_t)(b >> 16), ep) << 16);
-    y = u32x4{y.y, y.z, y.w, w};
-    r = u32x4{r.y, r.z, r.w, b};
+  u32x4 o;
+  if (ep == 1) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      o[q] = pack2<DT>(__fadd_rn(Elem<DT>::load(r[q]), Elem<DT>::load(y[q])),
+                       __fadd_rn(Elem<DT>::load(r[q] >> 16), Elem<DT>::load(y[q] >> 16)));
+  } else {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const uint32_t g = pack2<DT>(silu_flat(Elem<DT>::load(r[q])), silu_flat(Elem<DT>::load(r[q] >> 16)));
+      o[q] = pack2<DT>(__fmul_rn(Elem<DT>::load(g), Elem<DT>::load(y[q])),
+                       __fmul_rn(Elem<DT>::load(g >> 16), Elem<DT>::load(y[q] >> 16)));
+    }
   }
-  return y;
+  return o;
 }
 
 // Eight values at Y + o (m .. m + 7 of a row of M, full: aligned and all below
