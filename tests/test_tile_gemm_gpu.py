@@ -40,6 +40,8 @@ def test_tile_splits_follow_the_split_plan():
     ((9728, 2560), 256, True, 64, 256, torch.float16, 0),    # 128 rows a workgroup
     ((9000, 2560), 250, False, 256, 0, torch.bfloat16, 1),   # the same, ragged both ways
     ((9730, 2560), 500, True, 64, 32, torch.bfloat16, 0),    # 256 rows a workgroup, M % 4 == 2
+    ((8190, 2560), 511, True, 64, 256, torch.float16, 2),    # 128 tiles of 256 rows: 256 of 128 rows run instead
+    ((8200, 2560), 512, False, 64, 0, torch.bfloat16, 1),    # one tile more: 256 rows a workgroup
     ((9728, 2176), 512, True, 128, 256, torch.float16, 2),   # 34 steps: a ring remainder of one past two chunks
     ((9728, 2048), 400, False, 64, 0, torch.bfloat16, 0),    # 32 steps: a remainder of two
     ((2560, 9728), 512, True, 64, 256, torch.bfloat16, 1),   # four K splits

@@ -375,7 +375,7 @@ double tile_estimate(int M, int K, int N) {
   const long long t64 = gemm_tiles(M, N, 64, 128) * z, t128 = gemm_tiles(M, N, 128, 128) * z,
                   t256 = gemm_tiles(M, N, 256, 128) * z;
   double us = t64 <= 256 ? steps / 2 * 0.75 + 5.0
-              : t256 >= 128 ? (double)((t256 + 255) / 256) * (steps * 0.95 + 5.0)
+              : t256 > 128 ? (double)((t256 + 255) / 256) * (steps * 0.95 + 5.0)
                             : (double)((t128 + 255) / 256) * (steps * 0.66 + 5.0);
   if (z > 1) us += 4.0 + (double)z * N * M * 8.0 / 4e6;
   return us;

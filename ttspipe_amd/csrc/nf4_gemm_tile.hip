@@ -27,10 +27,13 @@
 //   (at 16 copies 19.8, 19.5 and 23.2; 1024 x 1024 at 256 rows, where a short K
 //   leaves the prologue most of the launch, 10.9 against 10.4, and in 2 splits
 //   slower than the kernel before).
-// * 256 rows (W 8) where at least half the CUs get one: one code table serves
+// * 256 rows (W 8) where more than half the CUs get one: one code table serves
 //   eight waves, so it can hold 32 copies (64 KB: a lookup's 64 lanes then
 //   touch every bank the minimum number of times), -5 % against one copy.
-// * 128 rows (W 4) between: 9728 x 2560 at 256 rows 34.1 -> 28.0.
+// * 128 rows (W 4) between: 9728 x 2560 at 256 rows 34.1 -> 28.0. At 128 of the
+//   256-row tiles, where 128-row ones still fit one to a CU, they are the
+//   faster: 8192 x 2560 at 512 rows 33.4 -> 29.3, with a gate 42.6 -> 35.7; 4096 x
+//   1024 at 1000 rows with a gate 27.2 -> 21.7 (24.5 in the kernel before).
 // The SwiGLU form takes W 4 with one copy, so that two workgroups fit a CU
 // (9728 x 2560 at 512 rows 86 -> 73; W 8 with 32 copies was slower).
 #include "nf4_mfma.h"
@@ -475,7 +478,7 @@ int tile_form(const void* X, const TileMat& a, const float* LUT, void* Y, const 
   const long long nt = (long long)((N + BN - 1) / BN) * splits;
   if (tile_halves(M, N, splits))
     return launch_tile<DT, 2, 2, 1, false>(X, a, a, LUT, Y, R, epi, M, K, N, bs_shift, bs2_shift, splits, YP, st);
-  if ((M + 255) / 256 * nt >= 128)
+  if ((M + 255) / 256 * nt > 128)
     return launch_tile<DT, 8, 1, 32, false>(X, a, a, LUT, Y, R, epi, M, K, N, bs_shift, bs2_shift, splits, YP, st);
   return launch_tile<DT, 4, 1, 32, false>(X, a, a, LUT, Y, R, epi, M, K, N, bs_shift, bs2_shift, splits, YP, st);
 }
