@@ -157,7 +157,8 @@ int ttsp_nf4_gemm_few(const void* X, int x_dtype, const uint8_t* W, const uint8_
 /* Long prompts: the product in two launches, the weight dequantised once into
  * the caller's workspace, then a dense matrix kernel on it.
  * ttsp_nf4_gemm_dense_splits: the K splits it runs in, 0 where it does not
- * serve the shape (N below 513, small weights, byte offsets of 2^31 or more).
+ * serve the shape (N below 513, below 1024 where the tile kernel is estimated
+ * faster, small weights, byte offsets of 2^31 or more).
  * work: 16-byte aligned, 2 * M * K bytes of dense weights, then (splits > 1)
  * splits * N * M fp32 partial sums. Other arguments as ttsp_nf4_gemm's. */
 int ttsp_nf4_gemm_dense_splits(int M, int K, int N);
